@@ -97,22 +97,24 @@ int op_geometry(int64_t N, int64_t T, int64_t S, int64_t D, int64_t block, Geo &
     if (D > 256)
         return fail(RACE_ERR_UNSUPPORTED, "race_op: head dim D = %lld > 256 is not compiled", (long long)D);
     g.DP = D <= 32 ? 32 : D <= 64 ? 64 : D <= 128 ? 128 : 256;
-    // bucket tiles of at most 64 (the largest measured fastest at D = 32 and 64 for S = 64 and 128;
-    // 128-wide tiles at D = 32 are slower)
-    const int st_max = std::min(64, 4096 / g.DP);
-    g.ST = st_max;
-    for (int st : {16, 32, 64, 128})
-        if (st <= st_max && st >= S) {
+    // bucket tiles of up to 128: every V and gO row is read once for all of them and no partial
+    // outputs are summed
+    g.ST = 128;
+    for (int st : {16, 32, 64})
+        if (st >= S) {
             g.ST = st;
             break;
         }
-    if (!op_variant_exists(g.ST, g.DP))
-        return fail(RACE_ERR_UNSUPPORTED, "race_op: no kernel for tile (%d, %d)", g.ST, g.DP);
     g.C = OP_C;
     g.n_st = (int)cdiv(S, g.ST);
     g.S_pad = g.n_st * g.ST;
     g.Z = N;
-    g.CB = resolve_block(T, N * g.n_st, g.C, block, 2048);
+    if (block > 0) {
+        g.CB = resolve_block(T, N * g.n_st, g.C, block, 0);
+    } else {  // about 2048 workgroups, blocks of whole stages
+        const int64_t nb = std::max<int64_t>(1, cdiv(2048, N * g.n_st));
+        g.CB = std::min(std::max<int64_t>(64, rup(cdiv(T, nb), 64)), rup(T, g.C));
+    }
     g.NB = cdiv(T, g.CB);
     fill_ws_sizes(g);
     return RACE_OK;
@@ -408,11 +410,14 @@ int race_soft_hash_bwd_dscale(const race_hash_shape *sh, race_tensor x, int x_dt
 }
 
 // ============================================================================ op-level scan
+static int op_nck(const Geo &g) { return (int)cdiv(g.CB, op_stage_tokens(g.DP)); }
+static size_t op_checkpoints(const Geo &g) { return (size_t)g.Z * g.NB * op_nck(g) * g.S_pad; }
+
 static size_t op_bytes(const Geo &g, int64_t T, int64_t D, int backward)
 {
     size_t b = align256(g.state_elems_B * 4) + align256(g.state_elems_A * 4);
-    if (backward)  // the backward suffix states as double-floats (hi and lo arrays)
-        b += 2 * (align256(g.state_elems_B * 4) + align256(g.state_elems_A * 4));
+    if (backward)  // the suffix states as double-floats (hi and lo arrays), the A checkpoints of the reverse walk
+        b += 2 * (align256(g.state_elems_B * 4) + align256(g.state_elems_A * 4)) + align256(op_checkpoints(g) * 4);
     if (g.n_st > 1)
         b += align256((size_t)g.n_st * g.Z * T * D * 4);
     return b;
@@ -452,11 +457,22 @@ static ScanParams op_params(const Geo &g, int64_t T, int64_t S, int64_t D, float
     return P;
 }
 
-static int run_scan_op(ScanKernel k, const Geo &g, const ScanParams &P, hipStream_t s)
+static bool aligned16(const void *p) { return (reinterpret_cast<uintptr_t>(p) & 15) == 0; }
+
+static int run_scan_op(OpKernel k, const Geo &g, const ScanParams &P, hipStream_t s)
 {
-    ProfScope ps(RACE_PROF_OP_FWD_TOTALS + (int)k, s);
+    static const int prof_id[] = {RACE_PROF_OP_FWD_TOTALS, RACE_PROF_OP_FWD_READOUT, RACE_PROF_OP_BWD_TOTALS,
+                                  RACE_PROF_OP_BWD_MAIN, RACE_PROF_OP_BWD_MAIN};
+    ProfScope ps(prof_id[k], s);
     const dim3 grid((unsigned)g.NB, (unsigned)g.n_st, (unsigned)g.Z);
     return hip_check(launch_scan_op(k, g.ST, g.DP, P, grid, s), "race_op kernel launch");
+}
+
+// rows move as 16-byte runs where every row of the operands starts 16-byte aligned
+static void op_vec(ScanParams &P)
+{
+    P.vec = P.S % 4 == 0 && P.D % 4 == 0 && aligned16(P.pK) && aligned16(P.pQ) && aligned16(P.V) && aligned16(P.gO) &&
+            !((P.v.sb | P.v.sh | P.v.st | P.go.sb | P.go.sh | P.go.st) & 3);
 }
 
 static int op_check(const float *pK, const float *pQ, const float *V, float eps, void *ws,
@@ -515,10 +531,11 @@ static int op_fwd_impl(const float *pK, const float *pQ, const float *V, float *
         state_views(g, state, P.wsB, P.wsA);
     float *part = g.n_st > 1 ? cv.take((size_t)g.n_st * N * T * D) : nullptr;
     P.out = part ? OutView{part, T * D, 0, D, N * T * D, 1} : OutView{out, T * D, 0, D, 0, 1};
+    op_vec(P);
     const hipStream_t s = hs(stream);
-    RACE_TRY(run_scan_op(K_FWD_TOTALS, g, P, s));
+    RACE_TRY(run_scan_op(OP_TOTALS, g, P, s));
     RACE_TRY(hip_check(prof_block_scan(P.wsB, (int64_t)g.S_pad * g.DP, P.wsA, g.S_pad, (int)g.NB, (int)g.Z, 0, s), "block scan"));
-    RACE_TRY(run_scan_op(K_FWD_READOUT, g, P, s));
+    RACE_TRY(run_scan_op(OP_READOUT, g, P, s));
     if (part)
         RACE_TRY(hip_check(prof_reduce(part, g.n_st, N * T * D, OutView{out, T * D, 0, D, 0, 1},
                                                   (int)N, 1, (int)T, (int)D, s), "reduce partials"));
@@ -558,21 +575,25 @@ static int op_bwd_impl(const float *pK, const float *pQ, const float *V, const f
     P.ws2A = cv.take(g.state_elems_A);
     P.ws3B = cv.take(g.state_elems_B);
     P.ws3A = cv.take(g.state_elems_A);
+    P.ckA = cv.take(op_checkpoints(g));
+    P.NCK = op_nck(g);
     float *part = g.n_st > 1 ? cv.take((size_t)g.n_st * N * T * D) : nullptr;
     P.dv = part ? OutView{part, T * D, 0, D, N * T * D, 1} : OutView{gV, T * D, 0, D, 0, 1};
+    op_vec(P);
     const hipStream_t s = hs(stream);
     if (state) {  // forward block states kept by race_op_fwd_keep (only read from here on)
         state_views(g, state, P.wsB, P.wsA);
     } else {  // recomputed: nothing is saved between calls
-        RACE_TRY(run_scan_op(K_FWD_TOTALS, g, P, s));
+        RACE_TRY(run_scan_op(OP_TOTALS, g, P, s));
         RACE_TRY(hip_check(prof_block_scan(P.wsB, (int64_t)g.S_pad * g.DP, P.wsA, g.S_pad, (int)g.NB, (int)g.Z, 0, s),
                            "block scan"));
     }
-    RACE_TRY(run_scan_op(K_BWD_TOTALS, g, P, s));
+    RACE_TRY(run_scan_op(OP_GQ, g, P, s));
     RACE_TRY(hip_check(prof_block_scan(P.ws2B, (int64_t)g.S_pad * g.DP, P.ws2A, g.S_pad, (int)g.NB, (int)g.Z, 1, s,
                                        P.ws3B, P.ws3A),
                        "block scan"));
-    RACE_TRY(run_scan_op(K_BWD_MAIN, g, P, s));
+    RACE_TRY(run_scan_op(OP_GK, g, P, s));
+    RACE_TRY(run_scan_op(OP_GV, g, P, s));
     if (part)
         RACE_TRY(hip_check(prof_reduce(part, g.n_st, N * T * D, OutView{gV, T * D, 0, D, 0, 1},
                                                   (int)N, 1, (int)T, (int)D, s), "reduce partials"));
@@ -676,7 +697,8 @@ static int nc_totals(const Geo &g, ScanParams P, const float *w, const View &xv,
     P.zH = zH;
     P.wsB = wsB;
     P.wsA = wsA;
-    RACE_TRY(run_scan_op(K_FWD_TOTALS, g, P, s));
+    op_vec(P);
+    RACE_TRY(run_scan_op(OP_TOTALS, g, P, s));
     return hip_check(prof_block_scan(wsB, (int64_t)g.S_pad * g.DP, wsA, g.S_pad, (int)g.NB, (int)g.Z, 0, s), "block scan");
 }
 

@@ -20,22 +20,18 @@ struct Variant {
 // an uncompiled (ST, DP) pair.
 hipError_t launch_scan_qkv(ScanKernel k, int ST, int DP, const ScanParams &P, dim3 grid,
                            hipStream_t s);
-// fp32 probabilities-in variants (race_scan_op.hip).
-hipError_t launch_scan_op(ScanKernel k, int ST, int DP, const ScanParams &P, dim3 grid,
-                          hipStream_t s);
+// fp32 probabilities-in kernels of the op path (race_scan_op.hip): block totals, readout, gpQ with
+// the backward's block totals, gpK, gv
+enum OpKernel { OP_TOTALS = 0, OP_READOUT = 1, OP_GQ = 2, OP_GK = 3, OP_GV = 4 };
+hipError_t launch_scan_op(OpKernel k, int ST, int DP, const ScanParams &P, dim3 grid, hipStream_t s);
+int op_stage_tokens(int DP);  // tokens between A checkpoints (ScanParams::ckA)
 bool qkv_variant_exists(int ST, int DP);
 // fused bf16 forward kernels specialised on the hash bits (race_fused.hip)
 hipError_t launch_fused(ScanKernel k, int ST, int DP, int KB, const ScanParams &P, dim3 grid, hipStream_t s);
 bool fused_variant_exists(int ST, int DP, int KB);
 constexpr int FUSED_NW_FWD = 4, FUSED_NW_BWD = 8;
-bool op_variant_exists(int ST, int DP);
 constexpr int QKV_C = 32, QKV_NW = 4;
-// fp32 op path: waves per workgroup. 4 for the totals kernels; for the readout and backward main
-// kernels 8 at head-dim tiles of 64 and more, whose long sub-chunk phases hide more latency with
-// them (at 2^20 (token, head) pairs and D = 64: 1.57 -> 1.05 and 4.81 -> 3.50 ms; D = 128 and
-// 256 alike), and 4 at 32, where 8 measured slower
-constexpr int OP_C = 16, OP_NW_TOTALS = 4;
-constexpr int op_nw_main(int DP) { return DP >= 64 ? 8 : 4; }
+constexpr int OP_C = 16;  // tokens per sub-chunk of the op path
 
 // race_common.hip
 // scans wsB [Z][NB+1][elemsB] and wsA [Z][NB+1][elemsA] over the block axis in one launch; with

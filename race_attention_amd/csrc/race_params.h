@@ -27,7 +27,7 @@ struct OutView {
 };
 
 // One launch of the chunked causal scan.
-//   stream z:  op mode   z = n (one of N independent [T,S]/[T,D] streams)
+//   stream z:  op path   z = n (one of N independent [T,S]/[T,D] streams)
 //              qkv mode  z = b * Hkv + hk (one kv head; query heads hk*G .. hk*G+G-1)
 //   grid:      (NB blocks along T, n_st bucket tiles, Z streams)
 struct ScanParams {
@@ -42,7 +42,7 @@ struct ScanParams {
     View q, k, v, go;
     OutView out, dq, dk, dv;
     const float *planes;
-    // op mode (fp32): probabilities [N][T][S], values/grads rows of D floats. Stream z reads its
+    // op path (fp32): probabilities [N][T][S], values/grads rows of D floats. Stream z reads its
     // V / gO rows as a [Z / zH][zH][T][D] view: row t of z at (z / zH) sb + (z % zH) sh + t st,
     // strides in v / go (their p unused); contiguous [N][T][D] is zH = 1, sb = T D, st = D
     const float *pK, *pQ, *V, *gO;
@@ -51,9 +51,13 @@ struct ScanParams {
     // workspaces: block states [Z][NB+1][S_pad][DPw] and [Z][NB+1][S_pad]
     float *wsB, *wsA;    // forward: prefix (A, B) at each block start; slot NB = final
     float *ws2B, *ws2A;  // backward: suffix sums (of W^T go, gA) from each block's start
-    // generic backward kernels: low parts of the same suffix sums (ws2 + ws3 = a double-float)
+    // op path and generic bf16 backward kernels: low parts of the same suffix sums (ws2 + ws3 = a double-float)
     float *ws3B, *ws3A;
-    // op mode only: 1 = unnormalised causal linear attention, W = pQ (no 1/(A+eps), gA = 0)
+    // op path, backward: A at every stage start of every block, [Z][NB][NCK][S_pad]
+    float *ckA;
+    int NCK;
+    int vec;  // op path: every row of the operands starts 16-byte aligned
+    // op path only: 1 = unnormalised causal linear attention, W = pQ (no 1/(A+eps), gA = 0)
     int linear;
 };
 

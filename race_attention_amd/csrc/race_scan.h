@@ -27,13 +27,9 @@
 // phase1 / phase2 / phase3 split (forward_kernel.cu:8-13) lifted to blocks of
 // sub-chunks, with the per-timestep loops replaced by MFMA tiles and no atomics.
 //
-// Modes:
-//   MODE_QKV  bf16 q, k, v in; the soft-hash (race_common.py:56-72) is computed
-//             in-kernel from the projection planes, so the [T,S] probabilities
-//             never touch HBM; the backward runs the soft-hash backward in-kernel
-//             and writes dq, dk, dv.
-//   MODE_OP   fp32 probabilities pK, pQ [N,T,S] and V [N,T,D] in (the
-//             RaceCausalFn.apply interface, race_causal_cuda.py:47-69).
+// Inputs: bf16 q, k, v; the soft-hash (race_common.py:56-72) is computed in-kernel from the
+// projection planes, so the [T,S] probabilities never touch HBM; the backward runs the soft-hash
+// backward in-kernel and writes dq, dk, dv. (The fp32 op path, probabilities in: race_op_scan.h.)
 //
 // Tile ownership per wave (16x16 MFMA tiles, NW waves):
 //   [C x ST] tiles: wave owns whole bucket columns (all token tiles of them),
@@ -44,12 +40,9 @@
 
 namespace race {
 
-enum { MODE_OP = 0, MODE_QKV = 1 };
-
-template <class E, int MODE, int ST, int DP, int C, int NW>
+template <class E, int ST, int DP, int C, int NW>
 struct Cfg {
     using T = typename E::T;
-    static constexpr bool QKV = MODE == MODE_QKV;
     static constexpr int NW_ = NW;
     static constexpr int NTH = NW * 64;
     static constexpr int PD = E::PAD;
@@ -57,7 +50,7 @@ struct Cfg {
     static constexpr int NTS = ST / 16;
     static constexpr int NTD = DP / 16;
     // padded projection columns of one bucket tile: Lt*K <= ST/2 for K >= 1
-    static constexpr int LKPM = QKV ? ((ST / 2 > 32) ? ST / 2 : 32) : 16;
+    static constexpr int LKPM = (ST / 2 > 32) ? ST / 2 : 32;
     static constexpr int NTLM = LKPM / 16;
     static constexpr int TPW_CS = MTC * ((NTS + NW - 1) / NW);
     static constexpr int TPW_SD = (NTS * NTD + NW - 1) / NW;
@@ -131,51 +124,14 @@ RACE_DEV void load_rows_bf16(__bf16 *dst, __bf16 *dstT, const View &vw, int b, i
     }
 }
 
-// op mode: first row of stream z in a V / gO view (ScanParams::zH; zH <= 1: stream stride sb)
+// op path: first row of stream z in a V / gO view (ScanParams::zH; zH <= 1: stream stride sb)
 RACE_DEV const float *op_rows(const float *p, const View &v, int zH, int z)
 {
     return zH <= 1 ? p + (int64_t)z * v.sb : p + (int64_t)(z / zH) * v.sb + (int64_t)(z % zH) * v.sh;
 }
 
-// Register-staged copy of one sub-chunk of an fp32 [N][T][ld] tensor (rows t0 .. t0 + C, columns
-// col0 .. col0 + W): fetch() issues this thread's loads, put() stores them to LDS [C][LD] and / or
-// transposed [W][LDT]. Loads go to clamped rows and columns (always inside the tensor) and are
-// unconditional, so a later wait on the in-order memory counter does not have to drain them early;
-// put() writes zeros for rows >= nv and columns >= ncol. Fetching sub-chunk i + 1 before the
-// MFMA phase of sub-chunk i overlaps its memory latency with that phase.
-template <int C, int W, int NTH>
-struct SubChunkStage {
-    static constexpr int N = (C * W + NTH - 1) / NTH;
-    float x[N];
-
-    RACE_DEV void fetch(const float *src, int ld, int col0, int ncol, int t0, int t_last, int tid)
-    {
-#pragma unroll
-        for (int j = 0; j < N; ++j) {
-            const int i = tid + j * NTH, r = i / W, s = i % W;
-            x[j] = src[(int64_t)min(t0 + r, t_last) * ld + col0 + min(s, ncol - 1)];
-        }
-    }
-
-    template <class T, int LD, int LDT, bool ROW, bool TRN>
-    RACE_DEV void put(T *dst, T *dstT, int nv, int ncol, int tid) const
-    {
-#pragma unroll
-        for (int j = 0; j < N; ++j) {
-            const int i = tid + j * NTH, r = i / W, s = i % W;
-            if (C * W % NTH == 0 || i < C * W) {
-                const float v = (r < nv && s < ncol) ? x[j] : 0.0f;
-                if (ROW)
-                    dst[r * LD + s] = (T)v;
-                if (TRN)
-                    dstT[s * LDT + r] = (T)v;
-            }
-        }
-    }
-};
-
 // ------------------------------------------------------------------ soft-hash pieces
-// Constant planes fragments for this wave (QKV mode only):
+// Constant planes fragments for this wave:
 //  projection B operand (col j, k = d):   planes_T[d][l0*K + j]
 //  soft-hash-backward B operand (col d, k = j): same element, other orientation
 template <class E, class CF>

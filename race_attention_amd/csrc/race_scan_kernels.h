@@ -1,9 +1,10 @@
-// The four chunked-scan kernels (see race_scan.h for the math and layout).
+// The four chunked-scan kernels of the bf16 layer in their generic form: any table count and hash
+// bits, for what the fused kernels (race_fused.h) are not compiled for (see race_scan.h for the math and layout).
 //   race_fwd_totals   per-block totals (sum pK, sum pK^T v) -> workspace slot blk
 //   race_fwd_readout  per-block causal readout from the block-start state
-//   race_bwd_totals   forward-order pass: gpQ (op) / dq (qkv) and per-block
+//   race_bwd_totals   forward-order pass: dq and per-block
 //                     totals of gA and W^T go -> backward workspace slot blk
-//   race_bwd_main     forward-order pass with reverse suffix states: gpK, gv (op) / dk, dv (qkv)
+//   race_bwd_main     forward-order pass with reverse suffix states: dk, dv
 #pragma once
 #include "race_scan.h"
 
@@ -37,19 +38,6 @@ RACE_DEV void store_out_tile(const OutView &o, int b, int h, int st, int t0, int
                 reinterpret_cast<__bf16 *>(o.p)[off] = (__bf16)v[e];
         }
     }
-}
-
-// Store an accumulator tile of per-bucket values to an [N][T][S] fp32 tensor.
-RACE_DEV void store_probs_tile(float *dst, int S, int s0, int S_here, int t0, int nv, int m0,
-                               int n0, int lane, const f32x4 &v)
-{
-    const int r = acc_row(m0, lane), col = acc_col(n0, lane);
-    if (col >= S_here)
-        return;
-#pragma unroll
-    for (int e = 0; e < 4; ++e)
-        if (r + e < nv)
-            dst[(int64_t)(t0 + r + e) * S + s0 + col] = v[e];
 }
 
 template <class T>
@@ -105,14 +93,14 @@ RACE_DEV void put_hilo(float *hi, float *lo, double x)
 }
 
 // ============================================================================ forward totals
-template <class E, int MODE, int ST, int DP, int C, int NW>
+template <class E, int ST, int DP, int C, int NW>
 __global__ __launch_bounds__(NW * 64) void race_fwd_totals(const ScanParams P)
 {
-    using CF = Cfg<E, MODE, ST, DP, C, NW>;
+    using CF = Cfg<E, ST, DP, C, NW>;
     using T = typename E::T;
     constexpr int PD = CF::PD, NTH = CF::NTH;
     constexpr int LDX = DP + PD, LDC = C + PD, LDU = CF::LKPM + 1;
-    constexpr int XR = CF::QKV ? C : 1;
+    constexpr int XR = C;
     __shared__ __align__(16) T sX[XR][LDX];
     __shared__ __align__(16) T sVt[DP][LDC];
     __shared__ __align__(16) float sU[XR][LDU];
@@ -121,8 +109,7 @@ __global__ __launch_bounds__(NW * 64) void race_fwd_totals(const ScanParams P)
     const Ctx c = make_ctx(P, ST);
     __builtin_assume(c.wave >= 0 && c.wave < NW);  // (threadIdx.x < NW * 64)
     PlaneFrags<E, CF> pf;
-    if constexpr (CF::QKV)
-        pf.load(P, c);
+    pf.load(P, c);
     zero_lds(&sPKt[0][0], ST * LDC, c.tid, NTH);
 
     constexpr int TPW_A1 = (CF::NTS + NW - 1) / NW;
@@ -136,38 +123,22 @@ __global__ __launch_bounds__(NW * 64) void race_fwd_totals(const ScanParams P)
     __syncthreads();
 
     const int nsub = (c.t_end - c.t_begin + C - 1) / C;
-    // op mode: this sub-chunk's probabilities and values wait in registers, fetched one sub-chunk ahead
-    SubChunkStage<C, ST, NTH> stP;
-    SubChunkStage<C, DP, NTH> stV;
-    const float *srcP = P.pK + (int64_t)c.z * P.T * P.S, *srcV = op_rows(P.V, P.v, P.zH, c.z);
-    if constexpr (!CF::QKV) {
-        stP.fetch(srcP, P.S, c.s0, c.S_here, c.t_begin, P.T - 1, c.tid);
-        stV.fetch(srcV, (int)P.v.st, 0, P.D, c.t_begin, P.T - 1, c.tid);
-    }
     for (int sc = 0; sc < nsub; ++sc) {
         const int t0 = c.t_begin + sc * C;
         const int nv = min(C, c.t_end - t0);
-        if constexpr (CF::QKV) {
-            load_rows_bf16<C, DP, NTH, LDX, LDC, true, false>(&sX[0][0], nullptr, P.k, c.b, c.hk, t0, nv, c.tid);
-            load_rows_bf16<C, DP, NTH, LDX, LDC, false, true>(nullptr, &sVt[0][0], P.v, c.b, c.hk, t0, nv, c.tid);
-            __syncthreads();
-            project<E, CF, LDX, LDU>(&sX[0][0], &sU[0][0], pf, c, P.inv_scale);
-            __syncthreads();
-            const int R = P.R;
-            expand<CF, LDU>(&sU[0][0], c, P.K, [&](int t, int lt, const float *, const float *pr) {
-                const bool ok = t < nv;
+        load_rows_bf16<C, DP, NTH, LDX, LDC, true, false>(&sX[0][0], nullptr, P.k, c.b, c.hk, t0, nv, c.tid);
+        load_rows_bf16<C, DP, NTH, LDX, LDC, false, true>(nullptr, &sVt[0][0], P.v, c.b, c.hk, t0, nv, c.tid);
+        __syncthreads();
+        project<E, CF, LDX, LDU>(&sX[0][0], &sU[0][0], pf, c, P.inv_scale);
+        __syncthreads();
+        const int R = P.R;
+        expand<CF, LDU>(&sU[0][0], c, P.K, [&](int t, int lt, const float *, const float *pr) {
+            const bool ok = t < nv;
 #pragma unroll
-                for (int r = 0; r < 16; ++r)
-                    if (r < R)
-                        sPKt[lt * R + r][t] = (T)(ok ? pr[r] : 0.0f);
-            });
-        } else {
-            stP.template put<T, LDC, LDC, false, true>(nullptr, &sPKt[0][0], nv, c.S_here, c.tid);
-            stV.template put<T, LDC, LDC, false, true>(nullptr, &sVt[0][0], nv, P.D, c.tid);
-            // next sub-chunk (past the block end: clamped rows, never stored)
-            stP.fetch(srcP, P.S, c.s0, c.S_here, t0 + C, P.T - 1, c.tid);
-            stV.fetch(srcV, (int)P.v.st, 0, P.D, t0 + C, P.T - 1, c.tid);
-        }
+            for (int r = 0; r < 16; ++r)
+                if (r < R)
+                    sPKt[lt * R + r][t] = (T)(ok ? pr[r] : 0.0f);
+        });
         __syncthreads();
 #pragma unroll
         for (int i = 0; i < CF::TPW_SD; ++i) {
@@ -176,13 +147,11 @@ __global__ __launch_bounds__(NW * 64) void race_fwd_totals(const ScanParams P)
                 mma_tile<E, C>(accS[i], &sPKt[0][0], LDC, &sVt[0][0], LDC, (t / CF::NTD) * 16,
                                (t % CF::NTD) * 16, c.lane);
         }
-        if (!P.linear) {  // (grid-uniform) linear attention has no normaliser A
 #pragma unroll
-            for (int i = 0; i < TPW_A1; ++i) {
-                const int tn = c.wave + i * NW;
-                if (tn < CF::NTS)
-                    mma_tile_gen<E, C>(accA[i], PredAll(), 1.0f, &sPKt[0][0], LDC, 0, tn * 16, c.lane);
-            }
+        for (int i = 0; i < TPW_A1; ++i) {
+            const int tn = c.wave + i * NW;
+            if (tn < CF::NTS)
+                mma_tile_gen<E, C>(accA[i], PredAll(), 1.0f, &sPKt[0][0], LDC, 0, tn * 16, c.lane);
         }
         __syncthreads();
     }
@@ -209,14 +178,14 @@ __global__ __launch_bounds__(NW * 64) void race_fwd_totals(const ScanParams P)
 }
 
 // ============================================================================ forward readout
-template <class E, int MODE, int ST, int DP, int C, int NW>
+template <class E, int ST, int DP, int C, int NW>
 __global__ __launch_bounds__(NW * 64) void race_fwd_readout(const ScanParams P)
 {
-    using CF = Cfg<E, MODE, ST, DP, C, NW>;
+    using CF = Cfg<E, ST, DP, C, NW>;
     using T = typename E::T;
     constexpr int PD = CF::PD, NTH = CF::NTH, MTC = CF::MTC;
     constexpr int LDX = DP + PD, LDC = C + PD, LDS_ = ST + PD, LDU = CF::LKPM + 1, LDF = ST + 4;
-    constexpr int XR = CF::QKV ? C : 1;
+    constexpr int XR = C;
     __shared__ __align__(16) T sX[XR][LDX];
     __shared__ __align__(16) T sVt[DP][LDC];
     __shared__ __align__(16) float sU[XR][LDU];
@@ -231,8 +200,7 @@ __global__ __launch_bounds__(NW * 64) void race_fwd_readout(const ScanParams P)
     const Ctx c = make_ctx(P, ST);
     __builtin_assume(c.wave >= 0 && c.wave < NW);  // (threadIdx.x < NW * 64)
     PlaneFrags<E, CF> pf;
-    if constexpr (CF::QKV)
-        pf.load(P, c);
+    pf.load(P, c);
     zero_lds(&sPK[0][0], C * LDS_, c.tid, NTH);
     zero_lds(&sPKt[0][0], ST * LDC, c.tid, NTH);
     zero_lds(&sF[0][0], C * LDF, c.tid, NTH);
@@ -263,44 +231,25 @@ __global__ __launch_bounds__(NW * 64) void race_fwd_readout(const ScanParams P)
 
     f32x4 accA[CF::TPW_CS];
     const int nsub = (c.t_end - c.t_begin + C - 1) / C;
-    // op mode: this sub-chunk's pK, pQ and values wait in registers, fetched one sub-chunk ahead
-    SubChunkStage<C, ST, NTH> stK, stQ;
-    SubChunkStage<C, DP, NTH> stV;
-    const float *srcK = P.pK + (int64_t)c.z * P.T * P.S, *srcQ = P.pQ + (int64_t)c.z * P.T * P.S;
-    const float *srcV = op_rows(P.V, P.v, P.zH, c.z);
-    if constexpr (!CF::QKV) {
-        stK.fetch(srcK, P.S, c.s0, c.S_here, c.t_begin, P.T - 1, c.tid);
-        stQ.fetch(srcQ, P.S, c.s0, c.S_here, c.t_begin, P.T - 1, c.tid);
-        stV.fetch(srcV, (int)P.v.st, 0, P.D, c.t_begin, P.T - 1, c.tid);
-    }
     for (int sc = 0; sc < nsub; ++sc) {
         const int t0 = c.t_begin + sc * C;
         const int nv = min(C, c.t_end - t0);
-        if constexpr (CF::QKV) {
-            load_rows_bf16<C, DP, NTH, LDX, LDC, true, false>(&sX[0][0], nullptr, P.k, c.b, c.hk, t0, nv, c.tid);
-            load_rows_bf16<C, DP, NTH, LDX, LDC, false, true>(nullptr, &sVt[0][0], P.v, c.b, c.hk, t0, nv, c.tid);
-            __syncthreads();
-            project<E, CF, LDX, LDU>(&sX[0][0], &sU[0][0], pf, c, P.inv_scale);
-            __syncthreads();
-            const int R = P.R;
-            expand<CF, LDU>(&sU[0][0], c, P.K, [&](int t, int lt, const float *, const float *pr) {
-                const bool ok = t < nv;
+        load_rows_bf16<C, DP, NTH, LDX, LDC, true, false>(&sX[0][0], nullptr, P.k, c.b, c.hk, t0, nv, c.tid);
+        load_rows_bf16<C, DP, NTH, LDX, LDC, false, true>(nullptr, &sVt[0][0], P.v, c.b, c.hk, t0, nv, c.tid);
+        __syncthreads();
+        project<E, CF, LDX, LDU>(&sX[0][0], &sU[0][0], pf, c, P.inv_scale);
+        __syncthreads();
+        const int R = P.R;
+        expand<CF, LDU>(&sU[0][0], c, P.K, [&](int t, int lt, const float *, const float *pr) {
+            const bool ok = t < nv;
 #pragma unroll
-                for (int r = 0; r < 16; ++r)
-                    if (r < R) {
-                        const T x = (T)(ok ? pr[r] : 0.0f);
-                        sPK[t][lt * R + r] = x;
-                        sPKt[lt * R + r][t] = x;
-                    }
-            });
-        } else {
-            stK.template put<T, LDS_, LDC, true, true>(&sPK[0][0], &sPKt[0][0], nv, c.S_here, c.tid);
-            stQ.template put<float, LDF, LDF, true, false>(&sF[0][0], nullptr, nv, c.S_here, c.tid);
-            stV.template put<T, LDC, LDC, false, true>(nullptr, &sVt[0][0], nv, P.D, c.tid);
-            stK.fetch(srcK, P.S, c.s0, c.S_here, t0 + C, P.T - 1, c.tid);
-            stQ.fetch(srcQ, P.S, c.s0, c.S_here, t0 + C, P.T - 1, c.tid);
-            stV.fetch(srcV, (int)P.v.st, 0, P.D, t0 + C, P.T - 1, c.tid);
-        }
+            for (int r = 0; r < 16; ++r)
+                if (r < R) {
+                    const T x = (T)(ok ? pr[r] : 0.0f);
+                    sPK[t][lt * R + r] = x;
+                    sPKt[lt * R + r][t] = x;
+                }
+        });
         __syncthreads();
 
         // A = A0 + Tri pK  (and its last row: the carry into the next sub-chunk)
@@ -309,7 +258,7 @@ __global__ __launch_bounds__(NW * 64) void race_fwd_readout(const ScanParams P)
         for (int i = 0; i < CF::TPW_CS; ++i) {
             const int tm = i % MTC, tn = c.wave + (i / MTC) * NW;
             carry[i] = 0.0f;
-            if (tn < CF::NTS && !P.linear) {  // (linear attention: no normaliser)
+            if (tn < CF::NTS) {
                 const float a0 = sA0[tn * 16 + (c.lane & 15)];
                 accA[i] = f32x4{a0, a0, a0, a0};
                 mma_tile_gen<E, C>(accA[i], PredTrilIncl(), 1.0f, &sPKt[0][0], LDC, tm * 16, tn * 16, c.lane);
@@ -324,24 +273,22 @@ __global__ __launch_bounds__(NW * 64) void race_fwd_readout(const ScanParams P)
                 sA0[tn * 16 + (c.lane & 15)] = carry[i];
         }
 
-        const int G = CF::QKV ? P.G : 1;
+        const int G = P.G;
         for (int g = 0; g < G; ++g) {
             const int hq = c.hk * P.G + g;
-            if constexpr (CF::QKV) {
-                load_rows_bf16<C, DP, NTH, LDX, LDC, true, false>(&sX[0][0], nullptr, P.q, c.b, hq, t0, nv, c.tid);
-                __syncthreads();
-                project<E, CF, LDX, LDU>(&sX[0][0], &sU[0][0], pf, c, P.inv_scale);
-                __syncthreads();
-                const int R = P.R;
-                expand<CF, LDU>(&sU[0][0], c, P.K, [&](int t, int lt, const float *, const float *pr) {
-                    const bool ok = t < nv;
+            load_rows_bf16<C, DP, NTH, LDX, LDC, true, false>(&sX[0][0], nullptr, P.q, c.b, hq, t0, nv, c.tid);
+            __syncthreads();
+            project<E, CF, LDX, LDU>(&sX[0][0], &sU[0][0], pf, c, P.inv_scale);
+            __syncthreads();
+            const int R = P.R;
+            expand<CF, LDU>(&sU[0][0], c, P.K, [&](int t, int lt, const float *, const float *pr) {
+                const bool ok = t < nv;
 #pragma unroll
-                    for (int r = 0; r < 16; ++r)
-                        if (r < R)
-                            sF[t][lt * R + r] = ok ? pr[r] : 0.0f;
-                });
-                __syncthreads();
-            }
+                for (int r = 0; r < 16; ++r)
+                    if (r < R)
+                        sF[t][lt * R + r] = ok ? pr[r] : 0.0f;
+            });
+            __syncthreads();
             // W = pQ / (A + eps)
 #pragma unroll
             for (int i = 0; i < CF::TPW_CS; ++i) {
@@ -350,7 +297,7 @@ __global__ __launch_bounds__(NW * 64) void race_fwd_readout(const ScanParams P)
                     const int r = acc_row(tm * 16, c.lane), col = acc_col(tn * 16, c.lane);
 #pragma unroll
                     for (int e = 0; e < 4; ++e)
-                        sW[r + e][col] = (T)(P.linear ? sF[r + e][col] : sF[r + e][col] * frcp(accA[i][e] + P.eps));
+                        sW[r + e][col] = (T)(sF[r + e][col] * frcp(accA[i][e] + P.eps));
                 }
             }
             __syncthreads();
@@ -387,10 +334,7 @@ __global__ __launch_bounds__(NW * 64) void race_fwd_readout(const ScanParams P)
                 if (t < MTC * CF::NTD) {
                     const int m0 = (t / CF::NTD) * 16, n0 = (t % CF::NTD) * 16;
                     mma_tile<E, C>(accO[i], &sPm[0][0], LDC, &sVt[0][0], LDC, m0, n0, c.lane);
-                    if constexpr (CF::QKV)
-                        store_out_tile(P.out, c.b, hq, c.st, t0, nv, P.D, m0, n0, c.lane, accO[i]);
-                    else
-                        store_out_tile(P.out, c.z, 0, c.st, t0, nv, P.D, m0, n0, c.lane, accO[i]);
+                    store_out_tile(P.out, c.b, hq, c.st, t0, nv, P.D, m0, n0, c.lane, accO[i]);
                 }
             }
         }
@@ -409,19 +353,14 @@ __global__ __launch_bounds__(NW * 64) void race_fwd_readout(const ScanParams P)
 }
 
 // ============================================================================ backward totals
-// op mode's fp32 64 x 64 tile: three 4-wave workgroups per CU (168 VGPRs) instead of two
-template <int MODE, int ST, int DP, int NW>
-constexpr int bwd_totals_waves_per_eu() { return MODE == 0 && ST == 64 && DP == 64 && NW == 4 ? 3 : 1; }
-
-template <class E, int MODE, int ST, int DP, int C, int NW>
-__global__ __launch_bounds__(NW * 64) __attribute__((amdgpu_waves_per_eu(bwd_totals_waves_per_eu<MODE, ST, DP, NW>())))
-void race_bwd_totals(const ScanParams P)
+template <class E, int ST, int DP, int C, int NW>
+__global__ __launch_bounds__(NW * 64) void race_bwd_totals(const ScanParams P)
 {
-    using CF = Cfg<E, MODE, ST, DP, C, NW>;
+    using CF = Cfg<E, ST, DP, C, NW>;
     using T = typename E::T;
     constexpr int PD = CF::PD, NTH = CF::NTH, MTC = CF::MTC;
     constexpr int LDX = DP + PD, LDC = C + PD, LDU = CF::LKPM + 1, LDF = ST + 4, LDG = CF::LKPM + PD;
-    constexpr int XR = CF::QKV ? C : 1;
+    constexpr int XR = C;
     constexpr int NCG = CF::TPW_CS / MTC;  // bucket-column groups per wave
     __shared__ __align__(16) T sX[XR][LDX];
     __shared__ __align__(16) T sV[C][LDX];
@@ -440,10 +379,8 @@ void race_bwd_totals(const ScanParams P)
     const Ctx c = make_ctx(P, ST);
     __builtin_assume(c.wave >= 0 && c.wave < NW);  // (threadIdx.x < NW * 64)
     PlaneFrags<E, CF> pf;
-    if constexpr (CF::QKV) {
-        pf.load(P, c);
-        zero_lds(&sGU[0][0], XR * LDG, c.tid, NTH);
-    }
+    pf.load(P, c);
+    zero_lds(&sGU[0][0], XR * LDG, c.tid, NTH);
     zero_lds(&sPKt[0][0], ST * LDC, c.tid, NTH);
     zero_lds(&sF[0][0], C * LDF, c.tid, NTH);
 
@@ -481,41 +418,22 @@ void race_bwd_totals(const ScanParams P)
     f32x4 accA[CF::TPW_CS], accW[CF::TPW_CS], accG[CF::TPW_CS], accGA[CF::TPW_CS];
     f32x4 accT[CF::TPW_SD];
     const int nsub = (c.t_end - c.t_begin + C - 1) / C;
-    // op mode: this sub-chunk's pK, values, pQ and output gradient wait in registers, fetched one
-    // sub-chunk ahead
-    SubChunkStage<C, ST, NTH> stK, stQ;
-    SubChunkStage<C, DP, NTH> stV, stG;
-    const float *srcK = P.pK + (int64_t)c.z * P.T * P.S, *srcQ = P.pQ + (int64_t)c.z * P.T * P.S;
-    const float *srcV = op_rows(P.V, P.v, P.zH, c.z), *srcG = op_rows(P.gO, P.go, P.zH, c.z);
-    auto fetch_op = [&](int t) {
-        stK.fetch(srcK, P.S, c.s0, c.S_here, t, P.T - 1, c.tid);
-        stV.fetch(srcV, (int)P.v.st, 0, P.D, t, P.T - 1, c.tid);
-        stQ.fetch(srcQ, P.S, c.s0, c.S_here, t, P.T - 1, c.tid);
-        stG.fetch(srcG, (int)P.go.st, 0, P.D, t, P.T - 1, c.tid);
-    };
-    if constexpr (!CF::QKV)
-        fetch_op(c.t_begin);
     for (int sc = 0; sc < nsub; ++sc) {
         const int t0 = c.t_begin + sc * C;
         const int nv = min(C, c.t_end - t0);
-        if constexpr (CF::QKV) {
-            load_rows_bf16<C, DP, NTH, LDX, LDC, true, false>(&sX[0][0], nullptr, P.k, c.b, c.hk, t0, nv, c.tid);
-            load_rows_bf16<C, DP, NTH, LDX, LDC, true, true>(&sV[0][0], &sVt[0][0], P.v, c.b, c.hk, t0, nv, c.tid);
-            __syncthreads();
-            project<E, CF, LDX, LDU>(&sX[0][0], &sU[0][0], pf, c, P.inv_scale);
-            __syncthreads();
-            const int R = P.R;
-            expand<CF, LDU>(&sU[0][0], c, P.K, [&](int t, int lt, const float *, const float *pr) {
-                const bool ok = t < nv;
+        load_rows_bf16<C, DP, NTH, LDX, LDC, true, false>(&sX[0][0], nullptr, P.k, c.b, c.hk, t0, nv, c.tid);
+        load_rows_bf16<C, DP, NTH, LDX, LDC, true, true>(&sV[0][0], &sVt[0][0], P.v, c.b, c.hk, t0, nv, c.tid);
+        __syncthreads();
+        project<E, CF, LDX, LDU>(&sX[0][0], &sU[0][0], pf, c, P.inv_scale);
+        __syncthreads();
+        const int R = P.R;
+        expand<CF, LDU>(&sU[0][0], c, P.K, [&](int t, int lt, const float *, const float *pr) {
+            const bool ok = t < nv;
 #pragma unroll
-                for (int r = 0; r < 16; ++r)
-                    if (r < R)
-                        sPKt[lt * R + r][t] = (T)(ok ? pr[r] : 0.0f);
-            });
-        } else {
-            stK.template put<T, LDC, LDC, false, true>(nullptr, &sPKt[0][0], nv, c.S_here, c.tid);
-            stV.template put<T, LDX, LDC, true, true>(&sV[0][0], &sVt[0][0], nv, P.D, c.tid);
-        }
+            for (int r = 0; r < 16; ++r)
+                if (r < R)
+                    sPKt[lt * R + r][t] = (T)(ok ? pr[r] : 0.0f);
+        });
         __syncthreads();
 
         float carry[CF::TPW_CS];
@@ -524,9 +442,7 @@ void race_bwd_totals(const ScanParams P)
             const int tm = i % MTC, tn = c.wave + (i / MTC) * NW;
             carry[i] = 0.0f;
             accA[i] = f32x4{0.f, 0.f, 0.f, 0.f};
-            if (tn < CF::NTS && P.linear) {
-                accA[i] = f32x4{1.f, 1.f, 1.f, 1.f};  // linear attention: W = pQ
-            } else if (tn < CF::NTS) {
+            if (tn < CF::NTS) {
                 const float a0 = sA0[tn * 16 + (c.lane & 15)];
                 accA[i] = f32x4{a0, a0, a0, a0};
                 mma_tile_gen<E, C>(accA[i], PredTrilIncl(), 1.0f, &sPKt[0][0], LDC, tm * 16, tn * 16, c.lane);
@@ -550,28 +466,22 @@ void race_bwd_totals(const ScanParams P)
 #pragma unroll
         for (int i = 0; i < CF::TPW_SD; ++i)
             accT[i] = f32x4{0.f, 0.f, 0.f, 0.f};
-        const int G = CF::QKV ? P.G : 1;
+        const int G = P.G;
         for (int g = 0; g < G; ++g) {
             const int hq = c.hk * P.G + g;
-            if constexpr (CF::QKV) {
-                load_rows_bf16<C, DP, NTH, LDX, LDC, true, false>(&sX[0][0], nullptr, P.q, c.b, hq, t0, nv, c.tid);
-                load_rows_bf16<C, DP, NTH, LDX, LDC, true, true>(&sGO[0][0], &sGOt[0][0], P.go, c.b, hq, t0, nv, c.tid);
-                __syncthreads();
-                project<E, CF, LDX, LDU>(&sX[0][0], &sU[0][0], pf, c, P.inv_scale);
-                __syncthreads();
-                const int R = P.R;
-                expand<CF, LDU>(&sU[0][0], c, P.K, [&](int t, int lt, const float *, const float *pr) {
-                    const bool ok = t < nv;
+            load_rows_bf16<C, DP, NTH, LDX, LDC, true, false>(&sX[0][0], nullptr, P.q, c.b, hq, t0, nv, c.tid);
+            load_rows_bf16<C, DP, NTH, LDX, LDC, true, true>(&sGO[0][0], &sGOt[0][0], P.go, c.b, hq, t0, nv, c.tid);
+            __syncthreads();
+            project<E, CF, LDX, LDU>(&sX[0][0], &sU[0][0], pf, c, P.inv_scale);
+            __syncthreads();
+            const int R = P.R;
+            expand<CF, LDU>(&sU[0][0], c, P.K, [&](int t, int lt, const float *, const float *pr) {
+                const bool ok = t < nv;
 #pragma unroll
-                    for (int r = 0; r < 16; ++r)
-                        if (r < R)
-                            sF[t][lt * R + r] = ok ? pr[r] : 0.0f;
-                });
-            } else {
-                stQ.template put<float, LDF, LDF, true, false>(&sF[0][0], nullptr, nv, c.S_here, c.tid);
-                stG.template put<T, LDX, LDC, true, true>(&sGO[0][0], &sGOt[0][0], nv, P.D, c.tid);
-                fetch_op(t0 + C);  // next sub-chunk (op mode has one query head: once per sub-chunk)
-            }
+                for (int r = 0; r < 16; ++r)
+                    if (r < R)
+                        sF[t][lt * R + r] = ok ? pr[r] : 0.0f;
+            });
             __syncthreads();
             // W = pQ/(A+eps) -> sWt ; gW = go St^T ; Mg = tril(go V^T)
 #pragma unroll
@@ -610,16 +520,12 @@ void race_bwd_totals(const ScanParams P)
                 const int tm = i % MTC, tn = c.wave + (i / MTC) * NW;
                 if (tn < CF::NTS) {
                     mma_tile<E, C>(accG[i], &sMg[0][0], LDC, &sPKt[0][0], LDC, tm * 16, tn * 16, c.lane);
-                    if (!P.linear)
-                        ga_accum(accGA[i], accG[i], accA[i], accW[i]);
+                    ga_accum(accGA[i], accG[i], accA[i], accW[i]);
                     f32x4 gpq;
 #pragma unroll
                     for (int e = 0; e < 4; ++e)
                         gpq[e] = accG[i][e] * accA[i][e];
                     accG[i] = gpq;
-                    if constexpr (!CF::QKV)
-                        store_probs_tile(P.gpQ + (int64_t)c.z * P.T * P.S, P.S, c.s0, c.S_here, t0, nv,
-                                         tm * 16, tn * 16, c.lane, gpq);
                 }
             }
 #pragma unroll
@@ -629,42 +535,40 @@ void race_bwd_totals(const ScanParams P)
                     mma_tile<E, C>(accT[i], &sWt[0][0], LDC, &sGOt[0][0], LDC, (t / CF::NTD) * 16,
                                    (t % CF::NTD) * 16, c.lane);
             }
-            if constexpr (CF::QKV) {
-                // dq through the soft-hash backward
+            // dq through the soft-hash backward
 #pragma unroll
-                for (int i = 0; i < CF::TPW_CS; ++i) {
-                    const int tm = i % MTC, tn = c.wave + (i / MTC) * NW;
-                    if (tn < CF::NTS)
-                        st_rm(&sF[0][0], LDF, tm * 16, tn * 16, c.lane, accG[i]);
-                }
-                __syncthreads();
-                const int R = P.R, K = P.K;
-                const float scale = P.scale, inv_scale = P.inv_scale;
-                expand<CF, LDU>(&sU[0][0], c, K, [&](int t, int lt, const float *u, const float *pr) {
-                    float gp[16], gproj[4];
+            for (int i = 0; i < CF::TPW_CS; ++i) {
+                const int tm = i % MTC, tn = c.wave + (i / MTC) * NW;
+                if (tn < CF::NTS)
+                    st_rm(&sF[0][0], LDF, tm * 16, tn * 16, c.lane, accG[i]);
+            }
+            __syncthreads();
+            const int K = P.K;
+            const float scale = P.scale, inv_scale = P.inv_scale;
+            expand<CF, LDU>(&sU[0][0], c, K, [&](int t, int lt, const float *u, const float *pr) {
+                float gp[16], gproj[4];
 #pragma unroll
-                    for (int r = 0; r < 16; ++r)
-                        gp[r] = (r < R) ? sF[t][lt * R + r] : 0.0f;
-                    softhash_bwd(u, pr, gp, K, scale, inv_scale, gproj);
+                for (int r = 0; r < 16; ++r)
+                    gp[r] = (r < R) ? sF[t][lt * R + r] : 0.0f;
+                softhash_bwd(u, pr, gp, K, scale, inv_scale, gproj);
 #pragma unroll
-                    for (int k = 0; k < 4; ++k)
-                        if (k < K)
-                            sGU[t][lt * K + k] = (T)gproj[k];
-                });
-                __syncthreads();
+                for (int k = 0; k < 4; ++k)
+                    if (k < K)
+                        sGU[t][lt * K + k] = (T)gproj[k];
+            });
+            __syncthreads();
 #pragma unroll
-                for (int i = 0; i < CF::TPW_CD; ++i) {
-                    const int t = c.wave + i * NW;
-                    if (t < MTC * CF::NTD) {
-                        const int m0 = (t / CF::NTD) * 16, n0 = (t % CF::NTD) * 16;
-                        f32x4 acc = {0.f, 0.f, 0.f, 0.f};
-                        const T *pa = &sGU[0][0] + (m0 + (c.lane & 15)) * LDG + (c.lane >> 4) * E::KPL;
+            for (int i = 0; i < CF::TPW_CD; ++i) {
+                const int t = c.wave + i * NW;
+                if (t < MTC * CF::NTD) {
+                    const int m0 = (t / CF::NTD) * 16, n0 = (t % CF::NTD) * 16;
+                    f32x4 acc = {0.f, 0.f, 0.f, 0.f};
+                    const T *pa = &sGU[0][0] + (m0 + (c.lane & 15)) * LDG + (c.lane >> 4) * E::KPL;
 #pragma unroll
-                        for (int kb = 0; kb < CF::KB_L; ++kb)
-                            if (kb * E::KSTEP < c.LKP)
-                                E::mma(acc, E::ld(pa + kb * E::KSTEP), pf.back[i][kb]);
-                        store_out_tile(P.dq, c.b, hq, c.st, t0, nv, P.D, m0, n0, c.lane, acc);
-                    }
+                    for (int kb = 0; kb < CF::KB_L; ++kb)
+                        if (kb * E::KSTEP < c.LKP)
+                            E::mma(acc, E::ld(pa + kb * E::KSTEP), pf.back[i][kb]);
+                    store_out_tile(P.dq, c.b, hq, c.st, t0, nv, P.D, m0, n0, c.lane, acc);
                 }
             }
             __syncthreads();
@@ -723,20 +627,15 @@ void race_bwd_totals(const ScanParams P)
 // backward totals kernel added (see ga_accum), so the subtraction cancels exactly:
 //   dS_end(c)   = dS_start(c) - W_c^T go_c
 //   gAhat_end(c)= gAhat_start(c) - colsum(gA_c)
-// two 8-wave workgroups per CU where the 64 x 64 tile's LDS allows them (81.7 KB): 128 VGPRs
-template <int ST, int DP, int NW>
-constexpr int bwd_main_waves_per_eu() { return ST == 64 && DP == 64 && NW == 8 ? 4 : 1; }
-
-template <class E, int MODE, int ST, int DP, int C, int NW>
-__global__ __launch_bounds__(NW * 64) __attribute__((amdgpu_waves_per_eu(bwd_main_waves_per_eu<ST, DP, NW>())))
-void race_bwd_main(const ScanParams P)
+template <class E, int ST, int DP, int C, int NW>
+__global__ __launch_bounds__(NW * 64) void race_bwd_main(const ScanParams P)
 {
-    using CF = Cfg<E, MODE, ST, DP, C, NW>;
+    using CF = Cfg<E, ST, DP, C, NW>;
     using T = typename E::T;
     constexpr int PD = CF::PD, NTH = CF::NTH, MTC = CF::MTC;
     constexpr int LDX = DP + PD, LDC = C + PD, LDS_ = ST + PD, LDU = CF::LKPM + 1, LDF = ST + 4;
     constexpr int LDG = CF::LKPM + PD;
-    constexpr int XR = CF::QKV ? C : 1;
+    constexpr int XR = C;
     __shared__ __align__(16) T sX[XR][LDX];
     __shared__ __align__(16) T sV[C][LDX];
     __shared__ __align__(16) T sVt[DP][LDC];
@@ -761,14 +660,13 @@ void race_bwd_main(const ScanParams P)
     __shared__ __align__(16) T sMp[C][LDC];
     __shared__ float sA0[ST];
     __shared__ double sGAe[ST];  // suffix of gA after the current sub-chunk (fp64)
-    static_assert(!CF::QKV || sizeof(T) * XR * LDG <= sizeof(float) * XR * LDU, "sGU alias");
+    static_assert(sizeof(T) * XR * LDG <= sizeof(float) * XR * LDU, "sGU alias");
     T *sGU = reinterpret_cast<T *>(&sUq[0][0]);
 
     const Ctx c = make_ctx(P, ST);
     __builtin_assume(c.wave >= 0 && c.wave < NW);  // (threadIdx.x < NW * 64)
     PlaneFrags<E, CF> pf;
-    if constexpr (CF::QKV)
-        pf.load(P, c);
+    pf.load(P, c);
     zero_lds(&sPK[0][0], C * LDS_, c.tid, NTH);
     zero_lds(&sPKt[0][0], ST * LDC, c.tid, NTH);
     zero_lds(&sF[0][0], C * LDF, c.tid, NTH);
@@ -811,44 +709,25 @@ void race_bwd_main(const ScanParams P)
     f32x4 accA[CF::TPW_CS], accW[CF::TPW_CS], accG[CF::TPW_CS], accGA[CF::TPW_CS], accPK[CF::TPW_CS];
     f32x4 accV[CF::TPW_CD], accT[CF::TPW_SD];
     const int nsub = (c.t_end - c.t_begin + C - 1) / C;
-    // op mode: this sub-chunk's pK, values, pQ and output gradient wait in registers, fetched one
-    // sub-chunk ahead
-    SubChunkStage<C, ST, NTH> stK, stQ;
-    SubChunkStage<C, DP, NTH> stV, stG;
-    const float *srcK = P.pK + (int64_t)c.z * P.T * P.S, *srcQ = P.pQ + (int64_t)c.z * P.T * P.S;
-    const float *srcV = op_rows(P.V, P.v, P.zH, c.z), *srcG = op_rows(P.gO, P.go, P.zH, c.z);
-    auto fetch_op = [&](int t) {
-        stK.fetch(srcK, P.S, c.s0, c.S_here, t, P.T - 1, c.tid);
-        stV.fetch(srcV, (int)P.v.st, 0, P.D, t, P.T - 1, c.tid);
-        stQ.fetch(srcQ, P.S, c.s0, c.S_here, t, P.T - 1, c.tid);
-        stG.fetch(srcG, (int)P.go.st, 0, P.D, t, P.T - 1, c.tid);
-    };
-    if constexpr (!CF::QKV)
-        fetch_op(c.t_begin);
     for (int sc = 0; sc < nsub; ++sc) {
         const int t0 = c.t_begin + sc * C;
         const int nv = min(C, c.t_end - t0);
-        if constexpr (CF::QKV) {
-            load_rows_bf16<C, DP, NTH, LDX, LDC, true, false>(&sX[0][0], nullptr, P.k, c.b, c.hk, t0, nv, c.tid);
-            load_rows_bf16<C, DP, NTH, LDX, LDC, true, true>(&sV[0][0], &sVt[0][0], P.v, c.b, c.hk, t0, nv, c.tid);
-            __syncthreads();
-            project<E, CF, LDX, LDU>(&sX[0][0], &sUk[0][0], pf, c, P.inv_scale);
-            __syncthreads();
-            const int R = P.R;
-            expand<CF, LDU>(&sUk[0][0], c, P.K, [&](int t, int lt, const float *, const float *pr) {
-                const bool ok = t < nv;
+        load_rows_bf16<C, DP, NTH, LDX, LDC, true, false>(&sX[0][0], nullptr, P.k, c.b, c.hk, t0, nv, c.tid);
+        load_rows_bf16<C, DP, NTH, LDX, LDC, true, true>(&sV[0][0], &sVt[0][0], P.v, c.b, c.hk, t0, nv, c.tid);
+        __syncthreads();
+        project<E, CF, LDX, LDU>(&sX[0][0], &sUk[0][0], pf, c, P.inv_scale);
+        __syncthreads();
+        const int R = P.R;
+        expand<CF, LDU>(&sUk[0][0], c, P.K, [&](int t, int lt, const float *, const float *pr) {
+            const bool ok = t < nv;
 #pragma unroll
-                for (int r = 0; r < 16; ++r)
-                    if (r < R) {
-                        const T x = (T)(ok ? pr[r] : 0.0f);
-                        sPK[t][lt * R + r] = x;
-                        sPKt[lt * R + r][t] = x;
-                    }
-            });
-        } else {
-            stK.template put<T, LDS_, LDC, true, true>(&sPK[0][0], &sPKt[0][0], nv, c.S_here, c.tid);
-            stV.template put<T, LDX, LDC, true, true>(&sV[0][0], &sVt[0][0], nv, P.D, c.tid);
-        }
+            for (int r = 0; r < 16; ++r)
+                if (r < R) {
+                    const T x = (T)(ok ? pr[r] : 0.0f);
+                    sPK[t][lt * R + r] = x;
+                    sPKt[lt * R + r][t] = x;
+                }
+        });
         // the state at this sub-chunk's start, for gW = go St^T
 #pragma unroll
         for (int i = 0; i < CF::TPW_SD; ++i) {
@@ -867,9 +746,7 @@ void race_bwd_main(const ScanParams P)
             accA[i] = f32x4{0.f, 0.f, 0.f, 0.f};
             accGA[i] = f32x4{0.f, 0.f, 0.f, 0.f};
             accPK[i] = f32x4{0.f, 0.f, 0.f, 0.f};
-            if (tn < CF::NTS && P.linear) {
-                accA[i] = f32x4{1.f, 1.f, 1.f, 1.f};  // linear attention: W = pQ
-            } else if (tn < CF::NTS) {
+            if (tn < CF::NTS) {
                 const float a0 = sA0[tn * 16 + (c.lane & 15)];
                 accA[i] = f32x4{a0, a0, a0, a0};
                 mma_tile_gen<E, C>(accA[i], PredTrilIncl(), 1.0f, &sPKt[0][0], LDC, tm * 16, tn * 16, c.lane);
@@ -893,28 +770,22 @@ void race_bwd_main(const ScanParams P)
                 sA0[tn * 16 + (c.lane & 15)] = carry[i];
         }
 
-        const int G = CF::QKV ? P.G : 1;
+        const int G = P.G;
         for (int g = 0; g < G; ++g) {
             const int hq = c.hk * P.G + g;
-            if constexpr (CF::QKV) {
-                load_rows_bf16<C, DP, NTH, LDX, LDC, true, false>(&sX[0][0], nullptr, P.q, c.b, hq, t0, nv, c.tid);
-                load_rows_bf16<C, DP, NTH, LDX, LDC, true, true>(&sGO[0][0], &sGOt[0][0], P.go, c.b, hq, t0, nv, c.tid);
-                __syncthreads();
-                project<E, CF, LDX, LDU>(&sX[0][0], &sUq[0][0], pf, c, P.inv_scale);
-                __syncthreads();
-                const int R = P.R;
-                expand<CF, LDU>(&sUq[0][0], c, P.K, [&](int t, int lt, const float *, const float *pr) {
-                    const bool ok = t < nv;
+            load_rows_bf16<C, DP, NTH, LDX, LDC, true, false>(&sX[0][0], nullptr, P.q, c.b, hq, t0, nv, c.tid);
+            load_rows_bf16<C, DP, NTH, LDX, LDC, true, true>(&sGO[0][0], &sGOt[0][0], P.go, c.b, hq, t0, nv, c.tid);
+            __syncthreads();
+            project<E, CF, LDX, LDU>(&sX[0][0], &sUq[0][0], pf, c, P.inv_scale);
+            __syncthreads();
+            const int R = P.R;
+            expand<CF, LDU>(&sUq[0][0], c, P.K, [&](int t, int lt, const float *, const float *pr) {
+                const bool ok = t < nv;
 #pragma unroll
-                    for (int r = 0; r < 16; ++r)
-                        if (r < R)
-                            sF[t][lt * R + r] = ok ? pr[r] : 0.0f;
-                });
-            } else {
-                stQ.template put<float, LDF, LDF, true, false>(&sF[0][0], nullptr, nv, c.S_here, c.tid);
-                stG.template put<T, LDX, LDC, true, true>(&sGO[0][0], &sGOt[0][0], nv, P.D, c.tid);
-                fetch_op(t0 + C);  // next sub-chunk (op mode has one query head: once per sub-chunk)
-            }
+                for (int r = 0; r < 16; ++r)
+                    if (r < R)
+                        sF[t][lt * R + r] = ok ? pr[r] : 0.0f;
+            });
             __syncthreads();
             // W -> sW, sWt ; gW = go St^T ; Mg = tril(go V^T) -> sMg, sMv
 #pragma unroll
@@ -971,8 +842,7 @@ void race_bwd_main(const ScanParams P)
                 const int tm = i % MTC, tn = c.wave + (i / MTC) * NW;
                 if (tn < CF::NTS) {
                     mma_tile<E, C>(accG[i], &sMg[0][0], LDC, &sPKt[0][0], LDC, tm * 16, tn * 16, c.lane);
-                    if (!P.linear)
-                        ga_accum(accGA[i], accG[i], accA[i], accW[i]);
+                    ga_accum(accGA[i], accG[i], accA[i], accW[i]);
                     mma_tile<E, C>(accPK[i], &sMv[0][0], LDC, &sWt[0][0], LDC, tm * 16, tn * 16, c.lane);
                 }
             }
@@ -1013,24 +883,22 @@ void race_bwd_main(const ScanParams P)
                 st_cm(&sdSt[0][0], LDS_, m0, n0, c.lane, accDS[i]);
             }
         }
-        if (!P.linear) {  // (grid-uniform) linear attention has no gA
 #pragma unroll
-            for (int j = 0; j < CF::TPW_CS / MTC; ++j) {
-                const float tot = col_total<MTC>(accGA, j);
-                const int tn = c.wave + j * NW;
-                if (tn < CF::NTS && c.lane < 16)
-                    sGAe[tn * 16 + c.lane] -= (double)tot;
-            }
+        for (int j = 0; j < CF::TPW_CS / MTC; ++j) {
+            const float tot = col_total<MTC>(accGA, j);
+            const int tn = c.wave + j * NW;
+            if (tn < CF::NTS && c.lane < 16)
+                sGAe[tn * 16 + c.lane] -= (double)tot;
+        }
 #pragma unroll
-            for (int i = 0; i < CF::TPW_CS; ++i) {
-                const int tm = i % MTC, tn = c.wave + (i / MTC) * NW;
-                if (tn < CF::NTS)
-                    st_rm(&sF[0][0], LDF, tm * 16, tn * 16, c.lane, accGA[i]);
-            }
+        for (int i = 0; i < CF::TPW_CS; ++i) {
+            const int tm = i % MTC, tn = c.wave + (i / MTC) * NW;
+            if (tn < CF::NTS)
+                st_rm(&sF[0][0], LDF, tm * 16, tn * 16, c.lane, accGA[i]);
         }
         __syncthreads();
         // gAhat_t = gAhat_end + sum_{tau>=t, tau in this sub-chunk} gA_tau
-        for (int s = c.tid; s < ST && !P.linear; s += NTH) {
+        for (int s = c.tid; s < ST; s += NTH) {
             float run = (float)sGAe[s];
             for (int t = C - 1; t >= 0; --t) {
                 run += sF[t][s];
@@ -1057,16 +925,10 @@ void race_bwd_main(const ScanParams P)
             const int tm = i % MTC, tn = c.wave + (i / MTC) * NW;
             if (tn < CF::NTS) {
                 const int r = acc_row(tm * 16, c.lane), col = acc_col(tn * 16, c.lane);
-                if (!P.linear) {
 #pragma unroll
-                    for (int e = 0; e < 4; ++e)
-                        accPK[i][e] += sF[r + e][col];
-                }
-                if constexpr (CF::QKV)
-                    st_rm(&sF[0][0], LDF, tm * 16, tn * 16, c.lane, accPK[i]);
-                else
-                    store_probs_tile(P.gpK + (int64_t)c.z * P.T * P.S, P.S, c.s0, c.S_here, t0, nv,
-                                     tm * 16, tn * 16, c.lane, accPK[i]);
+                for (int e = 0; e < 4; ++e)
+                    accPK[i][e] += sF[r + e][col];
+                st_rm(&sF[0][0], LDF, tm * 16, tn * 16, c.lane, accPK[i]);
             }
         }
 #pragma unroll
@@ -1074,44 +936,39 @@ void race_bwd_main(const ScanParams P)
             const int t = c.wave + i * NW;
             if (t < MTC * CF::NTD) {
                 const int m0 = (t / CF::NTD) * 16, n0 = (t % CF::NTD) * 16;
-                if constexpr (CF::QKV)
-                    store_out_tile(P.dv, c.b, c.hk, c.st, t0, nv, P.D, m0, n0, c.lane, accV[i]);
-                else
-                    store_out_tile(P.dv, c.z, 0, c.st, t0, nv, P.D, m0, n0, c.lane, accV[i]);
+                store_out_tile(P.dv, c.b, c.hk, c.st, t0, nv, P.D, m0, n0, c.lane, accV[i]);
             }
         }
-        if constexpr (CF::QKV) {
-            // dk through the soft-hash backward (sGU aliases sUq, whose q values are dead)
-            for (int i = c.tid; i < C * LDG; i += NTH)
-                sGU[i] = (T)0.0f;
-            __syncthreads();
-            const int R = P.R, K = P.K;
-            const float scale = P.scale, inv_scale = P.inv_scale;
-            expand<CF, LDU>(&sUk[0][0], c, K, [&](int t, int lt, const float *u, const float *pr) {
-                float gp[16], gproj[4];
+        // dk through the soft-hash backward (sGU aliases sUq, whose q values are dead)
+        for (int i = c.tid; i < C * LDG; i += NTH)
+            sGU[i] = (T)0.0f;
+        __syncthreads();
+        const int K = P.K;
+        const float scale = P.scale, inv_scale = P.inv_scale;
+        expand<CF, LDU>(&sUk[0][0], c, K, [&](int t, int lt, const float *u, const float *pr) {
+            float gp[16], gproj[4];
 #pragma unroll
-                for (int r = 0; r < 16; ++r)
-                    gp[r] = (r < R) ? sF[t][lt * R + r] : 0.0f;
-                softhash_bwd(u, pr, gp, K, scale, inv_scale, gproj);
+            for (int r = 0; r < 16; ++r)
+                gp[r] = (r < R) ? sF[t][lt * R + r] : 0.0f;
+            softhash_bwd(u, pr, gp, K, scale, inv_scale, gproj);
 #pragma unroll
-                for (int k = 0; k < 4; ++k)
-                    if (k < K)
-                        sGU[t * LDG + lt * K + k] = (T)gproj[k];
-            });
-            __syncthreads();
+            for (int k = 0; k < 4; ++k)
+                if (k < K)
+                    sGU[t * LDG + lt * K + k] = (T)gproj[k];
+        });
+        __syncthreads();
 #pragma unroll
-            for (int i = 0; i < CF::TPW_CD; ++i) {
-                const int t = c.wave + i * NW;
-                if (t < MTC * CF::NTD) {
-                    const int m0 = (t / CF::NTD) * 16, n0 = (t % CF::NTD) * 16;
-                    f32x4 acc = {0.f, 0.f, 0.f, 0.f};
-                    const T *pa = sGU + (m0 + (c.lane & 15)) * LDG + (c.lane >> 4) * E::KPL;
+        for (int i = 0; i < CF::TPW_CD; ++i) {
+            const int t = c.wave + i * NW;
+            if (t < MTC * CF::NTD) {
+                const int m0 = (t / CF::NTD) * 16, n0 = (t % CF::NTD) * 16;
+                f32x4 acc = {0.f, 0.f, 0.f, 0.f};
+                const T *pa = sGU + (m0 + (c.lane & 15)) * LDG + (c.lane >> 4) * E::KPL;
 #pragma unroll
-                    for (int kb = 0; kb < CF::KB_L; ++kb)
-                        if (kb * E::KSTEP < c.LKP)
-                            E::mma(acc, E::ld(pa + kb * E::KSTEP), pf.back[i][kb]);
-                    store_out_tile(P.dk, c.b, c.hk, c.st, t0, nv, P.D, m0, n0, c.lane, acc);
-                }
+                for (int kb = 0; kb < CF::KB_L; ++kb)
+                    if (kb * E::KSTEP < c.LKP)
+                        E::mma(acc, E::ld(pa + kb * E::KSTEP), pf.back[i][kb]);
+                store_out_tile(P.dk, c.b, c.hk, c.st, t0, nv, P.D, m0, n0, c.lane, acc);
             }
         }
         // St += pK^T V

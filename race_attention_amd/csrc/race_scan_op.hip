@@ -1,48 +1,63 @@
-// fp32 probabilities-in instantiations of the scan kernels (MODE_OP, EngF32).
+// Instantiations of the fp32 op-path scan kernels (race_op_scan.h), one per bucket tile and padded
+// head dim, and their dispatch.
 #include "race_launch.h"
-#include "race_scan_kernels.h"
+#include "race_op_scan.h"
 
 namespace race {
 
-template <int ST, int DP>
-static hipError_t launch_v(ScanKernel k, const ScanParams &P, dim3 grid, hipStream_t s)
+template <int ST, int DP, bool VEC>
+static hipError_t launch_v(OpKernel k, const ScanParams &P, dim3 grid, hipStream_t s)
 {
-    constexpr int C = OP_C, NWT = OP_NW_TOTALS, NWM = op_nw_main(DP);
+    // the bucket kernels of a 128-bucket tile run as two workgroups of 64 buckets: V and gO are
+    // read twice, but two or three independent workgroups share a CU instead of one (before the
+    // suffixes moved to fp64, 200003 tokens x 4 streams, S = 128, D = 64: gq 565 -> 535, gk 521 ->
+    // 508 us; 32 buckets: 785 and 560)
+    constexpr int BT = ST < 64 ? ST : 64;
+    const dim3 bucket(BT * 4), value(OpCfg<ST, DP>::DW * 64);
+    const dim3 bgrid(grid.x, grid.y * (ST / BT), grid.z);
     switch (k) {
-    case K_FWD_TOTALS:
-        hipLaunchKernelGGL((race_fwd_totals<EngF32, MODE_OP, ST, DP, C, NWT>), grid, dim3(NWT * 64), 0, s, P);
+    case OP_TOTALS:
+        hipLaunchKernelGGL((race_op_totals<BT, DP, VEC>), bgrid, bucket, 0, s, P);
         break;
-    case K_FWD_READOUT:
-        hipLaunchKernelGGL((race_fwd_readout<EngF32, MODE_OP, ST, DP, C, NWM>), grid, dim3(NWM * 64), 0, s, P);
+    case OP_READOUT:
+        if (P.linear)
+            hipLaunchKernelGGL((race_op_out<ST, DP, false, true, VEC>), grid, value, 0, s, P);
+        else
+            hipLaunchKernelGGL((race_op_out<ST, DP, false, false, VEC>), grid, value, 0, s, P);
         break;
-    case K_BWD_TOTALS:
-        hipLaunchKernelGGL((race_bwd_totals<EngF32, MODE_OP, ST, DP, C, NWT>), grid, dim3(NWT * 64), 0, s, P);
+    case OP_GQ:
+        if (P.linear)
+            hipLaunchKernelGGL((race_op_gq<BT, DP, true, VEC>), bgrid, bucket, 0, s, P);
+        else
+            hipLaunchKernelGGL((race_op_gq<BT, DP, false, VEC>), bgrid, bucket, 0, s, P);
         break;
-    case K_BWD_MAIN:
-        hipLaunchKernelGGL((race_bwd_main<EngF32, MODE_OP, ST, DP, C, NWM>), grid, dim3(NWM * 64), 0, s, P);
+    case OP_GK:
+        if (P.linear)
+            hipLaunchKernelGGL((race_op_gk<BT, DP, true, VEC>), bgrid, bucket, 0, s, P);
+        else
+            hipLaunchKernelGGL((race_op_gk<BT, DP, false, VEC>), bgrid, bucket, 0, s, P);
+        break;
+    case OP_GV:
+        if (P.linear)
+            hipLaunchKernelGGL((race_op_out<ST, DP, true, true, VEC>), grid, value, 0, s, P);
+        else
+            hipLaunchKernelGGL((race_op_out<ST, DP, true, false, VEC>), grid, value, 0, s, P);
         break;
     }
     return hipGetLastError();
 }
 
-// (ST, DP) with ST * DP <= 4096 (fp32 operands and three state copies in LDS)
 #define RACE_OP_VARIANTS(X) \
     X(16, 32) X(32, 32) X(64, 32) X(128, 32) \
-    X(16, 64) X(32, 64) X(64, 64) \
-    X(16, 128) X(32, 128) \
-    X(16, 256)
+    X(16, 64) X(32, 64) X(64, 64) X(128, 64) \
+    X(16, 128) X(32, 128) X(64, 128) X(128, 128) \
+    X(16, 256) X(32, 256) X(64, 256) X(128, 256)
 
-bool op_variant_exists(int ST, int DP)
-{
-#define X(a, b) if (ST == a && DP == b) return true;
-    RACE_OP_VARIANTS(X)
-#undef X
-    return false;
-}
+int op_stage_tokens(int DP) { return op_stage(DP); }
 
-hipError_t launch_scan_op(ScanKernel k, int ST, int DP, const ScanParams &P, dim3 grid, hipStream_t s)
+hipError_t launch_scan_op(OpKernel k, int ST, int DP, const ScanParams &P, dim3 grid, hipStream_t s)
 {
-#define X(a, b) if (ST == a && DP == b) return launch_v<a, b>(k, P, grid, s);
+#define X(a, b) if (ST == a && DP == b) return P.vec ? launch_v<a, b, true>(k, P, grid, s) : launch_v<a, b, false>(k, P, grid, s);
     RACE_OP_VARIANTS(X)
 #undef X
     return hipErrorInvalidValue;

@@ -1,4 +1,4 @@
-// bf16 fused q/k/v instantiations of the scan kernels (MODE_QKV, EngBF16).
+// bf16 fused q/k/v instantiations of the scan kernels (EngBF16).
 #include "race_launch.h"
 #include "race_scan_kernels.h"
 
@@ -11,16 +11,16 @@ static hipError_t launch_v(ScanKernel k, const ScanParams &P, dim3 grid, hipStre
     const dim3 block(NW * 64);
     switch (k) {
     case K_FWD_TOTALS:
-        hipLaunchKernelGGL((race_fwd_totals<EngBF16, MODE_QKV, ST, DP, C, NW>), grid, block, 0, s, P);
+        hipLaunchKernelGGL((race_fwd_totals<EngBF16, ST, DP, C, NW>), grid, block, 0, s, P);
         break;
     case K_FWD_READOUT:
-        hipLaunchKernelGGL((race_fwd_readout<EngBF16, MODE_QKV, ST, DP, C, NW>), grid, block, 0, s, P);
+        hipLaunchKernelGGL((race_fwd_readout<EngBF16, ST, DP, C, NW>), grid, block, 0, s, P);
         break;
     case K_BWD_TOTALS:
-        hipLaunchKernelGGL((race_bwd_totals<EngBF16, MODE_QKV, ST, DP, C, NW>), grid, block, 0, s, P);
+        hipLaunchKernelGGL((race_bwd_totals<EngBF16, ST, DP, C, NW>), grid, block, 0, s, P);
         break;
     case K_BWD_MAIN:
-        hipLaunchKernelGGL((race_bwd_main<EngBF16, MODE_QKV, ST, DP, C, NW>), grid, block, 0, s, P);
+        hipLaunchKernelGGL((race_bwd_main<EngBF16, ST, DP, C, NW>), grid, block, 0, s, P);
         break;
     }
     return hipGetLastError();

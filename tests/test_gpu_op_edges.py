@@ -1,0 +1,86 @@
+"""The fp32 op-path kernels at the edges of their tiles, against the fp64 oracle: sub-chunks of 16
+tokens, stages of 16 / 32, bucket tiles of 16 .. 128 (and several), head-dim tiles of 32 .. 256, and
+operands whose rows are not 16-byte aligned, which move as single floats.
+
+Bars as tests/test_gpu_op.py: forward 2e-5, gradients 1e-4 or twice what the reference formula itself
+loses in fp32 (gradProbsK cancels at a sequence's first tokens)."""
+import pytest
+import torch
+
+from oracle import race_oracle as orc
+from race_ref import check, fp32_formula_floor, make_probs, oracle_op
+
+pytestmark = pytest.mark.gpu
+EPS = 1e-6
+
+
+def probs(N, T, S, D, seed):
+    pk, pq, v, go = make_probs(N, T, 1, S, D, seed, "raw")
+    return pk + 0.05, pq, v, go  # (bounded away from 0: the bars are those of ordinary masses)
+
+
+@pytest.mark.parametrize("N,T,S,D,block", [
+    (1, 15, 15, 30, 0), (2, 16, 16, 32, 0), (2, 17, 17, 33, 0), (3, 31, 32, 64, 16), (1, 33, 33, 65, 0),
+    (2, 65, 64, 128, 48), (2, 129, 65, 129, 0), (1, 200, 128, 64, 80), (2, 97, 129, 64, 0), (1, 70, 300, 96, 32),
+    (1, 1, 128, 256, 0), (2, 130, 127, 255, 64)])
+def test_tile_edges(dev, N, T, S, D, block):
+    from race_attention_amd.race_causal_cuda import race_backward, race_fused_fwd
+    print(f"edges N={N} T={T} S={S} D={D} block={block}", flush=True)
+    pk, pq, v, go = probs(N, T, S, D, seed=T + S + D)
+    out_t, gpk_t, gpq_t, gv_t, _, _ = oracle_op(pk, pq, v, go, EPS)
+    pkc, pqc, vc, goc = (x.float().to(dev) for x in (pk, pq, v, go))
+    check("out", race_fused_fwd(pkc, pqc, vc, EPS, block), out_t, 2e-5)
+    floors = fp32_formula_floor(pk, pq, v, go, EPS, (gpk_t, gpq_t, gv_t))
+    for name, g, ref, f in zip(("gpK", "gpQ", "gV"), race_backward(pkc, pqc, vc, goc, EPS, block),
+                               (gpk_t, gpq_t, gv_t), floors):
+        check(name, g, ref, max(1e-4, 2.0 * f))
+
+
+@pytest.mark.parametrize("T,E,M", [(15, 15, 31), (16, 16, 32), (33, 17, 64), (65, 64, 65), (100, 129, 128)])
+def test_linear_tile_edges(dev, T, E, M):
+    from race_attention_amd.linear_attention import causal_linear_attention
+    g = torch.Generator().manual_seed(T)
+    Q, K, V, G = (torch.randn(2, 1, T, n, generator=g) for n in (E, E, M, M))
+    ref_in = [x.double().requires_grad_() for x in (Q, K, V)]
+    ref = orc.causal_linear_ref(*ref_in)
+    ref.backward(G.double())
+    got_in = [x.to(dev).requires_grad_() for x in (Q, K, V)]
+    got = causal_linear_attention(*got_in)
+    got.backward(G.to(dev))
+    # sums of at most T * E products of O(1) terms in fp32
+    check("out", got, ref, 2e-5)
+    for name, a, b in zip("QKV", got_in, ref_in):
+        check("g" + name, a.grad, b.grad, 2e-5)
+
+
+@pytest.mark.parametrize("S,D", [(24, 64), (128, 128), (64, 256)])
+def test_unaligned_rows_equal_aligned_ones(dev, S, D):
+    """Rows that start 4 bytes off a 16-byte boundary take the kernels that move single floats: the
+    same arithmetic, so the results are bitwise those of the aligned operands."""
+    from race_attention_amd.race_causal_cuda import race_backward, race_fused_fwd
+    args = [x.float().to(dev) for x in probs(2, 150, S, D, seed=S)]
+
+    def shifted(x):
+        buf = torch.empty(x.numel() + 1, device=dev)
+        y = buf[1:].view(x.shape)
+        y.copy_(x)
+        assert y.data_ptr() % 16 == 4 and y.is_contiguous()
+        return y
+
+    off = [shifted(x) for x in args]
+    assert torch.equal(race_fused_fwd(*args[:3], EPS), race_fused_fwd(*off[:3], EPS))
+    for name, a, b in zip(("gpK", "gpQ", "gV"), race_backward(*args, EPS), race_backward(*off, EPS)):
+        assert torch.equal(a, b), name
+
+
+def test_values_beyond_a_block_do_not_leak(dev):
+    """A non-finite value row reaches the outputs of its own and later tokens only: rows behind a
+    block's or a sequence's end are read as zeros, never multiplied by zero probabilities."""
+    from race_attention_amd.race_causal_cuda import race_fused_fwd
+    pk, pq, v, _ = (x.float().to(dev) for x in probs(2, 96, 24, 64, seed=3))
+    clean = race_fused_fwd(pk, pq, v, EPS, 48)
+    v[0, 48] = float("nan")  # first row of the second block
+    v[1, 0] = float("inf")   # first row of the second stream
+    out = race_fused_fwd(pk, pq, v, EPS, 48)
+    assert torch.equal(out[0, :48], clean[0, :48])
+    assert not torch.isfinite(out[0, 48:]).any()
