@@ -10,6 +10,8 @@
 #include "race_launch.h"
 #include "race_softhash.h"
 
+#include <type_traits>
+
 namespace race {
 
 // ============================================================================ block scan
@@ -1173,111 +1175,136 @@ hipError_t softhash_prepare(int D, int LK)
 // updated in place: A += pK, Bs += pK (x) v (inclusive prefix: the new token is
 // part of its own readout), then out_g = sum_s pQ_g[s] Bs[s,:] / (A[s] + eps)
 // for the G query heads of the group.
-template <class TX, int D, int GM>
-__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(GM <= 4 ? 8 : 1))) void race_decode_step(DecodeParams P)
+//
+// Large batches are bound by the state's bytes, small ones by the chain of dependent steps in one
+// workgroup. The chain has one memory latency: planes, inputs and the first state rows are all
+// loaded at once straight to the registers that use them (in that order, so that waiting for the
+// inputs does not wait for the state), a projection is shared by D / 8 lanes of one wave (8 products
+// each, then lane shuffles), and the probabilities are products of per-bit sigmoids, one per thread.
+// Four workgroups of 256 threads per CU within 128 VGPRs: fewer registers spill (6 waves per SIMD:
+// 39 us, 8: 51), and eight small workgroups per CU that all start with their inputs (the former
+// kernel) leave the memory idle meanwhile. 32 q / 8 kv heads, D = 64, S = 128, bf16 (us per step):
+// 8 sequences 10.4 -> 7 (kernel alone), 64: 14.7 -> 10.2, 128: 18.5 -> 14.6, 256: 26.6 -> 24.3
+// (5.7 TB/s), 600: 66.1 -> 62.9; 256 sequences at D = 128: 67.9 -> 58.0.
+template <class TX>
+struct DecRow8 {  // 8 consecutive elements of a row of any alignment
+    struct __attribute__((packed, aligned(sizeof(TX)))) Raw {
+        TX x[8];
+    } r;
+    RACE_DEV void load(const TX *p) { r = *reinterpret_cast<const Raw *>(p); }
+    RACE_DEV float operator[](int e) const { return (float)r.x[e]; }
+};
+
+template <class TX, int D, int GM, int NT>
+__global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(GM <= 4 ? 1024 / NT : 1)))
+void race_decode_step(DecodeParams P)
 {
-    // thread layout of the state update: TPR threads per bucket row (VEC floats each), RIF
-    // rows per pass over the state, PFR rows per thread loaded together; GM >= G query heads.
-    // Registers stay within 64 per lane and LDS within 20 KB, so eight workgroups fit a CU
-    // and a 256-CU device runs the 2048 (sequence, kv head) pairs of a decode batch in one round.
-    constexpr int VEC = 4, TPR = D / VEC, RIF = 256 / TPR, PFR = 4, NWV = 4;
+    // state update: TPR threads per bucket row (VEC floats each), RIF rows per pass over the state,
+    // PFR rows per thread loaded together; GM >= G query heads
+    constexpr int VEC = 4, TPR = D / VEC, RIF = NT / TPR, PFR = 4, NWV = NT / 64;
+    // projection: PARTS lanes share a column, CPW columns per wave and pass
+    constexpr int PARTS = D / 8, CPW = 64 / PARTS;
     extern __shared__ float sm[];
-    const int G = P.G, LK = P.L * P.K, R = 1 << P.K, S = P.L * R;
-    const bool pl_lds = D * LK <= DEC_PL_LDS;  // planes staged in LDS
-    float *sIn = sm;                  // [G + 2][D]: k, v, q_0 .. q_{G-1}
-    float *sU = sIn + (G + 2) * D;    // [G + 1][LK]: u for k, q_g
-    float *sP = sU + (G + 1) * LK;    // [G + 1][S]: pK, pQ_g
+    const int G = P.G, LK = P.L * P.K, K = P.K, S = P.L << K;
+    float *sS1 = sm;                  // [G + 1][LK] sigmoid(2u) of k, q_0 .. q_{G-1}
+    float *sS0 = sS1 + (G + 1) * LK;  // [G + 1][LK] sigmoid(-2u)
+    float *sP = sS0 + (G + 1) * LK;   // [G + 1][S]: pK, pQ_g
     float *sRed = sP + (G + 1) * S;   // [NWV][G][D]: readout partial sums per wave
-    float *sPl = sRed + NWV * G * D;  // [D][LK] planes (pl_lds)
     const int z = blockIdx.x;         // b * Hkv + hk
-    const int b = z / P.Hkv, hk = z % P.Hkv;
+    const int wv = threadIdx.x >> 6, lane = threadIdx.x & 63;
     const int rr = threadIdx.x / TPR, dv = (threadIdx.x % TPR) * VEC;
+    const int part = lane / CPW;
     float *A = P.A + (int64_t)z * S;
     float *Bs = P.Bs + (int64_t)z * S * D;
+    const TX *q = reinterpret_cast<const TX *>(P.q) + (int64_t)z * G * D;  // (b * Hkv + hk) * G + g
+    const TX *k = reinterpret_cast<const TX *>(P.k) + (int64_t)z * D;
+    const TX *v = reinterpret_cast<const TX *>(P.v) + (int64_t)z * D;
     f32x4 bpre[PFR];
-    float apre[PFR];
-    // first PFR rows of this thread: loads of clamped rows (always inside the state), all in
-    // flight together. Issued once no later global load has to be waited for before the update
-    // (the memory counter is in order): after the planes are in LDS, or after the projections.
-    auto prefetch_state = [&]() {
+    float apre[PFR], vv[VEC];
+    // loads of clamped rows (always inside the state), all in flight together
+    auto load_state = [&](int s0) {
 #pragma unroll
         for (int j = 0; j < PFR; ++j) {
-            const int sr = min(rr + j * RIF, S - 1);
+            const int sr = min(s0 + rr + j * RIF, S - 1);
             bpre[j] = *reinterpret_cast<const f32x4 *>(Bs + (int64_t)sr * D + dv);
             apre[j] = A[sr];
         }
     };
-    const TX *q = reinterpret_cast<const TX *>(P.q);
-    const TX *k = reinterpret_cast<const TX *>(P.k);
-    const TX *v = reinterpret_cast<const TX *>(P.v);
-    for (int i = threadIdx.x; i < (G + 2) * D; i += 256) {
-        const int row = i / D, d = i % D;
-        float x;
-        if (row == 0)
-            x = (float)k[((int64_t)b * P.Hkv + hk) * D + d];
-        else if (row == 1)
-            x = (float)v[((int64_t)b * P.Hkv + hk) * D + d];
-        else
-            x = (float)q[((int64_t)b * P.Hkv * G + hk * G + (row - 2)) * D + d];
-        sIn[row * D + d] = x;
-    }
-    if (pl_lds) {
-        for (int i = threadIdx.x; i < D * LK; i += 256) {
-            const float pl = P.planes[i];
-            sPl[i] = P.round_planes ? (float)(__bf16)pl : pl;
+    auto load_value = [&]() {
+#pragma unroll
+        for (int e = 0; e < VEC; ++e)
+            vv[e] = (float)v[dv + e];
+    };
+    // one pass over NWV x CPW columns (the first one also issues the state loads)
+    auto project = [&](int j0, auto first) {
+        const int j = j0 + lane % CPW, jc = min(j, LK - 1);
+        float pl[8], acc[GM + 1];
+        DecRow8<TX> x[GM + 1];
+#pragma unroll
+        for (int e = 0; e < 8; ++e)
+            pl[e] = P.planes[(part * 8 + e) * LK + jc];
+        x[0].load(k + part * 8);
+#pragma unroll
+        for (int g = 0; g < GM; ++g)
+            x[1 + g].load(q + min(g, G - 1) * D + part * 8);
+        if constexpr (first) {
+            load_value();
+            load_state(0);
         }
-    }
-    __syncthreads();
-    if (pl_lds)
-        prefetch_state();
-    // projections: row 0 = k, rows 1.. = q_g
-    for (int i = threadIdx.x; i < (G + 1) * LK; i += 256) {
-        const int row = i / LK, j = i % LK;
-        const float *x = sIn + (row == 0 ? 0 : row + 1) * D;
-        float acc = 0.0f;
-        if (pl_lds) {
-            for (int d = 0; d < D; ++d)
-                acc += x[d] * sPl[d * LK + j];
-        } else {
-#pragma unroll 8
-            for (int d = 0; d < D; ++d) {
-                const float pl = P.planes[d * LK + j];
-                acc += x[d] * (P.round_planes ? (float)(__bf16)pl : pl);
+#pragma unroll
+        for (int e = 0; e < 8; ++e)
+            pl[e] = P.round_planes ? (float)(__bf16)pl[e] : pl[e];
+#pragma unroll
+        for (int r = 0; r < GM + 1; ++r) {
+            acc[r] = 0.0f;
+#pragma unroll
+            for (int e = 0; e < 8; ++e)
+                acc[r] += x[r][e] * pl[e];
+        }
+#pragma unroll
+        for (int r = 0; r < GM + 1; ++r)
+#pragma unroll
+            for (int m = CPW; m < 64; m <<= 1)
+                acc[r] += __shfl_xor(acc[r], m, 64);
+        // lane group `part` finishes the rows part, part + PARTS of this column
+#pragma unroll
+        for (int r0 = 0; r0 < GM + 1; r0 += PARTS) {
+            float a = acc[r0];
+#pragma unroll
+            for (int r = r0 + 1; r < min(r0 + PARTS, GM + 1); ++r)
+                a = part == r - r0 ? acc[r] : a;
+            const int row = r0 + part;
+            if (row <= G && j < LK) {
+                const float e = __expf(-2.0f * sig_arg(tanh_f(a) * P.inv_scale));
+                const float s1 = frcp(1.0f + e);
+                sS1[row * LK + j] = s1;
+                sS0[row * LK + j] = e * s1;
             }
         }
-        sU[row * LK + j] = tanh_f(acc) * P.inv_scale;
-    }
-    if (!pl_lds)
-        prefetch_state();
+    };
+    project(wv * CPW, std::true_type());
+    for (int j0 = (wv + NWV) * CPW; j0 < LK; j0 += NWV * CPW)
+        project(j0, std::false_type());
     __syncthreads();
-    for (int i = threadIdx.x; i < (G + 1) * P.L; i += 256) {
-        const int row = i / P.L, l = i % P.L;
-        float u[4], p[16];
-        for (int kk = 0; kk < 4; ++kk)
-            u[kk] = (kk < P.K) ? sU[row * LK + l * P.K + kk] : 0.0f;
-        expand_probs(u, P.K, p);
-        for (int r = 0; r < 16; ++r)
-            if (r < R)
-                sP[row * S + l * R + r] = p[r];
+    for (int i = threadIdx.x; i < (G + 1) * S; i += NT) {
+        const int row = i / S, s = i % S;
+        const int c0 = row * LK + (s >> K) * K;
+        float p = 1.0f;
+        for (int b = 0; b < K; ++b)  // bit 0 is the most significant one
+            p *= (s >> (K - 1 - b)) & 1 ? sS1[c0 + b] : sS0[c0 + b];
+        sP[i] = p;
     }
     __syncthreads();
     // state update + readout, PFR rows per thread at a time
     float acc[GM][VEC];
+#pragma unroll
     for (int g = 0; g < GM; ++g)
+#pragma unroll
         for (int e = 0; e < VEC; ++e)
             acc[g][e] = 0.0f;
-    float vv[VEC];
-    for (int e = 0; e < VEC; ++e)
-        vv[e] = sIn[D + dv + e];
     for (int s0 = 0; s0 < S; s0 += PFR * RIF) {
-        if (s0 > 0) {
-#pragma unroll
-            for (int j = 0; j < PFR; ++j) {
-                const int sr = min(s0 + rr + j * RIF, S - 1);
-                bpre[j] = *reinterpret_cast<const f32x4 *>(Bs + (int64_t)sr * D + dv);
-                apre[j] = A[sr];
-            }
-        }
+        if (s0 > 0)
+            load_state(s0);
 #pragma unroll
         for (int j = 0; j < PFR; ++j) {
             const int s = s0 + rr + j * RIF;
@@ -1285,15 +1312,18 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(GM <= 4 ? 8
                 const float pk = sP[s];
                 const float a = apre[j] + pk;
                 f32x4 bv = bpre[j];
+#pragma unroll
                 for (int e = 0; e < VEC; ++e)
                     bv[e] += pk * vv[e];
                 *reinterpret_cast<f32x4 *>(Bs + (int64_t)s * D + dv) = bv;
                 if (dv == 0)
                     A[s] = a;
                 const float inv = frcp(a + P.eps);
+#pragma unroll
                 for (int g = 0; g < GM; ++g)
                     if (g < G) {
                         const float w = sP[(1 + g) * S + s] * inv;
+#pragma unroll
                         for (int e = 0; e < VEC; ++e)
                             acc[g][e] += w * bv[e];
                     }
@@ -1302,51 +1332,59 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(GM <= 4 ? 8
     }
     // the rows of one wave share the lanes' head-dim columns: lanes l, l + TPR, ... add up by
     // shuffles, then one partial sum per wave goes through LDS
-    const int wv = threadIdx.x >> 6;
+#pragma unroll
     for (int g = 0; g < GM; ++g)
         if (g < G)
+#pragma unroll
             for (int e = 0; e < VEC; ++e) {
                 float x = acc[g][e];
 #pragma unroll
                 for (int m = TPR; m < 64; m <<= 1)
                     x += __shfl_xor(x, m, 64);
-                if ((threadIdx.x & 63) < TPR)
+                if (lane < TPR)
                     sRed[(wv * G + g) * D + dv + e] = x;
             }
     __syncthreads();
-    TX *out = reinterpret_cast<TX *>(P.out);
-    for (int i = threadIdx.x; i < G * D; i += 256) {
-        const int g = i / D, d = i % D;
+    TX *out = reinterpret_cast<TX *>(P.out) + (int64_t)z * G * D;
+    for (int i = threadIdx.x; i < G * D; i += NT) {
         float sum = 0.0f;
+#pragma unroll
         for (int r = 0; r < NWV; ++r)
-            sum += sRed[(r * G + g) * D + d];
-        out[((int64_t)b * P.Hkv * G + hk * G + g) * D + d] = (TX)sum;
+            sum += sRed[r * G * D + i];
+        out[i] = (TX)sum;
     }
 }
 
-// dynamic LDS of one decode workgroup (floats): inputs, soft bits, probabilities, partial sums
-static size_t decode_smem(const DecodeParams &P)
+// dynamic LDS of one decode workgroup (floats): sigmoids, probabilities, partial sums
+static size_t decode_smem(const DecodeParams &P, int NT)
 {
-    const int LK = P.L * P.K, S = P.L << P.K, NWV = 4;
-    const size_t pl = P.D * LK <= DEC_PL_LDS ? (size_t)P.D * LK : 0;
-    return sizeof(float) * ((size_t)(P.G + 2) * P.D + (size_t)(P.G + 1) * LK + (size_t)(P.G + 1) * S +
-                            (size_t)NWV * P.G * P.D + pl);
+    const int LK = P.L * P.K, S = P.L << P.K;
+    return sizeof(float) * ((size_t)(P.G + 1) * (2 * LK + S) + (size_t)(NT / 64) * P.G * P.D);
 }
 
 hipError_t launch_decode(const DecodeParams &P, int bf16, hipStream_t s)
 {
-    const dim3 grid((unsigned)(P.B * P.Hkv));
-    const size_t smem = decode_smem(P);
-    if (smem > 64 * 1024)
-        return hipErrorInvalidValue;
     if (P.G < 1 || P.G > DEC_GMAX)
         return hipErrorInvalidValue;
-#define DEC(TX, DD, GM) hipLaunchKernelGGL((race_decode_step<TX, DD, GM>), grid, dim3(256), smem, s, P)
-#define DEC_G(TX, DD)                 \
-    if (P.G == 1) DEC(TX, DD, 1);     \
-    else if (P.G == 2) DEC(TX, DD, 2); \
-    else if (P.G <= 4) DEC(TX, DD, 4); \
-    else DEC(TX, DD, 8)
+    const int z = P.B * P.Hkv;
+    const dim3 grid((unsigned)z);
+    // up to two workgroups per CU: 512 threads have a whole 128-bucket state in flight (8 sequences
+    // x 8 kv heads 8.0 -> 6.6 us); beyond, 256 threads (1024 pairs: 14.6 against 17.9 us)
+    const bool wide = z <= DEC_WIDE && decode_smem(P, 512) <= 64 * 1024;
+    const int NT = wide ? 512 : 256;
+    const size_t smem = decode_smem(P, NT);
+    if (smem > 64 * 1024)
+        return hipErrorInvalidValue;
+#define DEC(TX, DD, GM)                                                                                  \
+    if (wide)                                                                                            \
+        hipLaunchKernelGGL((race_decode_step<TX, DD, GM, 512>), grid, dim3(512), smem, s, P);            \
+    else                                                                                                 \
+        hipLaunchKernelGGL((race_decode_step<TX, DD, GM, 256>), grid, dim3(256), smem, s, P)
+#define DEC_G(TX, DD)                    \
+    if (P.G == 1) { DEC(TX, DD, 1); }    \
+    else if (P.G == 2) { DEC(TX, DD, 2); } \
+    else if (P.G <= 4) { DEC(TX, DD, 4); } \
+    else { DEC(TX, DD, 8); }
     if (P.D == 64) {
         if (bf16) { DEC_G(__bf16, 64); } else { DEC_G(float, 64); }
     } else if (P.D == 128) {
