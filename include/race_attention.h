@@ -215,6 +215,13 @@ size_t race_qkv_scratch_bytes(const race_qkv_shape *sh, int backward);
 int race_qkv_fwd(const race_qkv_shape *sh, race_tensor q, race_tensor k, race_tensor v,
                  const float *planes_T, race_tensor out, int out_dtype, void *state,
                  size_t state_bytes, void *scratch, size_t scratch_bytes, race_stream stream);
+/* race_qkv_fwd that leaves the final bucket state in A [B*Hkv][S], Bs [B*Hkv][S][D] (fp32, Bs
+ * 16-byte aligned), as race_qkv_fwd followed by race_qkv_final_state, for prompts: `workspace`
+ * (race_qkv_state_bytes bytes) holds nothing afterwards that a backward could use. */
+int race_qkv_prefill(const race_qkv_shape *sh, race_tensor q, race_tensor k, race_tensor v,
+                     const float *planes_T, race_tensor out, int out_dtype, float *A, float *Bs,
+                     void *workspace, size_t workspace_bytes, void *scratch, size_t scratch_bytes,
+                     race_stream stream);
 /* go bf16; dq, dk, dv bf16 (overwritten, not accumulated). */
 int race_qkv_bwd(const race_qkv_shape *sh, race_tensor q, race_tensor k, race_tensor v,
                  race_tensor go, const float *planes_T, const void *state, size_t state_bytes,

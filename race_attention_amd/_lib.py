@@ -91,6 +91,8 @@ SIGNATURES = {
     "race_qkv_scratch_bytes": (ctypes.c_size_t, [ctypes.POINTER(QKVShape), ctypes.c_int]),
     "race_qkv_fwd": (ctypes.c_int, [ctypes.POINTER(QKVShape), Tensor4, Tensor4, Tensor4, _vp, Tensor4,
                                     ctypes.c_int, _vp, ctypes.c_size_t, _vp, ctypes.c_size_t, _vp]),
+    "race_qkv_prefill": (ctypes.c_int, [ctypes.POINTER(QKVShape), Tensor4, Tensor4, Tensor4, _vp, Tensor4,
+                                        ctypes.c_int, _vp, _vp, _vp, ctypes.c_size_t, _vp, ctypes.c_size_t, _vp]),
     "race_qkv_bwd": (ctypes.c_int, [ctypes.POINTER(QKVShape), Tensor4, Tensor4, Tensor4, Tensor4, _vp, _vp,
                                     ctypes.c_size_t, Tensor4, Tensor4, Tensor4, _vp, ctypes.c_size_t, _vp]),
     "race_qkv_final_state": (ctypes.c_int, [ctypes.POINTER(QKVShape), _vp, ctypes.c_size_t, _vp, _vp, _vp]),

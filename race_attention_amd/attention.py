@@ -98,10 +98,12 @@ def race_causal_attention(q, k, v, planes_T, L, Kbits, scale=None, eps=1e-6, out
     return RaceAttentionFn.apply(q, k, v, planes_T, L, Kbits, scale, eps, out_dtype, block)
 
 
-def race_causal_attention_with_state(q, k, v, planes_T, L, Kbits, scale=None, eps=1e-6, out_dtype=None):
+def race_causal_attention_with_state(q, k, v, planes_T, L, Kbits, scale=None, eps=1e-6, out_dtype=None,
+                                     state_out=None):
     """Forward only (no autograd): (out, A [B*Hkv,S], Bs [B*Hkv,S,D]) -- the output and
     the final bucket state (race_prefix_ref's A_final / B_final, race_common.py:88-90),
-    which seeds race_attention_amd.decode.RaceDecodeState."""
+    which seeds race_attention_amd.decode.RaceDecodeState. `state_out` gives the (A, Bs)
+    to write (contiguous fp32); new tensors otherwise."""
     _lib.require_device(q, k, v, planes_T)
     if scale is None:
         scale = math.sqrt(q.shape[-1])
@@ -109,21 +111,27 @@ def race_causal_attention_with_state(q, k, v, planes_T, L, Kbits, scale=None, ep
         raise _lib.RaceError("fused RACE needs bf16 q/k/v with head dim 64 or 128 and K <= 4")
     q, k, v = _bf16_rows(q), _bf16_rows(k), _bf16_rows(v)
     B, Hq, T, D = q.shape
-    Hkv = k.shape[1]
+    Hkv, S = k.shape[1], L << Kbits
+    if k.shape != (B, Hkv, T, D) or v.shape != k.shape or Hq % Hkv:
+        raise ValueError(f"q {tuple(q.shape)} / k {tuple(k.shape)} / v {tuple(v.shape)} mismatch")
     planes = planes_T.detach().float().contiguous()
     out_dtype = out_dtype or q.dtype
     sh = qkv_shape(q, k, L, Kbits, scale, eps, 0)
     lib = _lib.lib()
-    state = _lib.workspace(lib.race_qkv_state_bytes(sh), q.device)
+    work = _lib.workspace(lib.race_qkv_state_bytes(sh), q.device)
     scratch = _lib.workspace(lib.race_qkv_scratch_bytes(sh, 0), q.device)
     out = torch.empty(B, Hq, T, D, dtype=out_dtype, device=q.device)
+    if state_out is None:
+        A = torch.empty(B * Hkv, S, dtype=torch.float32, device=q.device)
+        Bs = torch.empty(B * Hkv, S, D, dtype=torch.float32, device=q.device)
+    else:
+        A, Bs = state_out
+        if (A.shape != (B * Hkv, S) or Bs.shape != (B * Hkv, S, D) or not (A.is_contiguous() and Bs.is_contiguous())
+                or A.dtype != torch.float32 or Bs.dtype != torch.float32 or A.device != q.device
+                or Bs.device != q.device):
+            raise ValueError(f"state_out must be contiguous fp32 [{B * Hkv},{S}] and [{B * Hkv},{S},{D}] on {q.device}")
     qv, kv_, vv, ov = (_lib.view4(t)[0] for t in (q, k, v, out))
-    _lib.check(lib.race_qkv_fwd(sh, qv, kv_, vv, _lib.ptr(planes), ov, _lib.dtype_code(out_dtype),
-                                _lib.ptr(state), state.numel(), _lib.ptr(scratch), scratch.numel(),
-                                _lib.stream_of(q)), "race_qkv_fwd")
-    S = L << Kbits
-    A = torch.empty(B * Hkv, S, dtype=torch.float32, device=q.device)
-    Bs = torch.empty(B * Hkv, S, D, dtype=torch.float32, device=q.device)
-    _lib.check(lib.race_qkv_final_state(sh, _lib.ptr(state), state.numel(), _lib.ptr(A), _lib.ptr(Bs),
-                                        _lib.stream_of(q)), "race_qkv_final_state")
+    _lib.check(lib.race_qkv_prefill(sh, qv, kv_, vv, _lib.ptr(planes), ov, _lib.dtype_code(out_dtype), _lib.ptr(A),
+                                    _lib.ptr(Bs), _lib.ptr(work), work.numel(), _lib.ptr(scratch), scratch.numel(),
+                                    _lib.stream_of(q)), "race_qkv_prefill")
     return out, A, Bs

@@ -1002,22 +1002,29 @@ static int qkv_inputs(const race_qkv_shape *sh, const race_tensor &q, const race
     return RACE_OK;
 }
 
-int race_qkv_fwd(const race_qkv_shape *sh, race_tensor q, race_tensor k, race_tensor v, const float *planes_T,
-                 race_tensor out, int out_dtype, void *state, size_t state_bytes, void *scratch_buf,
-                 size_t scratch_bytes, race_stream stream)
+// A sequence of one block on the fused kernels: the readout starts from the zero state and leaves
+// the final one itself, without the totals pass, the block scan and the copies of the final state
+// (a prompt of 512 tokens for 256 sequences, 32 / 8 heads of 64, S = 128: 826 -> 477 us, of which 91
+// were the totals, 127 the scan and 105 the state's extraction, copies and fills).
+static bool qkv_single(const race_qkv_shape *sh, const Geo &g) { return g.NB == 1 && !qkv_generic(sh, g); }
+
+// The forward; with A and Bs (both or none) also the final state, dense.
+static int qkv_fwd_impl(const race_qkv_shape *sh, race_tensor q, race_tensor k, race_tensor v, const float *planes_T,
+                        race_tensor out, int out_dtype, void *state, size_t state_bytes, void *scratch_buf,
+                        size_t scratch_bytes, float *A, float *Bs, race_stream stream, const char *who)
 {
     Geo g;
     RACE_TRY(qkv_geometry(sh, g));
-    RACE_TRY(qkv_inputs(sh, q, k, v, planes_T, "race_qkv_fwd"));
+    RACE_TRY(qkv_inputs(sh, q, k, v, planes_T, who));
     if (out_dtype != RACE_F32 && out_dtype != RACE_BF16)
-        return fail(RACE_ERR_INVALID, "race_qkv_fwd: out_dtype must be RACE_F32 or RACE_BF16");
-    RACE_TRY(check_view(out, "race_qkv_fwd: out", false));
+        return fail(RACE_ERR_INVALID, "%s: out_dtype must be RACE_F32 or RACE_BF16", who);
+    RACE_TRY(check_view(out, who, false));
     const size_t need_state = race_qkv_state_bytes(sh), need_scr = qkv_scratch(sh, g, 0);
     if (!state || state_bytes < need_state)
-        return fail(RACE_ERR_WORKSPACE, "race_qkv_fwd: state of %zu bytes needed, got %zu", need_state,
+        return fail(RACE_ERR_WORKSPACE, "%s: state of %zu bytes needed, got %zu", who, need_state,
                     state ? state_bytes : 0);
     if (need_scr && (!scratch_buf || scratch_bytes < need_scr))
-        return fail(RACE_ERR_WORKSPACE, "race_qkv_fwd: scratch of %zu bytes needed, got %zu", need_scr,
+        return fail(RACE_ERR_WORKSPACE, "%s: scratch of %zu bytes needed, got %zu", who, need_scr,
                     scratch_buf ? scratch_bytes : 0);
     ScanParams P = qkv_params(sh, g);
     P.q = to_view(q);
@@ -1038,21 +1045,59 @@ int race_qkv_fwd(const race_qkv_shape *sh, race_tensor q, race_tensor k, race_te
         P.out = to_out(out, out_dtype == RACE_F32);
     }
     const hipStream_t s = hs(stream);
-    RACE_TRY(run_scan_qkv(K_FWD_TOTALS, g, P, s));
-    RACE_TRY(hip_check(prof_block_scan(P.wsB, (int64_t)g.S_pad * g.DP, P.wsA, g.S_pad, (int)g.NB, (int)g.Z, 0, s), "block scan"));
+    P.single = qkv_single(sh, g);
+    if (P.single && A) {  // straight to the caller's state; the workspace is not needed
+        P.finB = Bs;
+        P.finA = A;
+        P.finS = P.S;
+        P.finBz = (int64_t)P.S * D;
+        P.finAz = P.S;
+        P.wsB = P.wsA = nullptr;
+    } else if (P.single) {  // slot 1 of the workspace, zeros in slot 0
+        P.finS = g.S_pad;
+        P.finBz = 2 * (int64_t)g.S_pad * g.DP;
+        P.finAz = 2 * g.S_pad;
+        P.finB = P.wsB + P.finBz / 2;
+        P.finA = P.wsA + P.finAz / 2;
+    } else {
+        RACE_TRY(run_scan_qkv(K_FWD_TOTALS, g, P, s));
+        RACE_TRY(hip_check(prof_block_scan(P.wsB, (int64_t)g.S_pad * g.DP, P.wsA, g.S_pad, (int)g.NB, (int)g.Z, 0, s),
+                           "block scan"));
+    }
     if (g.seq) {
         for (int j = 0; j < g.n_st; ++j) {
             P.st_base = j;
             P.out = tile_out(j, g.n_st, part, to_out(out, out_dtype == RACE_F32), sh->Hq, T, D);
             RACE_TRY(run_scan_qkv(K_FWD_READOUT, g, P, s));
         }
-        return RACE_OK;
+    } else {
+        RACE_TRY(run_scan_qkv(K_FWD_READOUT, g, P, s));
+        if (part)
+            RACE_TRY(hip_check(prof_reduce(part, g.n_st, q_elems, to_out(out, out_dtype == RACE_F32), sh->B, sh->Hq,
+                                           sh->T, sh->D, s), "reduce partials"));
     }
-    RACE_TRY(run_scan_qkv(K_FWD_READOUT, g, P, s));
-    if (part)
-        RACE_TRY(hip_check(prof_reduce(part, g.n_st, q_elems, to_out(out, out_dtype == RACE_F32), sh->B,
-                                                  sh->Hq, sh->T, sh->D, s), "reduce partials"));
+    if (A && !P.single)
+        return hip_check(launch_state_extract(P.wsB, P.wsA, (int)g.NB, g.S_pad, g.DP, (int)g.Z, P.S, sh->D, A, Bs, s),
+                         "final state");
     return RACE_OK;
+}
+
+int race_qkv_fwd(const race_qkv_shape *sh, race_tensor q, race_tensor k, race_tensor v, const float *planes_T,
+                 race_tensor out, int out_dtype, void *state, size_t state_bytes, void *scratch_buf,
+                 size_t scratch_bytes, race_stream stream)
+{
+    return qkv_fwd_impl(sh, q, k, v, planes_T, out, out_dtype, state, state_bytes, scratch_buf, scratch_bytes, nullptr,
+                        nullptr, stream, "race_qkv_fwd");
+}
+
+int race_qkv_prefill(const race_qkv_shape *sh, race_tensor q, race_tensor k, race_tensor v, const float *planes_T,
+                     race_tensor out, int out_dtype, float *A, float *Bs, void *workspace, size_t workspace_bytes,
+                     void *scratch_buf, size_t scratch_bytes, race_stream stream)
+{
+    if (!A || !Bs)
+        return fail(RACE_ERR_INVALID, "race_qkv_prefill: null state output");
+    return qkv_fwd_impl(sh, q, k, v, planes_T, out, out_dtype, workspace, workspace_bytes, scratch_buf, scratch_bytes,
+                        A, Bs, stream, "race_qkv_prefill");
 }
 
 // Everything of race_qkv_bwd after its argument checks; `scr` holds qkv_scratch(sh, g, 1) bytes.
@@ -1126,9 +1171,10 @@ static int qkv_bwd_run(const race_qkv_shape *sh, const Geo &g, race_tensor q, ra
             RACE_TRY(run_scan_qkv(K_BWD_TOTALS, g, P, s));
         }
         P.st_base = 0;
-        RACE_TRY(hip_check(prof_block_scan(P.ws2B, (int64_t)g.S_pad * g.DP, P.ws2A, g.S_pad, (int)g.NB, (int)g.Z, 1,
-                                           s),
-                           "block scan"));
+        if (!qkv_single(sh, g))  // (one block: its total is its suffix)
+            RACE_TRY(hip_check(prof_block_scan(P.ws2B, (int64_t)g.S_pad * g.DP, P.ws2A, g.S_pad, (int)g.NB, (int)g.Z, 1,
+                                               s),
+                               "block scan"));
         for (int j = 0; j < g.n_st; ++j) {
             P.st_base = j;
             P.dk = tile_out(j, g.n_st, pk, to_out(dk, 0), sh->Hkv, T, D);
@@ -1151,9 +1197,10 @@ static int qkv_bwd_run(const race_qkv_shape *sh, const Geo &g, race_tensor q, ra
     }
     const hipStream_t s = hs(stream);
     RACE_TRY(run_scan_qkv(K_BWD_TOTALS, g, P, s));
-    RACE_TRY(hip_check(prof_block_scan(P.ws2B, (int64_t)g.S_pad * g.DP, P.ws2A, g.S_pad, (int)g.NB, (int)g.Z, 1, s,
-                                       generic ? P.ws3B : nullptr, generic ? P.ws3A : nullptr),
-                       "block scan"));
+    if (!qkv_single(sh, g))
+        RACE_TRY(hip_check(prof_block_scan(P.ws2B, (int64_t)g.S_pad * g.DP, P.ws2A, g.S_pad, (int)g.NB, (int)g.Z, 1, s,
+                                           generic ? P.ws3B : nullptr, generic ? P.ws3A : nullptr),
+                           "block scan"));
     RACE_TRY(run_scan_qkv(K_BWD_MAIN, g, P, s));
     if (g.n_st > 1) {
         RACE_TRY(hip_check(prof_reduce(pq, g.n_st, q_elems, to_out(dq, 0), sh->B, sh->Hq, sh->T, sh->D, s),

@@ -1397,28 +1397,29 @@ hipError_t launch_decode(const DecodeParams &P, int bf16, hipStream_t s)
     return hipGetLastError();
 }
 
-// final state slot NB of a forward workspace -> dense decode state
-__global__ void race_state_extract(const float *wsB, const float *wsA, int NB, int S_pad, int DPw,
-                                   int S, int D, float *A, float *Bs, int64_t total)
+// final state slot NB of a forward workspace -> dense decode state, 16 bytes per thread (D % 4 == 0)
+__global__ __launch_bounds__(256) void race_state_extract(const float *wsB, const float *wsA, int NB, int S_pad,
+                                                          int DPw, int S, int D, float *A, float *Bs, int64_t total)
 {
-    const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+    const int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x;
     if (i >= total)
         return;
-    const int d = (int)(i % (D + 1));
-    const int64_t r = i / (D + 1);
+    const int d = (int)(i % (D / 4)) * 4;
+    const int64_t r = i / (D / 4);  // z * S + s
     const int s = (int)(r % S);
-    const int64_t z = r / S;
-    const int64_t slot = z * (NB + 1) + NB;
-    if (d == D)
-        A[z * S + s] = wsA[slot * S_pad + s];
-    else
-        Bs[(z * S + s) * D + d] = wsB[(slot * S_pad + s) * DPw + d];
+    const int64_t row = (r / S * (NB + 1) + NB) * S_pad + s;
+    struct __attribute__((packed, aligned(4))) Run {  // (Bs of any alignment)
+        f32x4 x;
+    };
+    reinterpret_cast<Run *>(Bs + r * D + d)->x = *reinterpret_cast<const f32x4 *>(wsB + row * DPw + d);
+    if (d == 0)
+        A[r] = wsA[row];
 }
 
 hipError_t launch_state_extract(const float *wsB, const float *wsA, int NB, int S_pad, int DPw,
                                 int Z, int S, int D, float *A, float *Bs, hipStream_t s)
 {
-    const int64_t total = (int64_t)Z * S * (D + 1);
+    const int64_t total = (int64_t)Z * S * (D / 4);
     hipLaunchKernelGGL(race_state_extract, dim3((unsigned)((total + 255) / 256)), dim3(256), 0, s,
                        wsB, wsA, NB, S_pad, DPw, S, D, A, Bs, total);
     return hipGetLastError();

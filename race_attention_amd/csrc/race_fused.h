@@ -630,12 +630,12 @@ struct MoverRows {
         ra = *reinterpret_cast<gu32x4 *>(pa + t_off * sa + (uint64_t)oa);
         rb = *reinterpret_cast<gu32x4 *>(pb + t_off * sb + (uint64_t)ob);
     }
-    // the first tensor's chunk only
-    RACE_DEV void load_a(u32x4 &ra, int t_off, int nv) const
+    // the first tensor's chunk only, `shift` bytes on (another head)
+    RACE_DEV void load_a(u32x4 &ra, int t_off, int nv, int64_t shift = 0) const
     {
         const unsigned rr = (unsigned)min(row, nv - 1);
         const unsigned oa = (__umul24(rr, (unsigned)(sa >> 1)) + col) * 2u;
-        ra = *reinterpret_cast<gu32x4 *>(pa + t_off * sa + (uint64_t)oa);
+        ra = *reinterpret_cast<gu32x4 *>(pa + (t_off * sa + shift) + (uint64_t)oa);
     }
 };
 
@@ -695,7 +695,7 @@ void race_fused_fwd_readout(const ScanParams P)
         for (int i = 0; i < TPW_S; ++i) {
             const int t = wave + i * NW;
             accS[i] = f32x4{0.f, 0.f, 0.f, 0.f};
-            if (t < CF::NTS * CF::NTD) {
+            if (t < CF::NTS * CF::NTD && !P.single) {  // (uniform)
                 const int m0 = (t / CF::NTD) * 16, n0 = (t % CF::NTD) * 16;
                 const int r = acc_row(m0, lane), col = acc_col(n0, lane);
 #pragma unroll
@@ -705,7 +705,7 @@ void race_fused_fwd_readout(const ScanParams P)
         }
         const float *wA = P.wsA + slot * P.S_pad + c.s0;
         for (int s = tid; s < ST; s += NTH)
-            sA0[0][s] = wA[s] + P.eps;  // the carry holds A + eps
+            sA0[0][s] = P.single ? P.eps : wA[s] + P.eps;  // the carry holds A + eps
     }
 
     const int G = G1 ? 1 : P.G;  // G1: one query head per kv head, the head loop folds away
@@ -732,6 +732,7 @@ void race_fused_fwd_readout(const ScanParams P)
     wait_vmem_all();
     __syncthreads();
 
+    const int t_last = c.t_begin + (nsub - 1) * C;  // start of the last sub-chunk
     f32x4 accA[TPW_A];  // 1/(A+eps), transposed tiles, kept across query heads
     int prev_t0 = -1, prev_nv = 0, prev_h = 0;
     AccRows<C, DP, NTH> arO;
@@ -744,22 +745,26 @@ void race_fused_fwd_readout(const ScanParams P)
             const int t1 = t0 + C, nv1 = min(C, c.t_end - t1);
             if constexpr (SB) {
                 mvKV.load(pk[0], pv[0], t1 - c.t_begin, nv1);
-                if (G == 1)
+                if (G1)
                     mvQ.load_a(pq[0], t1 - c.t_begin, nv1);
             } else {
                 tile_load<CF>(pk, row_ptr(P.k, c.b, c.hk, t1), P.k.st, nv1, tid);
                 tile_load<CF>(pv, row_ptr(P.v, c.b, c.hk, t1), P.v.st, nv1, tid);
-                if (G == 1)
+                if (G1)
                     tile_load<CF>(pq, row_ptr(P.q, c.b, c.hk, t1), P.q.st, nv1, tid);
             }
         }
         for (int g = 0; g < G; ++g) {
             const int hq = c.hk * G + g;
-            if (g > 0) {  // further query heads of the group: load q synchronously
-                u32x4 tq[CF::PF];
-                tile_load<CF>(tq, row_ptr(P.q, c.b, hq, t0), P.q.st, nv, tid);
-                tile_store_kq<CF>(&sQ[0][0], tq, tid);
-                __syncthreads();
+            // (grouped heads) q of the next step, this sub-chunk's next head or the next one's first,
+            // in flight during this one (loaded when it began instead: 284 -> 265 us for 8 x 8192
+            // tokens, 32 / 8 heads of 64, S = 128)
+            if constexpr (!G1) {
+                const int g2 = g + 1 < G ? g + 1 : 0, t2 = g2 ? t0 : min(t0 + C, t_last), nv2 = min(C, c.t_end - t2);
+                if constexpr (SB)
+                    mvQ.load_a(pq[0], t2 - c.t_begin, nv2, (int64_t)g2 * P.q.sh * 2);
+                else
+                    tile_load<CF>(pq, row_ptr(P.q, c.b, c.hk * G + g2, t2), P.q.st, nv2, tid);
             }
             // ---- P1: soft-hash of k (first head only) and q; previous output rows to HBM
 #pragma unroll
@@ -889,20 +894,40 @@ void race_fused_fwd_readout(const ScanParams P)
                     const int nv1 = min(C, c.t_end - t0 - C);
                     tile_store_kq<CF>(&sK[0][0], pk, tid);
                     tile_store_rows<CF>(&sV[nxt][0][0], pv, nv1, tid);
-                    if (G == 1)
+                    if (G1)
                         tile_store_kq<CF>(&sQ[0][0], pq, tid);
-                    else {
-                        u32x4 tq[CF::PF];
-                        tile_load<CF>(tq, row_ptr(P.q, c.b, c.hk * G, t0 + C), P.q.st, nv1, tid);
-                        tile_store_kq<CF>(&sQ[0][0], tq, tid);
-                    }
                 }
             }
+            if (!G1)
+                tile_store_kq<CF>(&sQ[0][0], pq, tid);
             __syncthreads();
         }
     }
     // last output rows
     store_out<OT, C, DP, LDO, NTH>(P.out, c.b, prev_h, c.st, prev_t0, prev_nv, sO, arO, tid);
+    if (P.single) {  // (uniform) the one block's end is the sequence's
+        float *fB = P.finB + c.z * P.finBz, *fA = P.finA + c.z * P.finAz;
+#pragma unroll
+        for (int i = 0; i < TPW_S; ++i) {
+            const int t = wave + i * NW;
+            if (t < CF::NTS * CF::NTD) {
+                const int r = c.s0 + acc_row((t / CF::NTD) * 16, lane), col = acc_col((t % CF::NTD) * 16, lane);
+#pragma unroll
+                for (int e = 0; e < 4; ++e) {
+                    if (r + e < P.finS)
+                        fB[(int64_t)(r + e) * P.DPw + col] = accS[i][e];
+                    if (P.wsB)
+                        P.wsB[(slot * P.S_pad + r + e) * P.DPw + col] = 0.0f;
+                }
+            }
+        }
+        for (int s = tid; s < ST; s += NTH) {
+            if (c.s0 + s < P.finS)
+                fA[c.s0 + s] = sA0[nsub & 1][s] - P.eps;
+            if (P.wsA)
+                P.wsA[slot * P.S_pad + c.s0 + s] = 0.0f;
+        }
+    }
 }
 
 

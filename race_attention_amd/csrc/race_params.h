@@ -57,6 +57,12 @@ struct ScanParams {
     float *ckA;
     int NCK;
     int vec;  // op path: every row of the operands starts 16-byte aligned
+    // fused readout of a sequence that is one block: no totals pass and no block scan have run. The
+    // state starts at zero, and its final value goes to finB / finA (rows s < finS of stream z at
+    // z * finBz / z * finAz; DPw floats per row); with wsB, zeros go to block 0's prefix there.
+    int single, finS;
+    float *finB, *finA;
+    int64_t finBz, finAz;
     // op path only: 1 = unnormalised causal linear attention, W = pQ (no 1/(A+eps), gA = 0)
     int linear;
 };

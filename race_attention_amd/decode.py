@@ -46,10 +46,10 @@ class RaceDecodeState:
         The state must be fresh (prefill starts from zero)."""
         if self.tokens:
             raise RuntimeError("prefill on a non-empty state; call reset() first")
-        out, A, Bs = race_causal_attention_with_state(q, k, v, self.planes, self.L, self.K, self.scale,
-                                                      self.eps, out_dtype)
-        self.A.copy_(A)
-        self.Bs.copy_(Bs)
+        if k.shape[:2] != (self.B, self.Hkv) or k.shape[3] != self.D:
+            raise ValueError(f"prefill expects k/v [{self.B},{self.Hkv},T,{self.D}], got {tuple(k.shape)}")
+        out, _, _ = race_causal_attention_with_state(q, k, v, self.planes, self.L, self.K, self.scale, self.eps,
+                                                     out_dtype, (self.A, self.Bs))
         self.tokens = q.shape[2]
         return out
 
