@@ -40,7 +40,9 @@ typedef enum {
     RACE_ERR_HIP = 4          /* HIP runtime error while launching */
 } race_status;
 
-typedef enum { RACE_F32 = 0, RACE_BF16 = 1 } race_dtype;
+/* RACE_BF16_AS_F32 (soft-hash only): bf16 elements taken as the fp32 values they are, so that the
+ * planes are not rounded to bf16 */
+typedef enum { RACE_F32 = 0, RACE_BF16 = 1, RACE_BF16_AS_F32 = 2 } race_dtype;
 
 typedef void *race_stream; /* hipStream_t */
 

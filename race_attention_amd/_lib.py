@@ -15,6 +15,7 @@ LIB_PATH = os.path.join(_HERE, "librace_amd.so")
 
 RACE_F32 = 0
 RACE_BF16 = 1
+RACE_BF16_AS_F32 = 2  # soft-hash: bf16 elements, planes not rounded
 
 _i64 = ctypes.c_int64
 _vp = ctypes.c_void_p

@@ -32,16 +32,26 @@ def _bf16_rows(t):
     return t
 
 
+def _out_rows(B, H, T, D, dtype, device, bthd):
+    """A new [B,H,T,D] tensor, contiguous or (bthd) a view of contiguous [B,T,H,D] memory."""
+    if bthd:
+        return torch.empty(B, T, H, D, dtype=dtype, device=device).transpose(1, 2)
+    return torch.empty(B, H, T, D, dtype=dtype, device=device)
+
+
 def qkv_shape(q, k, L, Kbits, scale, eps, block=0):
     B, Hq, T, D = q.shape
     return _lib.QKVShape(B, Hq, k.shape[1], T, D, L, Kbits, float(scale), float(eps), int(block))
 
 
 class RaceAttentionFn(Function):
-    """out = causal RACE(q, k, v); q [B,Hq,T,D], k/v [B,Hkv,T,D] bf16, planes_T [D, L*K]."""
+    """out = causal RACE(q, k, v); q [B,Hq,T,D], k/v [B,Hkv,T,D] bf16, planes_T [D, L*K].
+
+    The gradients take the memory order of q, k and v, so that autograd hands them on without a
+    layout copy; the output is contiguous, or with `bthd` a [B,Hq,T,D] view of [B,T,Hq,D] memory."""
 
     @staticmethod
-    def forward(ctx, q, k, v, planes_T, L, Kbits, scale, eps, out_dtype, block):
+    def forward(ctx, q, k, v, planes_T, L, Kbits, scale, eps, out_dtype, block, bthd=False):
         _lib.require_device(q, k, v, planes_T)
         if not fused_supported(q, k, v, Kbits):
             raise _lib.RaceError("fused RACE needs bf16 q/k/v with head dim 64 or 128 and K <= 4")
@@ -57,7 +67,7 @@ class RaceAttentionFn(Function):
         lib = _lib.lib()
         state = _lib.workspace(lib.race_qkv_state_bytes(sh), q.device)
         scratch = _lib.workspace(lib.race_qkv_scratch_bytes(sh, 0), q.device)
-        out = torch.empty(B, Hq, T, D, dtype=out_dtype, device=q.device)
+        out = _out_rows(B, Hq, T, D, out_dtype, q.device, bthd)
         qv, _ = _lib.view4(q)
         kv_, _ = _lib.view4(k)
         vv, _ = _lib.view4(v)
@@ -77,14 +87,12 @@ class RaceAttentionFn(Function):
         sh = qkv_shape(q, k, L, Kbits, scale, eps, block)
         lib = _lib.lib()
         scratch = _lib.workspace(lib.race_qkv_scratch_bytes(sh, 1), q.device)
-        dq = torch.empty(q.shape, dtype=q.dtype, device=q.device)
-        dk = torch.empty(k.shape, dtype=k.dtype, device=k.device)
-        dv = torch.empty(v.shape, dtype=v.dtype, device=v.device)
+        dq, dk, dv = torch.empty_like(q), torch.empty_like(k), torch.empty_like(v)
         views = [_lib.view4(t)[0] for t in (q, k, v, go, dq, dk, dv)]
         _lib.check(lib.race_qkv_bwd(sh, views[0], views[1], views[2], views[3], _lib.ptr(planes),
                                     _lib.ptr(state), state.numel(), views[4], views[5], views[6],
                                     _lib.ptr(scratch), scratch.numel(), _lib.stream_of(q)), "race_qkv_bwd")
-        return dq, dk, dv, None, None, None, None, None, None, None
+        return dq, dk, dv, None, None, None, None, None, None, None, None
 
 
 def race_causal_attention(q, k, v, planes_T, L, Kbits, scale=None, eps=1e-6, out_dtype=None, block=0):
@@ -99,11 +107,11 @@ def race_causal_attention(q, k, v, planes_T, L, Kbits, scale=None, eps=1e-6, out
 
 
 def race_causal_attention_with_state(q, k, v, planes_T, L, Kbits, scale=None, eps=1e-6, out_dtype=None,
-                                     state_out=None):
+                                     state_out=None, bthd=False):
     """Forward only (no autograd): (out, A [B*Hkv,S], Bs [B*Hkv,S,D]) -- the output and
     the final bucket state (race_prefix_ref's A_final / B_final, race_common.py:88-90),
     which seeds race_attention_amd.decode.RaceDecodeState. `state_out` gives the (A, Bs)
-    to write (contiguous fp32); new tensors otherwise."""
+    to write (contiguous fp32); new tensors otherwise. `bthd`: out is a view of [B,T,Hq,D] memory."""
     _lib.require_device(q, k, v, planes_T)
     if scale is None:
         scale = math.sqrt(q.shape[-1])
@@ -120,7 +128,7 @@ def race_causal_attention_with_state(q, k, v, planes_T, L, Kbits, scale=None, ep
     lib = _lib.lib()
     work = _lib.workspace(lib.race_qkv_state_bytes(sh), q.device)
     scratch = _lib.workspace(lib.race_qkv_scratch_bytes(sh, 0), q.device)
-    out = torch.empty(B, Hq, T, D, dtype=out_dtype, device=q.device)
+    out = _out_rows(B, Hq, T, D, out_dtype, q.device, bthd)
     if state_out is None:
         A = torch.empty(B * Hkv, S, dtype=torch.float32, device=q.device)
         Bs = torch.empty(B * Hkv, S, D, dtype=torch.float32, device=q.device)

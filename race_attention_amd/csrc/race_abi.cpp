@@ -293,8 +293,8 @@ static int hash_common(const race_hash_shape *sh, const race_tensor &x, int x_dt
         return fail(RACE_ERR_UNSUPPORTED, "race_soft_hash: T = %d tokens, at most 2^30 are supported", sh->T);
     if (sh->K < 1 || sh->K > 8)
         return fail(RACE_ERR_UNSUPPORTED, "race_soft_hash: K = %d, supported 1..8", sh->K);
-    if (x_dtype != RACE_F32 && x_dtype != RACE_BF16)
-        return fail(RACE_ERR_INVALID, "race_soft_hash: dtype must be RACE_F32 or RACE_BF16");
+    if (x_dtype != RACE_F32 && x_dtype != RACE_BF16 && x_dtype != RACE_BF16_AS_F32)
+        return fail(RACE_ERR_INVALID, "race_soft_hash: dtype must be RACE_F32, RACE_BF16 or RACE_BF16_AS_F32");
     if (sh->D > 256 || (int64_t)sh->D * sh->L * sh->K > 16384)
         return fail(RACE_ERR_UNSUPPORTED, "race_soft_hash: D <= 256 and D*L*K <= 16384 required");
     if (!(sh->scale > 0.0f))
@@ -329,7 +329,7 @@ int race_soft_hash_fwd(const race_hash_shape *sh, race_tensor x, int x_dtype, co
     if (!probs)
         return fail(RACE_ERR_INVALID, "race_soft_hash_fwd: null probs");
     P.probs = probs;
-    return hip_check(prof_softhash(P, x_dtype == RACE_BF16, 0, hs(stream)), "race_soft_hash_fwd");
+    return hip_check(prof_softhash(P, x_dtype != RACE_F32, 0, hs(stream)), "race_soft_hash_fwd");
 }
 
 int race_soft_hash_bwd(const race_hash_shape *sh, race_tensor x, int x_dtype, const float *planes_T,
@@ -342,7 +342,7 @@ int race_soft_hash_bwd(const race_hash_shape *sh, race_tensor x, int x_dtype, co
     RACE_TRY(check_view(dx, "race_soft_hash_bwd: dx", false));
     P.gprobs = gprobs;
     P.dx = to_view(dx);
-    return hip_check(prof_softhash(P, x_dtype == RACE_BF16, 1, hs(stream)), "race_soft_hash_bwd");
+    return hip_check(prof_softhash(P, x_dtype != RACE_F32, 1, hs(stream)), "race_soft_hash_bwd");
 }
 
 int race_soft_hash_bwd_partials(const race_hash_shape *sh)
@@ -364,7 +364,7 @@ int race_soft_hash_bwd_scale(const race_hash_shape *sh, race_tensor x, int x_dty
     P.gprobs = gprobs;
     P.dx = to_view(dx);
     P.gscale = gscale_partials;
-    return hip_check(prof_softhash(P, x_dtype == RACE_BF16, 1, hs(stream)), "race_soft_hash_bwd_scale");
+    return hip_check(prof_softhash(P, x_dtype != RACE_F32, 1, hs(stream)), "race_soft_hash_bwd_scale");
 }
 
 // The same two calls with the scale read on the device (BatchedACE's learnable temperature,
@@ -383,7 +383,7 @@ int race_soft_hash_fwd_dscale(const race_hash_shape *sh, race_tensor x, int x_dt
         return fail(RACE_ERR_INVALID, "race_soft_hash_fwd_dscale: null probs");
     P.probs = probs;
     P.scale_dev = scale_dev;
-    return hip_check(prof_softhash(P, x_dtype == RACE_BF16, 0, hs(stream)), "race_soft_hash_fwd_dscale");
+    return hip_check(prof_softhash(P, x_dtype != RACE_F32, 0, hs(stream)), "race_soft_hash_fwd_dscale");
 }
 
 int race_soft_hash_bwd_dscale(const race_hash_shape *sh, race_tensor x, int x_dtype, const float *planes_T,
@@ -404,7 +404,7 @@ int race_soft_hash_bwd_dscale(const race_hash_shape *sh, race_tensor x, int x_dt
     P.gscale = gscale_partials;
     P.scale_dev = scale_dev;
     hipStream_t st = hs(stream);
-    RACE_TRY(hip_check(prof_softhash(P, x_dtype == RACE_BF16, 1, st), "race_soft_hash_bwd_dscale"));
+    RACE_TRY(hip_check(prof_softhash(P, x_dtype != RACE_F32, 1, st), "race_soft_hash_bwd_dscale"));
     return hip_check(launch_scale_grad(gscale_partials, race_soft_hash_bwd_partials(&s1), scale_dev, dscale, st),
                      "race_soft_hash_bwd_dscale: scale gradient");
 }

@@ -41,8 +41,9 @@ constexpr int op_stage(int DP) { return DP >= 128 ? 16 : 32; }
 // waves per SIMD asked of the register allocator: what the LDS allows of workgroups per CU, as far as
 // it does without spills in the main variants (gq at 3: 736 against 630 us, S = 128, D = 64). Without
 // it the value kernel's state lands in AGPRs and is copied on every use
-constexpr int op_waves_gk(int DP) { return DP <= 64 ? 3 : 2; }
-constexpr int op_waves_value(int DP) { return DP <= 128 ? 3 : 2; }
+constexpr int op_waves_gq(int ST, int DP) { return DP <= 64 || (DP <= 128 && ST > 16) ? 2 : 1; }
+constexpr int op_waves_gk(int DP) { return DP <= 64 ? 3 : DP <= 128 ? 2 : 1; }
+constexpr int op_waves_value(int ST, int DP) { return DP <= 128 && ST < 128 ? 3 : 2; }
 
 template <int ST, int DP>
 struct OpCfg {
@@ -437,7 +438,7 @@ __global__ __launch_bounds__(ST * 4) void race_op_totals(const ScanParams P)
 // Forward walk: gW = go St^T + tril(go V^T) pK, gpQ = gW / (A + eps), the block totals of W^T go
 // and gA = -gpQ W, and A at every stage start for the reverse walks.
 template <int ST, int DP, bool LIN, bool VEC>
-__global__ __launch_bounds__(ST * 4) __attribute__((amdgpu_waves_per_eu(2))) void race_op_gq(const ScanParams P)
+__global__ __launch_bounds__(ST * 4) __attribute__((amdgpu_waves_per_eu(op_waves_gq(ST, DP)))) void race_op_gq(const ScanParams P)
 {
     using CF = OpCfg<ST, DP>;
     constexpr int NTD = CF::NTD, NW = ST / 16, NTH = ST * 4, TS = CF::TS, NSUB = TS / 16, LDM = 24;
@@ -632,7 +633,7 @@ __global__ __launch_bounds__(ST * 4) __attribute__((amdgpu_waves_per_eu(op_waves
 // Per stage: W (and pK) of all buckets to LDS, the 16 x 16 products over the buckets, then each
 // wave walks the stage on its own with its columns of the state in registers.
 template <int ST, int DP, bool REV, bool LIN, bool VEC>
-__global__ __launch_bounds__((OpCfg<ST, DP>::DW * 64)) __attribute__((amdgpu_waves_per_eu(op_waves_value(DP)))) void race_op_out(const ScanParams P)
+__global__ __launch_bounds__((OpCfg<ST, DP>::DW * 64)) __attribute__((amdgpu_waves_per_eu(op_waves_value(ST, DP)))) void race_op_out(const ScanParams P)
 {
     using CF = OpCfg<ST, DP>;
     constexpr int NTS = CF::NTS, NW = CF::DW, TD = CF::TD, TS = CF::DTS, NSUB = TS / 16, LDM = 24;

@@ -40,16 +40,17 @@ class RaceDecodeState:
         self.Bs.zero_()
         self.tokens = 0
 
-    def prefill(self, q, k, v, out_dtype=None):
+    def prefill(self, q, k, v, out_dtype=None, bthd=False):
         """Causal RACE over a prompt (q [B,Hq,T,D], k/v [B,Hkv,T,D] bf16) that also
-        leaves this state at the end of the prompt. Returns the prompt's output.
+        leaves this state at the end of the prompt. Returns the prompt's output [B,Hq,T,D]
+        (`bthd`: a view of [B,T,Hq,D] memory).
         The state must be fresh (prefill starts from zero)."""
         if self.tokens:
             raise RuntimeError("prefill on a non-empty state; call reset() first")
         if k.shape[:2] != (self.B, self.Hkv) or k.shape[3] != self.D:
             raise ValueError(f"prefill expects k/v [{self.B},{self.Hkv},T,{self.D}], got {tuple(k.shape)}")
         out, _, _ = race_causal_attention_with_state(q, k, v, self.planes, self.L, self.K, self.scale, self.eps,
-                                                     out_dtype, (self.A, self.Bs))
+                                                     out_dtype, (self.A, self.Bs), bthd)
         self.tokens = q.shape[2]
         return out
 

@@ -30,10 +30,12 @@ import torch
 import torch.nn as nn
 import torch.nn.functional as F
 
-from .attention import race_causal_attention
+from torch.autograd import Function
+
+from .attention import RaceAttentionFn
 from .decode import RaceDecodeState
-from .race_causal_cuda import RaceCausalFn
-from .race_common import build_planes_protos, soft_hash_probs
+from .race_causal_cuda import op_state, race_backward, race_fused_fwd
+from .race_common import SoftHashFn, build_planes_protos
 
 
 @dataclass
@@ -108,20 +110,66 @@ class RaceStateCache:
         self.prev_embedding = None
 
 
+def _streams(x):
+    """[B,T,H,D] activations as contiguous fp32 streams [B*H,T,D], cast and laid out in one pass."""
+    B, T, H, D = x.shape
+    x = x.transpose(1, 2)
+    x = x.contiguous() if x.dtype == torch.float32 else x.to(torch.float32, memory_format=torch.contiguous_format)
+    return x.view(B * H, T, D)
+
+
+def _activations(x, B, dtype):
+    """The inverse: [B*H,T,D] fp32 streams as contiguous [B,T,H,D] activations of `dtype`."""
+    x = x.view(B, -1, *x.shape[1:]).transpose(1, 2)
+    return x.contiguous() if dtype == torch.float32 else x.to(dtype, memory_format=torch.contiguous_format)
+
+
+def _per_query_head(x, rep):
+    """[B*Hkv, ...] streams repeated for the `rep` query heads of each group."""
+    return x if rep == 1 else x.unsqueeze(1).expand(-1, rep, *x.shape[1:]).reshape(x.shape[0] * rep, *x.shape[1:])
+
+
+def _group_sum(x, rep):
+    """The transpose of _per_query_head, in fp32."""
+    return x if rep == 1 else x.view(x.shape[0] // rep, rep, *x.shape[1:]).sum(1)
+
+
+class _RaceScanFn(Function):
+    """y [B,T,Hq,D] = causal RACE in fp32 of probsK [B*Hkv,T,S], probsQ [B*Hq,T,S] (fp32) and
+    v [B,T,Hkv,D], y in `dtype`; query head h reads kv head h // (Hq / Hkv)."""
+
+    @staticmethod
+    def forward(ctx, probsK, probsQ, v, eps, dtype):
+        rep = probsQ.shape[0] // probsK.shape[0]
+        pK, V = _per_query_head(probsK, rep), _per_query_head(_streams(v), rep)
+        state = op_state(pK, V)  # the forward block states stay there for the backward
+        out = race_fused_fwd(pK, probsQ, V, eps, 0, state=state)
+        ctx.save_for_backward(pK, probsQ, V, state)
+        ctx.cfg = (float(eps), v.shape[0], v.dtype, rep)
+        return _activations(out, v.shape[0], dtype)
+
+    @staticmethod
+    def backward(ctx, grad):
+        pK, probsQ, V, state = ctx.saved_tensors
+        eps, B, v_dtype, rep = ctx.cfg
+        gpk, gpq, gv = race_backward(pK, probsQ, V, _streams(grad), eps, 0, state=state)
+        return _group_sum(gpk, rep), gpq, _activations(_group_sum(gv, rep), B, v_dtype), None, None
+
+
 def race_attend_fp32(q, k, v, planes_T, protos_T, L, Kbits, eps):
     """The reference seam's attention core (gpt.py:132-140) on [B,T,H,D] activations: fp32
-    soft-hash (fp32 planes) and fp32 causal scan on the HIP kernels, k and v repeated over each
-    query-head group; returns y [B,T,Hq,D] in q's dtype."""
-    B, T, Hq, D = q.shape
-    rep = Hq // k.shape[2]
-    qf = q.transpose(1, 2).contiguous().float()
-    kf = k.transpose(1, 2).contiguous().float()
-    vf = v.transpose(1, 2).contiguous().float()
-    if rep > 1:
-        kf, vf = kf.repeat_interleave(rep, 1), vf.repeat_interleave(rep, 1)
-    probsK, probsQ, V2, N = soft_hash_probs(qf, kf, vf, planes_T, protos_T, L, Kbits, 1, True)
-    y = RaceCausalFn.apply(probsK, probsQ, V2, eps).view(B, Hq, T, D)
-    return y.transpose(1, 2).to(q.dtype)
+    soft-hash (fp32 planes) and fp32 causal scan on the HIP kernels, the key probabilities and v
+    repeated over each query-head group; returns y [B,T,Hq,D] in q's dtype. bf16 q and k are read as
+    they are (their values are exact in fp32; the planes stay fp32), in the activations' own layout."""
+    if protos_T.shape[1] != 1 << Kbits:
+        raise ValueError(f"protos_T has {protos_T.shape[1]} corners, expected 2^{Kbits}")
+
+    def probs(x):
+        if x.dtype not in (torch.float32, torch.bfloat16):
+            x = x.float()
+        return SoftHashFn.apply(x.transpose(1, 2), planes_T, L, Kbits, 1, False, math.sqrt(x.shape[3]), True)
+
+    return _RaceScanFn.apply(probs(k), probs(q), v, eps, q.dtype)
 
 
 def race_attend(q, k, v, planes_T, L, Kbits, eps, state=None, precision="bf16", protos_T=None):
@@ -139,9 +187,10 @@ def race_attend(q, k, v, planes_T, L, Kbits, eps, state=None, precision="bf16", 
         raise ValueError(f"race precision must be 'fp32' or 'bf16', got {precision!r}")
     qt, kt, vt = q.transpose(1, 2), k.transpose(1, 2), v.transpose(1, 2)
     if state is None:
-        return race_causal_attention(qt, kt, vt, planes_T, L, Kbits, eps=eps, out_dtype=q.dtype).transpose(1, 2)
+        return RaceAttentionFn.apply(qt, kt, vt, planes_T, L, Kbits, math.sqrt(q.shape[3]), eps, q.dtype, 0,
+                                     True).transpose(1, 2)
     if state.tokens == 0 and q.shape[1] > 1:
-        return state.prefill(qt, kt, vt, out_dtype=q.dtype).transpose(1, 2)
+        return state.prefill(qt, kt, vt, out_dtype=q.dtype, bthd=True).transpose(1, 2)
     ys = [state.step(q[:, t].contiguous(), k[:, t].contiguous(), v[:, t].contiguous()) for t in range(q.shape[1])]
     return torch.stack(ys, 1)
 

@@ -177,4 +177,6 @@ class RaceCausalCuda(nn.Module):
         probsK, probsQ, V2, N = soft_hash_probs(Q, K, V, self.planes_T, self.protos_T,
                                                 self.L, self.Kbits, self.M, self.share_planes)
         out_NTD = RaceCausalFn.apply(probsK, probsQ, V2, self.eps)
+        if self.M == 1:
+            return out_NTD.view(B, H, T, D)  # (the mean of one copy)
         return out_NTD.view(self.M, B, H, T, D).mean(dim=0)

@@ -48,13 +48,16 @@ def _hash_shape(X, L, Kbits, M, unshared, scale):
 
 
 class SoftHashFn(Function):
-    """probs [Mp*B*H, T, L*2^K] fp32 of X [B,H,T,D] (Mp = M when unshared, else 1)."""
+    """probs [Mp*B*H, T, L*2^K] fp32 of X [B,H,T,D] (Mp = M when unshared, else 1). The planes of
+    bf16 X are rounded to bf16 as the reference's, unless `fp32_planes` (X cast to fp32 there)."""
 
     @staticmethod
-    def forward(ctx, X, planes_T, L, Kbits, M, unshared, scale):
+    def forward(ctx, X, planes_T, L, Kbits, M, unshared, scale, fp32_planes=False):
         _lib.require_device(X, planes_T)
         B, H, T, D = X.shape
         code = _lib.dtype_code(X.dtype)
+        if fp32_planes and code == _lib.RACE_BF16:
+            code = _lib.RACE_BF16_AS_F32
         planes = planes_T.detach().float().contiguous()
         xv, Xc = _lib.view4(X)
         Mp = M if unshared else 1
@@ -63,23 +66,23 @@ class SoftHashFn(Function):
         _lib.check(_lib.lib().race_soft_hash_fwd(sh, xv, code, _lib.ptr(planes), _lib.ptr(probs),
                                                  _lib.stream_of(X)), "race_soft_hash_fwd")
         ctx.save_for_backward(Xc, planes)
-        ctx.cfg = (L, Kbits, M, unshared, scale)
+        ctx.cfg = (L, Kbits, M, unshared, scale, code)
         return probs
 
     @staticmethod
     def backward(ctx, gprobs):
         Xc, planes = ctx.saved_tensors
-        L, Kbits, M, unshared, scale = ctx.cfg
+        L, Kbits, M, unshared, scale, code = ctx.cfg
         B, H, T, D = Xc.shape
         Mp = M if unshared else 1
         g = gprobs.float().contiguous().view(Mp, B * H, T, -1)
-        dX = torch.empty(B, H, T, D, dtype=Xc.dtype, device=Xc.device)
+        dX = torch.empty_like(Xc)  # in X's own memory order: no layout copy on the way to the leaf
         xv, _ = _lib.view4(Xc)
         dv, _ = _lib.view4(dX)
         sh = _hash_shape(Xc, L, Kbits, Mp, unshared, scale)
-        _lib.check(_lib.lib().race_soft_hash_bwd(sh, xv, _lib.dtype_code(Xc.dtype), _lib.ptr(planes),
-                                                 _lib.ptr(g), dv, _lib.stream_of(Xc)), "race_soft_hash_bwd")
-        return dX, None, None, None, None, None, None
+        _lib.check(_lib.lib().race_soft_hash_bwd(sh, xv, code, _lib.ptr(planes), _lib.ptr(g), dv,
+                                                 _lib.stream_of(Xc)), "race_soft_hash_bwd")
+        return dX, None, None, None, None, None, None, None
 
 
 def soft_hash_probs(Q, K, V, planes_T, protos_T, L, Kbits, M, share_planes=True, scale=None):

@@ -1,0 +1,74 @@
+"""Memory orders of the attention seam: outputs and gradients of race_attend stay in the [B,T,H,D]
+order of the activations (no layout copies), with the values of the contiguous [B,H,T,D] call."""
+import math
+
+import pytest
+import torch
+
+pytestmark = pytest.mark.gpu
+EPS = 1e-6
+
+
+@pytest.mark.parametrize("B,T,Hq,Hkv,D,L,K", [(2, 100, 4, 2, 64, 8, 4), (1, 513, 3, 3, 128, 3, 3), (2, 33, 6, 1, 64, 16, 4)])
+def test_attend_bf16_equals_contiguous_layout(dev, B, T, Hq, Hkv, D, L, K):
+    from race_attention_amd import build_planes_protos, race_causal_attention
+    from race_attention_amd.nanochat import race_attend
+    g = torch.Generator().manual_seed(T)
+    planes, _ = build_planes_protos(D, K, L, 1, device=dev, seed=0)
+    rows = [torch.randn(B, T, h, D, generator=g).to(torch.bfloat16) for h in (Hq, Hkv, Hkv, Hq)]
+    x = [t.to(dev).requires_grad_(True) for t in rows[:3]]
+    y = race_attend(*x, planes, L, K, EPS)
+    assert y.shape == (B, T, Hq, D) and y.is_contiguous()
+    y.backward(rows[3].to(dev))
+    z = [t.to(dev).transpose(1, 2).contiguous().requires_grad_(True) for t in rows[:3]]
+    o = race_causal_attention(*z, planes, L, K, eps=EPS)
+    assert o.is_contiguous()
+    o.backward(rows[3].to(dev).transpose(1, 2).contiguous())
+    assert torch.equal(y, o.transpose(1, 2))
+    for a, b in zip(x, z):
+        assert a.grad.is_contiguous() and torch.equal(a.grad, b.grad.transpose(1, 2))
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32, torch.float16])
+@pytest.mark.parametrize("Hq,Hkv,packed", [(4, 4, False), (4, 2, False), (2, 2, True)])
+def test_attend_fp32_equals_the_composed_ops(dev, dtype, Hq, Hkv, packed):
+    """race_attend's fp32 path against soft_hash_probs + RaceCausalFn on explicit fp32 copies: the same
+    kernels on the same values (bitwise), one rounding to the activations' dtype. `packed`: q, k, v are
+    slices of one [B,T,3,H,D] tensor, whose gradient collects all three."""
+    from race_attention_amd import RaceCausalFn, build_planes_protos, soft_hash_probs
+    from race_attention_amd.nanochat import race_attend
+    B, T, D, L, K = 2, 150, 64, 4, 4
+    g = torch.Generator().manual_seed(3)
+    planes, protos = build_planes_protos(D, K, L, 1, device=dev, seed=0)
+    rows = [torch.randn(B, T, h, D, generator=g).to(dtype) for h in (Hq, Hkv, Hkv, Hq)]
+
+    def composed(q, k, v):
+        rep = q.shape[2] // k.shape[2]
+        f = [t.transpose(1, 2).contiguous().float() for t in (q, k, v)]
+        if rep > 1:
+            f[1:] = [t.repeat_interleave(rep, 1) for t in f[1:]]
+        pK, pQ, V2, _ = soft_hash_probs(*f, planes, protos, L, K, 1, True, scale=math.sqrt(D))
+        return RaceCausalFn.apply(pK, pQ, V2, EPS).view(B, Hq, T, D).transpose(1, 2).to(q.dtype)
+
+    res = []
+    for fn in (lambda q, k, v: race_attend(q, k, v, planes, L, K, EPS, precision="fp32", protos_T=protos), composed):
+        if packed:
+            leaves = [torch.stack([t.to(dev) for t in rows[:3]], 2).requires_grad_(True)]
+            x = leaves[0].unbind(2)
+        else:
+            leaves = x = [t.to(dev).requires_grad_(True) for t in rows[:3]]
+        y = fn(*x)
+        assert y.dtype == dtype and y.shape == (B, T, Hq, D)
+        y.backward(rows[3].to(dev))
+        res.append([y.detach()] + [t.grad for t in leaves])
+    for i, (a, b) in enumerate(zip(*res)):
+        if Hq == Hkv or i < 2:
+            assert torch.equal(a, b), i
+        else:
+            # k, v of a group: the heads' fp32 gradients are summed before or behind the (linear)
+            # soft-hash backward, then rounded once. dk = J (gp - <p, gp>) cancels: each of a table's 16
+            # corner terms carries 2^-24 of |gp|, which is up to ~10 times |dk| at these sizes: 1e-5 of
+            # the largest dk; two results so rounded differ by one more ulp of the activations' dtype
+            ulp = torch.finfo(dtype).eps  # the spacing of a value's binade, of the value at most
+            over = ((a.float() - b.float()).abs() - ulp * b.float().abs() - 1e-5 * b.float().abs().max()).max().item()
+            assert over <= 0, (i, over)
