@@ -6,6 +6,7 @@ HIP library; there is no CPU or PyTorch fallback. A missing library or a
 non-ROCm tensor raises.
 """
 import ctypes
+import functools
 import os
 
 import torch
@@ -42,6 +43,12 @@ class DecodeShape(ctypes.Structure):
     _fields_ = [("B", ctypes.c_int), ("Hq", ctypes.c_int), ("Hkv", ctypes.c_int), ("D", ctypes.c_int),
                 ("L", ctypes.c_int), ("K", ctypes.c_int), ("scale", ctypes.c_float), ("eps", ctypes.c_float)]
 
+
+# Argument blocks by value, built once per shape (read by the library, never written): a struct of ten
+# fields costs as much to fill as a small launch
+hash_shape = functools.lru_cache(256)(HashShape)
+qkv_shape = functools.lru_cache(256)(QKVShape)
+decode_shape = functools.lru_cache(256)(DecodeShape)
 
 # exported symbol -> (restype, argtypes); kept in sync with include/race_attention.h
 SIGNATURES = {
@@ -159,17 +166,36 @@ def check(rc, what):
 
 def require_device(*tensors):
     for t in tensors:
-        if not isinstance(t, torch.Tensor) or t.device.type != "cuda":
+        if not isinstance(t, torch.Tensor) or not t.is_cuda:
             raise RaceError("race_attention_amd runs on a ROCm GPU: every tensor must be on a "
                             "'cuda' (HIP) device; there is no CPU path")
 
 
+@functools.lru_cache(1024)
+def _size(name, args):
+    return getattr(lib(), name)(*args)
+
+
+def size(name, *args):
+    """A race_*_bytes query, asked once per shape; 0 (a refused shape leaves its reason in
+    race_last_error, an empty buffer) is asked again."""
+    return _size(name, args) or getattr(lib(), name)(*args)
+
+
 def stream_of(t):
-    return _vp(torch.cuda.current_stream(t.device).cuda_stream)
+    """The current stream of t's device as an integer (without a Stream object, 3 us a call)."""
+    return torch._C._cuda_getCurrentRawStream(t.device.index)
 
 
 def ptr(t):
-    return _vp(t.data_ptr()) if t is not None else _vp(0)
+    return t.data_ptr() if t is not None else None
+
+
+def f32_planes(planes_T):
+    """Planes as the kernels read them: contiguous fp32, no copy where they are."""
+    if planes_T.dtype == torch.float32 and planes_T.is_contiguous():
+        return planes_T.detach()
+    return planes_T.detach().float().contiguous()
 
 
 def view4(t):

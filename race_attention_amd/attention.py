@@ -27,7 +27,8 @@ def fused_supported(q, k, v, Kbits):
 
 def _bf16_rows(t):
     """A [B,H,T,D] bf16 view whose rows the kernels can read as 16-byte vectors."""
-    if t.stride(3) != 1 or t.data_ptr() % 16 or any(s % 8 for s in t.stride()[:3]):
+    sb, sh, st, sd = t.stride()
+    if sd != 1 or t.data_ptr() % 16 or (sb | sh | st) % 8:
         t = t.contiguous()
     return t
 
@@ -41,7 +42,7 @@ def _out_rows(B, H, T, D, dtype, device, bthd):
 
 def qkv_shape(q, k, L, Kbits, scale, eps, block=0):
     B, Hq, T, D = q.shape
-    return _lib.QKVShape(B, Hq, k.shape[1], T, D, L, Kbits, float(scale), float(eps), int(block))
+    return _lib.qkv_shape(B, Hq, k.shape[1], T, D, L, Kbits, float(scale), float(eps), int(block))
 
 
 class RaceAttentionFn(Function):
@@ -59,7 +60,7 @@ class RaceAttentionFn(Function):
         if k.shape != (B, k.shape[1], T, D) or v.shape != k.shape or Hq % k.shape[1]:
             raise ValueError(f"q {tuple(q.shape)} / k {tuple(k.shape)} / v {tuple(v.shape)} mismatch")
         q, k, v = _bf16_rows(q), _bf16_rows(k), _bf16_rows(v)
-        planes = planes_T.detach().float().contiguous()
+        planes = _lib.f32_planes(planes_T)
         if planes.shape != (D, L * Kbits):
             raise ValueError(f"planes_T must be [{D}, {L * Kbits}], got {tuple(planes.shape)}")
         out_dtype = out_dtype or q.dtype
@@ -122,7 +123,7 @@ def race_causal_attention_with_state(q, k, v, planes_T, L, Kbits, scale=None, ep
     Hkv, S = k.shape[1], L << Kbits
     if k.shape != (B, Hkv, T, D) or v.shape != k.shape or Hq % Hkv:
         raise ValueError(f"q {tuple(q.shape)} / k {tuple(k.shape)} / v {tuple(v.shape)} mismatch")
-    planes = planes_T.detach().float().contiguous()
+    planes = _lib.f32_planes(planes_T)
     out_dtype = out_dtype or q.dtype
     sh = qkv_shape(q, k, L, Kbits, scale, eps, 0)
     lib = _lib.lib()

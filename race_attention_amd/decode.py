@@ -64,9 +64,9 @@ class RaceDecodeState:
         q, k, v = q.contiguous(), k.contiguous(), v.contiguous()
         if out is None:
             out = torch.empty_like(q)
-        sh = _lib.DecodeShape(self.B, self.Hq, self.Hkv, self.D, self.L, self.K, self.scale, self.eps)
-        _lib.check(_lib.lib().race_decode_step(sh, _lib.ptr(q), _lib.ptr(k), _lib.ptr(v), _lib.dtype_code(q.dtype),
-                                               _lib.ptr(self.planes), _lib.ptr(self.A), _lib.ptr(self.Bs),
-                                               _lib.ptr(out), _lib.stream_of(q)), "race_decode_step")
+        sh = _lib.decode_shape(self.B, self.Hq, self.Hkv, self.D, self.L, self.K, self.scale, self.eps)
+        _lib.check(_lib.lib().race_decode_step(sh, q.data_ptr(), k.data_ptr(), v.data_ptr(), _lib.dtype_code(q.dtype),
+                                               self.planes.data_ptr(), self.A.data_ptr(), self.Bs.data_ptr(),
+                                               out.data_ptr(), _lib.stream_of(q)), "race_decode_step")
         self.tokens += 1
         return out

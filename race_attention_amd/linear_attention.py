@@ -35,7 +35,7 @@ def linear_state(queries, values):
     """A buffer for the block states that causal_dot_product(..., state=) keeps for
     causal_dot_backward(..., state=)."""
     N, H, L, E = queries.shape
-    n = _lib.lib().race_op_state_bytes(N * H, L, E, values.shape[3], 0)
+    n = _lib.size("race_op_state_bytes", N * H, L, E, values.shape[3], 0)
     return state_buffer(n, queries.device, "race_op_state_bytes")
 
 
@@ -50,7 +50,7 @@ def causal_dot_product(queries, keys, values, product, state=None):
     Q, K, V = _flat(queries), _flat(keys), _flat(values)
     out, copy_out = _dest(product, (queries, keys, values, Q, K, V))
     lib = _lib.lib()
-    ws = _lib.workspace(lib.race_op_workspace_bytes(N * H, L, E, M, 0, 0), Q.device)
+    ws = _lib.workspace(_lib.size("race_op_workspace_bytes", N * H, L, E, M, 0, 0), Q.device)
     args = (_lib.ptr(Q), _lib.ptr(K), _lib.ptr(V), _lib.ptr(out), N * H, L, E, M, 0, _lib.ptr(ws), ws.numel())
     if state is None:
         _lib.check(lib.race_causal_dot_product(*args, _lib.stream_of(Q)), "race_causal_dot_product")
@@ -73,7 +73,7 @@ def causal_dot_backward(queries, keys, values, grad_out, grad_queries, grad_keys
     ins = (queries, keys, values, grad_out, Q, K, V, G)
     (gQ, cq), (gK, ck), (gV, cv) = _dest(grad_queries, ins), _dest(grad_keys, ins), _dest(grad_values, ins)
     lib = _lib.lib()
-    ws = _lib.workspace(lib.race_op_workspace_bytes(N * H, L, E, M, 0, 1), Q.device)
+    ws = _lib.workspace(_lib.size("race_op_workspace_bytes", N * H, L, E, M, 0, 1), Q.device)
     args = (_lib.ptr(Q), _lib.ptr(K), _lib.ptr(V), _lib.ptr(G), _lib.ptr(gQ), _lib.ptr(gK), _lib.ptr(gV), N * H, L, E,
             M, 0, _lib.ptr(ws), ws.numel())
     if state is None:

@@ -32,10 +32,11 @@ import torch.nn.functional as F
 
 from torch.autograd import Function
 
+from . import _lib
 from .attention import RaceAttentionFn
 from .decode import RaceDecodeState
 from .race_causal_cuda import op_state, race_backward, race_fused_fwd
-from .race_common import SoftHashFn, build_planes_protos
+from .race_common import build_planes_protos, hash_bwd, hash_code, hash_fwd
 
 
 @dataclass
@@ -134,42 +135,57 @@ def _group_sum(x, rep):
     return x if rep == 1 else x.view(x.shape[0] // rep, rep, *x.shape[1:]).sum(1)
 
 
-class _RaceScanFn(Function):
-    """y [B,T,Hq,D] = causal RACE in fp32 of probsK [B*Hkv,T,S], probsQ [B*Hq,T,S] (fp32) and
-    v [B,T,Hkv,D], y in `dtype`; query head h reads kv head h // (Hq / Hkv)."""
+class _RaceSeamFn(Function):
+    """y [B,T,Hq,D] = causal RACE in fp32 of activations q [B,T,Hq,D], k, v [B,T,Hkv,D], y in q's dtype;
+    query head h reads kv head h // (Hq / Hkv). bf16 q and k are hashed as they are (their values
+    are exact in fp32; the planes stay fp32), in the activations' own layout."""
 
     @staticmethod
-    def forward(ctx, probsK, probsQ, v, eps, dtype):
-        rep = probsQ.shape[0] // probsK.shape[0]
-        pK, V = _per_query_head(probsK, rep), _per_query_head(_streams(v), rep)
+    def forward(ctx, q, k, v, planes_T, L, Kbits, scale, eps):
+        _lib.require_device(q, k, v, planes_T)
+        B, T, Hq, D = q.shape
+        rep = Hq // k.shape[2]
+        if k.shape != (B, T, k.shape[2], D) or v.shape[:3] != k.shape[:3] or Hq % k.shape[2]:
+            raise ValueError(f"q {tuple(q.shape)} / k {tuple(k.shape)} / v {tuple(v.shape)} mismatch")
+        planes = _lib.f32_planes(planes_T)
+        kinds, rows = [], []
+        for x in (q, k):
+            if x.dtype not in (torch.float32, torch.bfloat16):
+                x = x.float()
+            code = hash_code(x, fp32_planes=True)
+            p, xc = hash_fwd(x.transpose(1, 2), planes, L, Kbits, 1, False, scale, code)
+            kinds.append((code, p))
+            rows.append(xc)
+        pQ, pK, V = kinds[0][1], _per_query_head(kinds[1][1], rep), _per_query_head(_streams(v), rep)
         state = op_state(pK, V)  # the forward block states stay there for the backward
-        out = race_fused_fwd(pK, probsQ, V, eps, 0, state=state)
-        ctx.save_for_backward(pK, probsQ, V, state)
-        ctx.cfg = (float(eps), v.shape[0], v.dtype, rep)
-        return _activations(out, v.shape[0], dtype)
+        out = race_fused_fwd(pK, pQ, V, eps, 0, state=state)
+        ctx.save_for_backward(*rows, planes, pK, pQ, V, state)
+        ctx.cfg = (L, Kbits, float(scale), float(eps), rep, kinds[0][0], kinds[1][0], q.dtype, k.dtype, v.dtype)
+        return _activations(out, B, q.dtype)
 
     @staticmethod
     def backward(ctx, grad):
-        pK, probsQ, V, state = ctx.saved_tensors
-        eps, B, v_dtype, rep = ctx.cfg
-        gpk, gpq, gv = race_backward(pK, probsQ, V, _streams(grad), eps, 0, state=state)
-        return _group_sum(gpk, rep), gpq, _activations(_group_sum(gv, rep), B, v_dtype), None, None
+        qc, kc, planes, pK, pQ, V, state = ctx.saved_tensors
+        L, Kbits, scale, eps, rep, q_code, k_code, q_dtype, k_dtype, v_dtype = ctx.cfg
+        gpk, gpq, gv = race_backward(pK, pQ, V, _streams(grad), eps, 0, state=state)
+        needs, dq, dk, dv = ctx.needs_input_grad, None, None, None
+        if needs[0]:
+            dq = hash_bwd(qc, planes, gpq, L, Kbits, 1, False, scale, q_code).transpose(1, 2).to(q_dtype)
+        if needs[1]:
+            dk = hash_bwd(kc, planes, _group_sum(gpk, rep), L, Kbits, 1, False, scale, k_code)
+            dk = dk.transpose(1, 2).to(k_dtype)
+        if needs[2]:
+            dv = _activations(_group_sum(gv, rep), qc.shape[0], v_dtype)
+        return dq, dk, dv, None, None, None, None, None
 
 
 def race_attend_fp32(q, k, v, planes_T, protos_T, L, Kbits, eps):
     """The reference seam's attention core (gpt.py:132-140) on [B,T,H,D] activations: fp32
     soft-hash (fp32 planes) and fp32 causal scan on the HIP kernels, the key probabilities and v
-    repeated over each query-head group; returns y [B,T,Hq,D] in q's dtype. bf16 q and k are read as
-    they are (their values are exact in fp32; the planes stay fp32), in the activations' own layout."""
+    repeated over each query-head group; returns y [B,T,Hq,D] in q's dtype."""
     if protos_T.shape[1] != 1 << Kbits:
         raise ValueError(f"protos_T has {protos_T.shape[1]} corners, expected 2^{Kbits}")
-
-    def probs(x):
-        if x.dtype not in (torch.float32, torch.bfloat16):
-            x = x.float()
-        return SoftHashFn.apply(x.transpose(1, 2), planes_T, L, Kbits, 1, False, math.sqrt(x.shape[3]), True)
-
-    return _RaceScanFn.apply(probs(k), probs(q), v, eps, q.dtype)
+    return _RaceSeamFn.apply(q, k, v, planes_T, L, Kbits, math.sqrt(q.shape[3]), eps)
 
 
 def race_attend(q, k, v, planes_T, L, Kbits, eps, state=None, precision="bf16", protos_T=None):

@@ -31,7 +31,7 @@ def race_nc_fwd(probsK, probsQ, V2, eps, block=0, state=None):
     N, T, S = pK.shape
     D = V.shape[2]
     lib = _lib.lib()
-    ws = _lib.workspace(lib.race_nc_op_workspace_bytes(N, T, S, D, block, 0), pK.device)
+    ws = _lib.workspace(_lib.size("race_nc_op_workspace_bytes", N, T, S, D, block, 0), pK.device)
     out = torch.empty(N, T, D, dtype=torch.float32, device=pK.device)
     args = (_lib.ptr(pK), _lib.ptr(pQ), _lib.ptr(V), _lib.ptr(out), N, T, S, D, float(eps), block, _lib.ptr(ws),
             ws.numel())
@@ -48,7 +48,7 @@ def race_nc_bwd(probsK, probsQ, V2, grad_out, eps, block=0, state=None):
     D = V.shape[2]
     gO = grad_out.float().contiguous()
     lib = _lib.lib()
-    ws = _lib.workspace(lib.race_nc_op_workspace_bytes(N, T, S, D, block, 1), pK.device)
+    ws = _lib.workspace(_lib.size("race_nc_op_workspace_bytes", N, T, S, D, block, 1), pK.device)
     gpK, gpQ, gV = torch.empty_like(pK), torch.empty_like(pQ), torch.empty_like(V)
     args = (_lib.ptr(pK), _lib.ptr(pQ), _lib.ptr(V), _lib.ptr(gO), _lib.ptr(gpK), _lib.ptr(gpQ), _lib.ptr(gV), N, T,
             S, D, float(eps), block, _lib.ptr(ws), ws.numel())
@@ -120,8 +120,8 @@ class RaceNonCausalViewFn(Function):
         Vv = _bhtd_rows(Vhf.float())
         out = torch.empty(M, B, T, H, D, dtype=torch.float32, device=Vv.device)
         lib = _lib.lib()
-        state = state_buffer(lib.race_op_state_bytes(N, T, S, D, 0), Vv.device, "race_op_state_bytes")
-        ws = _lib.workspace(lib.race_nc_op_workspace_bytes(N, T, S, D, 0, 0), Vv.device)
+        state = state_buffer(_lib.size("race_op_state_bytes", N, T, S, D, 0), Vv.device, "race_op_state_bytes")
+        ws = _lib.workspace(_lib.size("race_nc_op_workspace_bytes", N, T, S, D, 0, 0), Vv.device)
         vv, Vv = _lib.view4(Vv)
         ov, _ = _lib.view4(_bhtd(out))
         _lib.check(lib.race_nc_fwd_view(_lib.ptr(pK), _lib.ptr(pQ), vv, ov, M * B, H, T, S, D, float(eps), 0,
@@ -142,7 +142,7 @@ class RaceNonCausalViewFn(Function):
         gpK, gpQ = torch.empty_like(pK), torch.empty_like(pQ)
         gV = torch.empty(M, B, T, H, D, dtype=torch.float32, device=pK.device)
         lib = _lib.lib()
-        ws = _lib.workspace(lib.race_nc_op_workspace_bytes(N, T, S, D, 0, 1), pK.device)
+        ws = _lib.workspace(_lib.size("race_nc_op_workspace_bytes", N, T, S, D, 0, 1), pK.device)
         vv, _ = _lib.view4(Vv)
         gov, gv_in = _lib.view4(gv_in)
         gvv, _ = _lib.view4(_bhtd(gV))
@@ -167,7 +167,7 @@ class SoftHashTempFn(Function):
             scale = torch.tensor(float(scale), device=X.device)
         _lib.require_device(scale)
         sc = scale.detach().to(torch.float32).reshape(1).contiguous()
-        planes = planes_T.detach().float().contiguous()
+        planes = _lib.f32_planes(planes_T)
         xv, Xc = _lib.view4(X)
         Mp = M if unshared else 1
         probs = torch.empty(Mp * B * H, T, L << Kbits, dtype=torch.float32, device=X.device)

@@ -25,7 +25,7 @@ from torch.autograd import Function
 
 from . import _lib
 from .attention import RaceAttentionFn, fused_supported
-from .race_common import build_planes_protos, soft_hash_probs
+from .race_common import build_planes_protos, hash_bwd, hash_code, hash_fwd, soft_hash_probs
 
 
 def fwd_chunk(T):
@@ -44,7 +44,12 @@ def _op_inputs(probsK, probsQ, V2):
     if probsK.dim() != 3 or probsQ.shape != probsK.shape or V2.dim() != 3 or V2.shape[:2] != probsK.shape[:2]:
         raise ValueError("shapes must be probsK/probsQ [N,T,S] and V2 [N,T,D], got "
                          f"{tuple(probsK.shape)}, {tuple(probsQ.shape)}, {tuple(V2.shape)}")
-    return probsK.contiguous().float(), probsQ.contiguous().float(), V2.contiguous().float()
+    return _rows(probsK), _rows(probsQ), _rows(V2)
+
+
+def _rows(x):
+    """Contiguous fp32 (x itself where it is)."""
+    return x if x.dtype == torch.float32 and x.is_contiguous() else x.contiguous().float()
 
 
 def state_buffer(nbytes, device, what):
@@ -59,7 +64,7 @@ def op_state(probsK, V2, chunk=0):
     """A buffer for the forward block states that race_fused_fwd(..., state=) keeps for
     race_backward(..., state=)."""
     N, T, S = probsK.shape
-    n = _lib.lib().race_op_state_bytes(N, T, S, V2.shape[2], max(int(chunk), 0))
+    n = _lib.size("race_op_state_bytes", N, T, S, V2.shape[2], max(int(chunk), 0))
     return state_buffer(n, probsK.device, "race_op_state_bytes")
 
 
@@ -77,7 +82,7 @@ def race_fused_fwd(probsK, probsQ, V2, eps, chunk=0, state=None):
     D = V.shape[2]
     block = max(int(chunk), 0)
     L = _lib.lib()
-    ws = _lib.workspace(L.race_op_workspace_bytes(N, T, S, D, block, 0), pK.device)
+    ws = _lib.workspace(_lib.size("race_op_workspace_bytes", N, T, S, D, block, 0), pK.device)
     out = torch.empty(N, T, D, dtype=torch.float32, device=pK.device)
     args = (_lib.ptr(pK), _lib.ptr(pQ), _lib.ptr(V), _lib.ptr(out), N, T, S, D, float(eps), block, _lib.ptr(ws),
             ws.numel())
@@ -94,12 +99,12 @@ def race_backward(probsK, probsQ, V2, grad_out, eps, chunk=0, state=None):
     from it instead of recomputed."""
     pK, pQ, V = _op_inputs(probsK, probsQ, V2)
     _lib.require_device(grad_out)
-    gO = grad_out.contiguous().float()
+    gO = _rows(grad_out)
     N, T, S = pK.shape
     D = V.shape[2]
     block = max(int(chunk), 0)
     L = _lib.lib()
-    ws = _lib.workspace(L.race_op_workspace_bytes(N, T, S, D, block, 1), pK.device)
+    ws = _lib.workspace(_lib.size("race_op_workspace_bytes", N, T, S, D, block, 1), pK.device)
     gpk = torch.empty_like(pK)
     gpq = torch.empty_like(pQ)
     gv = torch.empty_like(V)
@@ -130,6 +135,37 @@ class RaceCausalFn(Function):
         pK, pQ, V, state = ctx.saved_tensors
         gpk, gpq, gv = race_backward(pK, pQ, V, grad_out, ctx.eps, 0, state=state)
         return gpk, gpq, gv, None
+
+
+class RaceLayerFn(Function):
+    """out [B,H,T,D] fp32 of the layer in fp32 (soft-hash of Q and K, causal scan) for Q, K, V [B,H,T,D]
+    of one shape with shared planes: soft_hash_probs and RaceCausalFn as one node of the graph (three nodes
+    and their views cost as much host time as the kernels of a 2048-token call)."""
+
+    @staticmethod
+    def forward(ctx, Q, K, V, planes_T, L, Kbits, scale, eps):
+        _lib.require_device(Q, K, V, planes_T)
+        B, H, T, D = Q.shape
+        planes, codes = _lib.f32_planes(planes_T), (hash_code(Q), hash_code(K))
+        pQ, Qc = hash_fwd(Q, planes, L, Kbits, 1, False, scale, codes[0])
+        pK, Kc = hash_fwd(K, planes, L, Kbits, 1, False, scale, codes[1])
+        V2 = _rows(V).view(B * H, T, D)
+        state = op_state(pK, V2)  # the forward block states stay there for the backward
+        out = race_fused_fwd(pK, pQ, V2, eps, 0, state=state)
+        ctx.save_for_backward(Qc, Kc, planes, pK, pQ, V2, state)
+        ctx.cfg = (L, Kbits, float(scale), float(eps), codes, V.dtype)
+        return out.view(B, H, T, D)
+
+    @staticmethod
+    def backward(ctx, grad_out):
+        Qc, Kc, planes, pK, pQ, V2, state = ctx.saved_tensors
+        L, Kbits, scale, eps, codes, v_dtype = ctx.cfg
+        B, H, T, D = Qc.shape
+        gpk, gpq, gv = race_backward(pK, pQ, V2, _rows(grad_out).view(B * H, T, D), eps, 0, state=state)
+        needs = ctx.needs_input_grad
+        dQ = hash_bwd(Qc, planes, gpq, L, Kbits, 1, False, scale, codes[0]) if needs[0] else None
+        dK = hash_bwd(Kc, planes, gpk, L, Kbits, 1, False, scale, codes[1]) if needs[1] else None
+        return dQ, dK, gv.view(B, H, T, D).to(v_dtype), None, None, None, None, None
 
 
 def race_cuda_fused(probsK, probsQ, V2, eps=1e-6):
@@ -174,9 +210,9 @@ class RaceCausalCuda(nn.Module):
             # the M ensemble copies share the planes, so their mean is one copy
             return RaceAttentionFn.apply(Q, K, V, self.planes_T, self.L, self.Kbits, math.sqrt(D),
                                          self.eps, torch.float32, 0)
+        if self.M == 1 and self.share_planes and Q.shape == K.shape == V.shape:
+            return RaceLayerFn.apply(Q, K, V, self.planes_T, self.L, self.Kbits, math.sqrt(D), self.eps)
         probsK, probsQ, V2, N = soft_hash_probs(Q, K, V, self.planes_T, self.protos_T,
                                                 self.L, self.Kbits, self.M, self.share_planes)
         out_NTD = RaceCausalFn.apply(probsK, probsQ, V2, self.eps)
-        if self.M == 1:
-            return out_NTD.view(B, H, T, D)  # (the mean of one copy)
         return out_NTD.view(self.M, B, H, T, D).mean(dim=0)

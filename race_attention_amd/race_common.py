@@ -44,27 +44,42 @@ def build_planes_protos(d_k, Kbits, L, M, device="cuda", share_planes=True,
 
 def _hash_shape(X, L, Kbits, M, unshared, scale):
     B, H, T, D = X.shape
-    return _lib.HashShape(B, H, T, D, L, Kbits, M, 1 if unshared else 0, float(scale))
+    return _lib.hash_shape(B, H, T, D, L, Kbits, M, 1 if unshared else 0, float(scale))
+
+
+def hash_fwd(X, planes, L, Kbits, M, unshared, scale, code):
+    """(probs [Mp*B*H, T, L*2^K], X as read) of X [B,H,T,D] and planes as _lib.f32_planes gives them."""
+    B, H, T, D = X.shape
+    xv, Xc = _lib.view4(X)
+    probs = torch.empty((M if unshared else 1) * B * H, T, L << Kbits, dtype=torch.float32, device=X.device)
+    _lib.check(_lib.lib().race_soft_hash_fwd(_hash_shape(X, L, Kbits, M, unshared, scale), xv, code, planes.data_ptr(),
+                                             probs.data_ptr(), _lib.stream_of(X)), "race_soft_hash_fwd")
+    return probs, Xc
+
+
+def hash_bwd(Xc, planes, gprobs, L, Kbits, M, unshared, scale, code):
+    """dX, in X's own memory order (no layout copy on the way to a leaf), from gprobs fp32 contiguous."""
+    dX = torch.empty_like(Xc)
+    sh = _hash_shape(Xc, L, Kbits, M if unshared else 1, unshared, scale)
+    _lib.check(_lib.lib().race_soft_hash_bwd(sh, _lib.view4(Xc)[0], code, planes.data_ptr(), gprobs.data_ptr(),
+                                             _lib.view4(dX)[0], _lib.stream_of(Xc)), "race_soft_hash_bwd")
+    return dX
+
+
+def hash_code(X, fp32_planes=False):
+    """The soft-hash's dtype code of X; bf16 X rounds the planes to bf16, unless `fp32_planes`."""
+    code = _lib.dtype_code(X.dtype)
+    return _lib.RACE_BF16_AS_F32 if fp32_planes and code == _lib.RACE_BF16 else code
 
 
 class SoftHashFn(Function):
-    """probs [Mp*B*H, T, L*2^K] fp32 of X [B,H,T,D] (Mp = M when unshared, else 1). The planes of
-    bf16 X are rounded to bf16 as the reference's, unless `fp32_planes` (X cast to fp32 there)."""
+    """probs [Mp*B*H, T, L*2^K] fp32 of X [B,H,T,D] (Mp = M when unshared, else 1)."""
 
     @staticmethod
-    def forward(ctx, X, planes_T, L, Kbits, M, unshared, scale, fp32_planes=False):
+    def forward(ctx, X, planes_T, L, Kbits, M, unshared, scale):
         _lib.require_device(X, planes_T)
-        B, H, T, D = X.shape
-        code = _lib.dtype_code(X.dtype)
-        if fp32_planes and code == _lib.RACE_BF16:
-            code = _lib.RACE_BF16_AS_F32
-        planes = planes_T.detach().float().contiguous()
-        xv, Xc = _lib.view4(X)
-        Mp = M if unshared else 1
-        probs = torch.empty(Mp * B * H, T, L << Kbits, dtype=torch.float32, device=X.device)
-        sh = _hash_shape(X, L, Kbits, M, unshared, scale)
-        _lib.check(_lib.lib().race_soft_hash_fwd(sh, xv, code, _lib.ptr(planes), _lib.ptr(probs),
-                                                 _lib.stream_of(X)), "race_soft_hash_fwd")
+        code, planes = hash_code(X), _lib.f32_planes(planes_T)
+        probs, Xc = hash_fwd(X, planes, L, Kbits, M, unshared, scale, code)
         ctx.save_for_backward(Xc, planes)
         ctx.cfg = (L, Kbits, M, unshared, scale, code)
         return probs
@@ -72,17 +87,7 @@ class SoftHashFn(Function):
     @staticmethod
     def backward(ctx, gprobs):
         Xc, planes = ctx.saved_tensors
-        L, Kbits, M, unshared, scale, code = ctx.cfg
-        B, H, T, D = Xc.shape
-        Mp = M if unshared else 1
-        g = gprobs.float().contiguous().view(Mp, B * H, T, -1)
-        dX = torch.empty_like(Xc)  # in X's own memory order: no layout copy on the way to the leaf
-        xv, _ = _lib.view4(Xc)
-        dv, _ = _lib.view4(dX)
-        sh = _hash_shape(Xc, L, Kbits, Mp, unshared, scale)
-        _lib.check(_lib.lib().race_soft_hash_bwd(sh, xv, code, _lib.ptr(planes), _lib.ptr(g), dv,
-                                                 _lib.stream_of(Xc)), "race_soft_hash_bwd")
-        return dX, None, None, None, None, None, None, None
+        return hash_bwd(Xc, planes, gprobs.float().contiguous(), *ctx.cfg), None, None, None, None, None, None
 
 
 def soft_hash_probs(Q, K, V, planes_T, protos_T, L, Kbits, M, share_planes=True, scale=None):
