@@ -462,7 +462,7 @@ static bool aligned16(const void *p) { return (reinterpret_cast<uintptr_t>(p) & 
 static int run_scan_op(OpKernel k, const Geo &g, const ScanParams &P, hipStream_t s)
 {
     static const int prof_id[] = {RACE_PROF_OP_FWD_TOTALS, RACE_PROF_OP_FWD_READOUT, RACE_PROF_OP_BWD_TOTALS,
-                                  RACE_PROF_OP_BWD_MAIN, RACE_PROF_OP_BWD_MAIN};
+                                  RACE_PROF_OP_BWD_MAIN};
     ProfScope ps(prof_id[k], s);
     const dim3 grid((unsigned)g.NB, (unsigned)g.n_st, (unsigned)g.Z);
     return hip_check(launch_scan_op(k, g.ST, g.DP, P, grid, s), "race_op kernel launch");
@@ -592,8 +592,7 @@ static int op_bwd_impl(const float *pK, const float *pQ, const float *V, const f
     RACE_TRY(hip_check(prof_block_scan(P.ws2B, (int64_t)g.S_pad * g.DP, P.ws2A, g.S_pad, (int)g.NB, (int)g.Z, 1, s,
                                        P.ws3B, P.ws3A),
                        "block scan"));
-    RACE_TRY(run_scan_op(OP_GK, g, P, s));
-    RACE_TRY(run_scan_op(OP_GV, g, P, s));
+    RACE_TRY(run_scan_op(OP_GKV, g, P, s));
     if (part)
         RACE_TRY(hip_check(prof_reduce(part, g.n_st, N * T * D, OutView{gV, T * D, 0, D, 0, 1},
                                                   (int)N, 1, (int)T, (int)D, s), "reduce partials"));

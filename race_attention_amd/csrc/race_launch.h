@@ -21,8 +21,8 @@ struct Variant {
 hipError_t launch_scan_qkv(ScanKernel k, int ST, int DP, const ScanParams &P, dim3 grid,
                            hipStream_t s);
 // fp32 probabilities-in kernels of the op path (race_scan_op.hip): block totals, readout, gpQ with
-// the backward's block totals, gpK, gv
-enum OpKernel { OP_TOTALS = 0, OP_READOUT = 1, OP_GQ = 2, OP_GK = 3, OP_GV = 4 };
+// the backward's block totals, gpK and gv
+enum OpKernel { OP_TOTALS = 0, OP_READOUT = 1, OP_GQ = 2, OP_GKV = 3 };
 hipError_t launch_scan_op(OpKernel k, int ST, int DP, const ScanParams &P, dim3 grid, hipStream_t s);
 int op_stage_tokens(int DP);  // tokens between A checkpoints (ScanParams::ckA)
 bool qkv_variant_exists(int ST, int DP);

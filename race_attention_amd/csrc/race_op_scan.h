@@ -20,13 +20,13 @@
 // gpQ that it wrote, instead of a second pass over go St^T with a second copy of the state.
 //
 // Measured against the kernels with the state in LDS that these replace (us, one MI355X):
-//   RACE, 200003 tokens x 4 streams, S = 128, D = 64: totals 189 -> 183, readout 525 -> 372 (and no
-//     partial outputs of two bucket tiles to add, 2 x 96), gpQ + totals 707 -> 630, gpK and gv
-//     1356 -> 540 + 415: 3.3 TB/s in the gpK kernel
-//   linear attention, 2^20 tokens x 4 streams, 64 x 64: 421 -> 432, 1205 -> 920, 1687 -> 1420,
-//     3185 -> 1035 + 1020: each at 3.8 - 5.0 TB/s of its compulsory reads and writes (a plain
-//     copy moves 4.8), so HBM bounds it
-//   32752 tokens x 6 streams, S = 24, D = 128: 35 -> 34, 76 -> 58, 153 -> 122, 337 -> 98 + 84
+//   RACE, 200003 tokens x 4 streams, S = 128, D = 64: totals 189 -> 176, readout 525 -> 365 (and no
+//     partial outputs of two bucket tiles to add, 2 x 96), gpQ + totals 707 -> 610, gpK and gv
+//     1356 -> 927
+//   linear attention, 2^20 tokens x 4 streams, 64 x 64: 421 -> 424, 1205 -> 895, 1687 -> 1390,
+//     3185 -> 1960: at 3.3 - 5.0 TB/s of the compulsory reads and writes (a plain copy moves 4.8)
+//     with the matrix cores busy 64, 74, 66 and 68 % of the time
+//   32752 tokens x 6 streams, S = 24, D = 128: 35 -> 29, 76 -> 60, 153 -> 119, 337 -> 89 + 84
 #pragma once
 #include <type_traits>
 
@@ -104,22 +104,42 @@ struct OpCtx {
     int64_t slot;
 };
 
+// (tile: this kernel's bucket tile of ST)
 template <int ST>
-RACE_DEV OpCtx op_ctx(const ScanParams &P)
+RACE_DEV OpCtx op_ctx(const ScanParams &P, int blk, int tile)
 {
     OpCtx c;
     c.lane = threadIdx.x & 63;
     c.wave = threadIdx.x >> 6;
     c.n = c.lane & 15;
     c.g = c.lane >> 4;
-    c.blk = blockIdx.x;
+    c.blk = blk;
     c.z = blockIdx.z;
-    c.s0 = blockIdx.y * ST;
+    c.s0 = tile * ST;
     c.S_here = min(ST, P.S - c.s0);
     c.t_begin = c.blk * P.CB;
     c.t_end = min(P.T, c.t_begin + P.CB);
     c.slot = (int64_t)c.z * (P.NB + 1) + c.blk;
     return c;
+}
+
+// Workgroup w of the NWG that share a block's rows. They are 8 apart in launch order, so they run side
+// by side on one XCD (workgroups go round the 8 in turn) and all but the first find the rows in its L2
+// or, at worst, in the Infinity Cache. The last NB % 8 blocks form a narrower group.
+template <int NWG>
+RACE_DEV void op_place(const ScanParams &P, int &blk, int &w)
+{
+    const int i = blockIdx.x, whole = P.NB & ~7, j = i - whole * NWG;
+    if (NWG == 1) {
+        w = 0;
+        blk = i;
+    } else if (j < 0) {
+        w = (i >> 3) % NWG;
+        blk = (i >> 3) / NWG * 8 + (i & 7);
+    } else {
+        w = j / (P.NB - whole);
+        blk = whole + j % (P.NB - whole);
+    }
 }
 
 // Rows of V (and go) of one stage into LDS, row-major [TS][DP + 8] and / or transposed
@@ -382,14 +402,16 @@ RACE_DEV void put_hilo(float *hi, float *lo, int64_t o, double v)
 
 // ============================================================================ block totals
 // sum pK^T v and sum pK of each block -> workspace slot blk
-template <int ST, int DP, bool VEC>
+template <int ST, int DP, int NWG, bool VEC>
 __global__ __launch_bounds__(ST * 4) void race_op_totals(const ScanParams P)
 {
     using CF = OpCfg<ST, DP>;
     constexpr int NTD = CF::NTD, NTH = ST * 4, TS = CF::TS, NSUB = TS / 16;
     using RS = RowStage<TS, DP, NTH, 1, VEC>;
     __shared__ __align__(16) float sVt[DP * RS::LDT];
-    const OpCtx c = op_ctx<ST>(P);
+    int blk, wg;
+    op_place<NWG>(P, blk, wg);
+    const OpCtx c = op_ctx<ST>(P, blk, blockIdx.y * NWG + wg);
     const int col = c.wave * 16 + c.n;
     const uint32_t S4 = P.S * 4, off = col < c.S_here ? 4 * c.g * S4 + (c.s0 + col) * 4 : OP_OOB;
     const typename RS::Src src = op_src<RS>(P.V, P.v, P.zH, c.z);
@@ -437,7 +459,7 @@ __global__ __launch_bounds__(ST * 4) void race_op_totals(const ScanParams P)
 // ============================================================================ gpQ and suffix totals
 // Forward walk: gW = go St^T + tril(go V^T) pK, gpQ = gW / (A + eps), the block totals of W^T go
 // and gA = -gpQ W, and A at every stage start for the reverse walks.
-template <int ST, int DP, bool LIN, bool VEC>
+template <int ST, int DP, int NWG, bool LIN, bool VEC>
 __global__ __launch_bounds__(ST * 4) __attribute__((amdgpu_waves_per_eu(op_waves_gq(ST, DP)))) void race_op_gq(const ScanParams P)
 {
     using CF = OpCfg<ST, DP>;
@@ -447,7 +469,9 @@ __global__ __launch_bounds__(ST * 4) __attribute__((amdgpu_waves_per_eu(op_waves
     __shared__ __align__(16) float sV[TS * RS::LDX], sGO[TS * RS::LDX];
     __shared__ __align__(16) float sVt[DP * RS::LDT], sGOt[DP * RS::LDT];
     __shared__ __align__(16) float sM[KS * NSUB * 16 * LDM];
-    const OpCtx c = op_ctx<ST>(P);
+    int blk, wg;
+    op_place<NWG>(P, blk, wg);
+    const OpCtx c = op_ctx<ST>(P, blk, blockIdx.y * NWG + wg);
     const int col = c.wave * 16 + c.n;
     const uint32_t S4 = P.S * 4, off = col < c.S_here ? 4 * c.g * S4 + (c.s0 + col) * 4 : OP_OOB;
     const typename RS::Src sv = op_src<RS>(P.V, P.v, P.zH, c.z), sg = op_src<RS>(P.gO, P.go, P.zH, c.z);
@@ -532,17 +556,21 @@ __global__ __launch_bounds__(ST * 4) __attribute__((amdgpu_waves_per_eu(op_waves
 // ============================================================================ gpK
 // Reverse walk: gpK = gAhat + V dS^T + triu(V go^T) W, with dS the sum of W^T go and gAhat that of
 // gA = -gpQ W over the tokens behind.
+template <int ST, int DP>
+struct OpGkLds {
+    static constexpr int TS = op_stage(DP), NW = ST / 16, NSUB = TS / 16, LDM = 24;
+    static constexpr int KS = op_shares(NW, NSUB, DP / 16), LDX = op_pitch(DP), LDT = op_pitch(TS);
+    float V[TS * LDX], GO[TS * LDX], GOt[DP * LDT], M[KS * NSUB * 16 * LDM];
+};
+
 template <int ST, int DP, bool LIN, bool VEC>
-__global__ __launch_bounds__(ST * 4) __attribute__((amdgpu_waves_per_eu(op_waves_gk(DP)))) void race_op_gk(const ScanParams P)
+RACE_DEV void op_gk(const ScanParams &P, const OpCtx &c, OpGkLds<ST, DP> &lds)
 {
     using CF = OpCfg<ST, DP>;
-    constexpr int NTD = CF::NTD, NW = ST / 16, NTH = ST * 4, TS = CF::TS, NSUB = TS / 16, LDM = 24;
-    constexpr int KS = op_shares(NW, NSUB, DP / 16);
+    using LD = OpGkLds<ST, DP>;
+    constexpr int NTD = CF::NTD, NW = LD::NW, NTH = ST * 4, TS = LD::TS, NSUB = LD::NSUB, LDM = LD::LDM, KS = LD::KS;
     using RS = RowStage<TS, DP, NTH, 2, VEC>;
-    __shared__ __align__(16) float sV[TS * RS::LDX], sGO[TS * RS::LDX];
-    __shared__ __align__(16) float sGOt[DP * RS::LDT];
-    __shared__ __align__(16) float sM[KS * NSUB * 16 * LDM];
-    const OpCtx c = op_ctx<ST>(P);
+    float *const sV = lds.V, *const sGO = lds.GO, *const sGOt = lds.GOt, *const sM = lds.M;
     const int col = c.wave * 16 + c.n;
     const uint32_t S4 = P.S * 4, off = col < c.S_here ? 4 * c.g * S4 + (c.s0 + col) * 4 : OP_OOB;
     const typename RS::Src sv = op_src<RS>(P.V, P.v, P.zH, c.z), sg = op_src<RS>(P.gO, P.go, P.zH, c.z);
@@ -627,24 +655,39 @@ __global__ __launch_bounds__(ST * 4) __attribute__((amdgpu_waves_per_eu(op_waves
     }
 }
 
+template <int ST, int DP, int NWG, bool LIN, bool VEC>
+__global__ __launch_bounds__(ST * 4) __attribute__((amdgpu_waves_per_eu(op_waves_gk(DP)))) void race_op_gk(const ScanParams P)
+{
+    __shared__ __align__(16) OpGkLds<ST, DP> lds;
+    int blk, wg;
+    op_place<NWG>(P, blk, wg);
+    op_gk<ST, DP, LIN, VEC>(P, op_ctx<ST>(P, blk, blockIdx.y * NWG + wg), lds);
+}
+
 // ============================================================================ readout / gv
 // REV = false: out[t] = sum_s W_t[s] sum_{tau <= t} pK_tau[s] v_tau
 // REV = true:  gv[t]  = sum_s pK_t[s] sum_{tau >= t} W_tau[s] go_tau   (blocks and stages in reverse)
 // Per stage: W (and pK) of all buckets to LDS, the 16 x 16 products over the buckets, then each
 // wave walks the stage on its own with its columns of the state in registers.
+template <int ST, int DP>
+struct OpValueLds {
+    using CF = OpCfg<ST, DP>;
+    static constexpr int TS = CF::DTS, NSUB = TS / 16, LDM = 24, LDS_ = op_pitch(ST), LDT = op_pitch(TS);
+    static constexpr int KS = op_shares(CF::DW, NSUB, CF::NTS);
+    float Q[TS * LDS_], K[TS * LDS_], Kt[ST * LDT], M[KS * NSUB * 16 * LDM];
+};
+
 template <int ST, int DP, bool REV, bool LIN, bool VEC>
-__global__ __launch_bounds__((OpCfg<ST, DP>::DW * 64)) __attribute__((amdgpu_waves_per_eu(op_waves_value(ST, DP)))) void race_op_out(const ScanParams P)
+RACE_DEV void op_value(const ScanParams &P, const OpCtx &c, OpValueLds<ST, DP> &lds)
 {
     using CF = OpCfg<ST, DP>;
-    constexpr int NTS = CF::NTS, NW = CF::DW, TD = CF::TD, TS = CF::DTS, NSUB = TS / 16, LDM = 24;
-    constexpr int LDS_ = op_pitch(ST), LDT = op_pitch(TS);
-    constexpr int KS = op_shares(NW, NSUB, NTS);
+    using LD = OpValueLds<ST, DP>;
+    constexpr int NTS = CF::NTS, NW = CF::DW, TD = CF::TD, TS = LD::TS, NSUB = LD::NSUB, LDM = LD::LDM;
+    constexpr int LDS_ = LD::LDS_, LDT = LD::LDT, KS = LD::KS;
     // W: a wave job covers CW buckets of the whole stage, lane (rg, lc): 4 tokens x 4 buckets
     constexpr int CW = 1024 / TS, NJ = ST / CW, JPW = (NJ + NW - 1) / NW, LC = CW / 4, RG = TS / 4;
     static_assert(NJ >= 1 && LC * RG == 64, "one job per 1024 probabilities");
-    __shared__ __align__(16) float sQ[TS * LDS_], sK[TS * LDS_], sKt[ST * LDT];
-    __shared__ __align__(16) float sM[KS * NSUB * 16 * LDM];
-    const OpCtx c = op_ctx<ST>(P);
+    float *const sQ = lds.Q, *const sK = lds.K, *const sKt = lds.Kt, *const sM = lds.M;
     const int rg = c.lane / LC, lc = c.lane % LC;
     const int64_t zoff = (int64_t)c.z * P.T * P.S;
     const float *xsrc = REV ? op_rows(P.gO, P.go, P.zH, c.z) : op_rows(P.V, P.v, P.zH, c.z);
@@ -819,6 +862,30 @@ __global__ __launch_bounds__((OpCfg<ST, DP>::DW * 64)) __attribute__((amdgpu_wav
         }
         __syncthreads();
     }
+}
+
+template <int ST, int DP, bool REV, bool LIN, bool VEC>
+__global__ __launch_bounds__((OpCfg<ST, DP>::DW * 64)) __attribute__((amdgpu_waves_per_eu(op_waves_value(ST, DP)))) void race_op_out(const ScanParams P)
+{
+    __shared__ __align__(16) OpValueLds<ST, DP> lds;
+    op_value<ST, DP, REV, LIN, VEC>(P, op_ctx<ST>(P, blockIdx.x, blockIdx.y), lds);
+}
+
+// ============================================================================ gpK and gv in one launch
+// The gpK workgroups of a block (ST / BT of them) and its gv workgroup side by side: both walk the block
+// in reverse over the same pQ, go, pK and A checkpoints.
+template <int ST, int BT, int DP, bool LIN, bool VEC>
+__global__ __launch_bounds__(BT * 4) __attribute__((amdgpu_waves_per_eu(op_waves_value(ST, DP)))) void race_op_gkv(const ScanParams P)
+{
+    static_assert(BT == OpCfg<ST, DP>::DW * 16, "one workgroup size");
+    constexpr int NB_ = ST / BT;
+    __shared__ __align__(16) union { OpGkLds<BT, DP> k; OpValueLds<ST, DP> v; } lds;
+    int blk, wg;
+    op_place<NB_ + 1>(P, blk, wg);
+    if (wg < NB_)
+        op_gk<BT, DP, LIN, VEC>(P, op_ctx<BT>(P, blk, blockIdx.y * NB_ + wg), lds.k);
+    else
+        op_value<ST, DP, true, LIN, VEC>(P, op_ctx<ST>(P, blk, blockIdx.y), lds.v);
 }
 
 }  // namespace race

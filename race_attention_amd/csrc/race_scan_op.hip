@@ -5,6 +5,12 @@
 
 namespace race {
 
+// gpK and gv in one launch wherever both kinds of workgroup have as many waves: 64 buckets and head dim
+// 64 (2^20 tokens x 4 streams, linear) 1995 -> 1960 us, 128 buckets (2048 tokens x 16 streams) 54.6 ->
+// 51.1, (200003 x 4) 916 -> 927 without the launch between them
+template <int ST, int BT, int DP>
+constexpr bool op_one_launch = BT == 16 * OpCfg<ST, DP>::DW;
+
 template <int ST, int DP, bool VEC>
 static hipError_t launch_v(OpKernel k, const ScanParams &P, dim3 grid, hipStream_t s)
 {
@@ -12,12 +18,17 @@ static hipError_t launch_v(OpKernel k, const ScanParams &P, dim3 grid, hipStream
     // read twice, but two or three independent workgroups share a CU instead of one (before the
     // suffixes moved to fp64, 200003 tokens x 4 streams, S = 128, D = 64: gq 565 -> 535, gk 521 ->
     // 508 us; 32 buckets: 785 and 560)
-    constexpr int BT = ST < 64 ? ST : 64;
+    // the bucket kernels of a 128-bucket tile run as two workgroups of 64 buckets: V and gO are
+    // read twice, but two or three independent workgroups share a CU instead of one (before the
+    // suffixes moved to fp64, 200003 tokens x 4 streams, S = 128, D = 64: gq 565 -> 535, gk 521 ->
+    // 508 us; 32 buckets: 785 and 560). Side by side (op_place) against one half of the buckets
+    // after the other: totals 182 -> 176, gq 623 -> 615, gk 527 -> 506
+    constexpr int BT = ST < 64 ? ST : 64, NWG = ST / BT;
     const dim3 bucket(BT * 4), value(OpCfg<ST, DP>::DW * 64);
-    const dim3 bgrid(grid.x, grid.y * (ST / BT), grid.z);
+    const dim3 bgrid(grid.x * NWG, grid.y, grid.z);
     switch (k) {
     case OP_TOTALS:
-        hipLaunchKernelGGL((race_op_totals<BT, DP, VEC>), bgrid, bucket, 0, s, P);
+        hipLaunchKernelGGL((race_op_totals<BT, DP, NWG, VEC>), bgrid, bucket, 0, s, P);
         break;
     case OP_READOUT:
         if (P.linear)
@@ -27,21 +38,24 @@ static hipError_t launch_v(OpKernel k, const ScanParams &P, dim3 grid, hipStream
         break;
     case OP_GQ:
         if (P.linear)
-            hipLaunchKernelGGL((race_op_gq<BT, DP, true, VEC>), bgrid, bucket, 0, s, P);
+            hipLaunchKernelGGL((race_op_gq<BT, DP, NWG, true, VEC>), bgrid, bucket, 0, s, P);
         else
-            hipLaunchKernelGGL((race_op_gq<BT, DP, false, VEC>), bgrid, bucket, 0, s, P);
+            hipLaunchKernelGGL((race_op_gq<BT, DP, NWG, false, VEC>), bgrid, bucket, 0, s, P);
         break;
-    case OP_GK:
-        if (P.linear)
-            hipLaunchKernelGGL((race_op_gk<BT, DP, true, VEC>), bgrid, bucket, 0, s, P);
-        else
-            hipLaunchKernelGGL((race_op_gk<BT, DP, false, VEC>), bgrid, bucket, 0, s, P);
-        break;
-    case OP_GV:
-        if (P.linear)
+    case OP_GKV:
+        if constexpr (op_one_launch<ST, BT, DP>) {
+            const dim3 vgrid(grid.x * (NWG + 1), grid.y, grid.z);
+            if (P.linear)
+                hipLaunchKernelGGL((race_op_gkv<ST, BT, DP, true, VEC>), vgrid, bucket, 0, s, P);
+            else
+                hipLaunchKernelGGL((race_op_gkv<ST, BT, DP, false, VEC>), vgrid, bucket, 0, s, P);
+        } else if (P.linear) {
+            hipLaunchKernelGGL((race_op_gk<BT, DP, NWG, true, VEC>), bgrid, bucket, 0, s, P);
             hipLaunchKernelGGL((race_op_out<ST, DP, true, true, VEC>), grid, value, 0, s, P);
-        else
+        } else {
+            hipLaunchKernelGGL((race_op_gk<BT, DP, NWG, false, VEC>), bgrid, bucket, 0, s, P);
             hipLaunchKernelGGL((race_op_out<ST, DP, true, false, VEC>), grid, value, 0, s, P);
+        }
         break;
     }
     return hipGetLastError();

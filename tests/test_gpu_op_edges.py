@@ -36,6 +36,22 @@ def test_tile_edges(dev, N, T, S, D, block):
         check(name, g, ref, max(1e-4, 2.0 * f))
 
 
+@pytest.mark.parametrize("S,D", [(20, 32), (32, 64), (40, 64), (128, 64), (129, 64)])
+@pytest.mark.parametrize("NB", [1, 7, 8, 9, 16, 27])
+def test_block_counts(dev, S, D, NB):
+    """Every block of a sequence is visited by all of its workgroups, which sit 8 apart in launch order:
+    whole groups of 8 blocks and what is left over, one to three workgroups per block."""
+    from race_attention_amd.race_causal_cuda import race_backward, race_fused_fwd
+    T = 32 * NB - 5
+    pk, pq, v, go = probs(2, T, S, D, seed=S + NB)
+    out_t, gpk_t, gpq_t, gv_t, _, _ = oracle_op(pk, pq, v, go, EPS)
+    args = [x.float().to(dev) for x in (pk, pq, v, go)]
+    check("out", race_fused_fwd(*args[:3], EPS, 32), out_t, 2e-5)
+    floors = fp32_formula_floor(pk, pq, v, go, EPS, (gpk_t, gpq_t, gv_t))
+    for name, g, ref, f in zip(("gpK", "gpQ", "gV"), race_backward(*args, EPS, 32), (gpk_t, gpq_t, gv_t), floors):
+        check(name, g, ref, max(1e-4, 2.0 * f))
+
+
 @pytest.mark.parametrize("T,E,M", [(15, 15, 31), (16, 16, 32), (33, 17, 64), (65, 64, 65), (100, 129, 128)])
 def test_linear_tile_edges(dev, T, E, M):
     from race_attention_amd.linear_attention import causal_linear_attention
