@@ -34,9 +34,10 @@ def _bf16_rows(t):
 
 
 def _out_rows(B, H, T, D, dtype, device, bthd):
-    """A new [B,H,T,D] tensor, contiguous or (bthd) a view of contiguous [B,T,H,D] memory."""
+    """A new [B,H,T,D] tensor, contiguous or (bthd) in the memory order of [B,T,H,D]. No view: autograd
+    refuses in-place changes to a view that a Function returns."""
     if bthd:
-        return torch.empty(B, T, H, D, dtype=dtype, device=device).transpose(1, 2)
+        return torch.empty_strided((B, H, T, D), (T * H * D, D, H * D, 1), dtype=dtype, device=device)
     return torch.empty(B, H, T, D, dtype=dtype, device=device)
 
 
@@ -49,7 +50,7 @@ class RaceAttentionFn(Function):
     """out = causal RACE(q, k, v); q [B,Hq,T,D], k/v [B,Hkv,T,D] bf16, planes_T [D, L*K].
 
     The gradients take the memory order of q, k and v, so that autograd hands them on without a
-    layout copy; the output is contiguous, or with `bthd` a [B,Hq,T,D] view of [B,T,Hq,D] memory."""
+    layout copy; the output is contiguous, or with `bthd` in the memory order of [B,T,Hq,D]."""
 
     @staticmethod
     def forward(ctx, q, k, v, planes_T, L, Kbits, scale, eps, out_dtype, block, bthd=False):
@@ -112,7 +113,7 @@ def race_causal_attention_with_state(q, k, v, planes_T, L, Kbits, scale=None, ep
     """Forward only (no autograd): (out, A [B*Hkv,S], Bs [B*Hkv,S,D]) -- the output and
     the final bucket state (race_prefix_ref's A_final / B_final, race_common.py:88-90),
     which seeds race_attention_amd.decode.RaceDecodeState. `state_out` gives the (A, Bs)
-    to write (contiguous fp32); new tensors otherwise. `bthd`: out is a view of [B,T,Hq,D] memory."""
+    to write (contiguous fp32); new tensors otherwise. `bthd`: out is in the memory order of [B,T,Hq,D]."""
     _lib.require_device(q, k, v, planes_T)
     if scale is None:
         scale = math.sqrt(q.shape[-1])

@@ -43,7 +43,7 @@ class RaceDecodeState:
     def prefill(self, q, k, v, out_dtype=None, bthd=False):
         """Causal RACE over a prompt (q [B,Hq,T,D], k/v [B,Hkv,T,D] bf16) that also
         leaves this state at the end of the prompt. Returns the prompt's output [B,Hq,T,D]
-        (`bthd`: a view of [B,T,Hq,D] memory).
+        (`bthd`: in the memory order of [B,T,Hq,D]).
         The state must be fresh (prefill starts from zero)."""
         if self.tokens:
             raise RuntimeError("prefill on a non-empty state; call reset() first")

@@ -161,7 +161,7 @@ class _RaceSeamFn(Function):
         out = race_fused_fwd(pK, pQ, V, eps, 0, state=state)
         ctx.save_for_backward(*rows, planes, pK, pQ, V, state)
         ctx.cfg = (L, Kbits, float(scale), float(eps), rep, kinds[0][0], kinds[1][0], q.dtype, k.dtype, v.dtype)
-        return _activations(out, B, q.dtype)
+        return _activations(out, B, q.dtype).detach()  # (no view, as attention._out_rows)
 
     @staticmethod
     def backward(ctx, grad):

@@ -154,7 +154,7 @@ class RaceLayerFn(Function):
         out = race_fused_fwd(pK, pQ, V2, eps, 0, state=state)
         ctx.save_for_backward(Qc, Kc, planes, pK, pQ, V2, state)
         ctx.cfg = (L, Kbits, float(scale), float(eps), codes, V.dtype)
-        return out.view(B, H, T, D)
+        return out.view(B, H, T, D).detach()  # (no view, as attention._out_rows)
 
     @staticmethod
     def backward(ctx, grad_out):

@@ -72,3 +72,29 @@ def test_attend_fp32_equals_the_composed_ops(dev, dtype, Hq, Hkv, packed):
             ulp = torch.finfo(dtype).eps  # the spacing of a value's binade, of the value at most
             over = ((a.float() - b.float()).abs() - ulp * b.float().abs() - 1e-5 * b.float().abs().max()).max().item()
             assert over <= 0, (i, over)
+
+
+@pytest.mark.parametrize("call", ["attend_bf16", "attend_fp32", "attend_fp32_f32_rows", "module_fp32"])
+@pytest.mark.parametrize("H", [1, 2])
+def test_outputs_change_in_place(dev, call, H):
+    """The outputs are no views of a Function's internals: a caller may scale or gate them in place."""
+    from race_attention_amd import RaceCausalCuda, build_planes_protos
+    from race_attention_amd.nanochat import race_attend
+    B, T, D, L, K = 1, 40, 64, 2, 3
+    planes, protos = build_planes_protos(D, K, L, 1, device=dev, seed=0)
+    mod = RaceCausalCuda(D, K, L, 1, device=dev, seed=0)
+    dtype = torch.bfloat16 if call in ("attend_bf16", "attend_fp32") else torch.float32
+    g = torch.Generator().manual_seed(1)
+    rows = [torch.randn(B, T, H, D, generator=g).to(dtype).to(dev) for _ in range(3)]
+
+    def grads(gate):
+        x = [r.clone().requires_grad_(True) for r in rows]
+        if call == "module_fp32":
+            y = mod(*(t.transpose(1, 2) for t in x))
+        else:
+            y = race_attend(*x, planes, L, K, EPS, precision="bf16" if call == "attend_bf16" else "fp32", protos_T=protos)
+        y = gate(y)
+        return (y, *torch.autograd.grad(y, x, torch.ones_like(y)))
+
+    for a, b in zip(grads(lambda y: y.mul_(2)), grads(lambda y: y * 2)):
+        assert torch.equal(a, b)
