@@ -47,10 +47,12 @@ class RaceDecodeState:
         The state must be fresh (prefill starts from zero)."""
         if self.tokens:
             raise RuntimeError("prefill on a non-empty state; call reset() first")
-        if k.shape[:2] != (self.B, self.Hkv) or k.shape[3] != self.D:
-            raise ValueError(f"prefill expects k/v [{self.B},{self.Hkv},T,{self.D}], got {tuple(k.shape)}")
-        out, _, _ = race_causal_attention_with_state(q, k, v, self.planes, self.L, self.K, self.scale, self.eps,
-                                                     out_dtype, (self.A, self.Bs), bthd)
+        own = (self.A, self.Bs) if q.shape[0] * k.shape[1] == self.B * self.Hkv and q.shape[3] == self.D else None
+        out, A, Bs = race_causal_attention_with_state(q, k, v, self.planes, self.L, self.K, self.scale, self.eps,
+                                                      out_dtype, own, bthd)
+        if own is None:  # one stream's prompt for all sequences (any other size is refused here)
+            self.A.copy_(A)
+            self.Bs.copy_(Bs)
         self.tokens = q.shape[2]
         return out
 

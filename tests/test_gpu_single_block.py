@@ -64,3 +64,23 @@ def test_prefill_many_streams_leaves_the_state_in_place(dev):
         assert st.tokens == T
     with pytest.raises(ValueError):
         RaceDecodeState(B // 2, Hq, Hkv, D, L, K, planes, device=dev).prefill(q, k, v)
+
+
+@pytest.mark.parametrize("T", [20, 3000])
+def test_prefill_forms(dev, T):
+    """One stream's prompt prefills the state of every sequence, and rows of k and v behind the prompt are
+    not read; a prompt of another number of streams, or with rows missing, is refused."""
+    from race_attention_amd import RaceDecodeState, build_planes_protos, race_causal_attention_with_state
+    D, L, K, B, G = 64, 8, 4, 5, 4
+    g = torch.Generator().manual_seed(T)
+    q, k, v = (torch.randn(1, h, T + 7, D, generator=g).to(torch.bfloat16).to(dev) for h in (G, 1, 1))
+    planes, _ = build_planes_protos(D, K, L, 1, device=dev, seed=2)
+    out, A, Bs = race_causal_attention_with_state(q[:, :, :T], k[:, :, :T], v[:, :, :T], planes, L, K, eps=EPS)
+    st = RaceDecodeState(B, G, 1, D, L, K, planes, eps=EPS, device=dev)
+    assert torch.equal(st.prefill(q[:, :, :T], k, v), out)
+    assert st.tokens == T and torch.equal(st.A, A.expand_as(st.A)) and torch.equal(st.Bs, Bs.expand_as(st.Bs))
+    two = [x.expand(2, -1, -1, -1) for x in (q, k, v)]
+    with pytest.raises(RuntimeError):
+        RaceDecodeState(B, G, 1, D, L, K, planes, eps=EPS, device=dev).prefill(*two)
+    with pytest.raises(ValueError):
+        race_causal_attention_with_state(q, k[:, :, :T], v, planes, L, K, eps=EPS)
