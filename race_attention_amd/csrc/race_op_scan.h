@@ -266,6 +266,10 @@ struct GroupSums {
     RACE_DEV float after(int g) const { return (g & 1 ? 0.0f : near) + (g & 2 ? 0.0f : far); }
 };
 
+// eps of bucket col: 1 for the padding, whose A is zero (eps = 0 is taken, and 0 / 0 of a padding bucket
+// would reach every output)
+RACE_DEV float op_eps(const ScanParams &P, const OpCtx &c, int col) { return col < c.S_here ? P.eps : 1.0f; }
+
 // inv = 1 / (A + eps) of a sub-chunk tile of pK; a0 (A before the sub-chunk) moves past it
 RACE_DEV f32x4 op_inv_a(const f32x4 &pk, float &a0, float eps, int g)
 {
@@ -483,6 +487,7 @@ __global__ __launch_bounds__(ST * 4) __attribute__((amdgpu_waves_per_eu(op_waves
     Suffix Tt[NTD] = {};
     op_ld_state<NTD>(St, P.wsB + (c.slot * P.S_pad + c.s0) * P.DPw, P.DPw, c);
     float a0 = LIN ? 0.0f : P.wsA[c.slot * P.S_pad + c.s0 + col];
+    const float eps = op_eps(P, c, col);
     double ga = 0.0;
     RS rs;
     auto fetch = [&](int t0) {
@@ -520,7 +525,7 @@ __global__ __launch_bounds__(ST * 4) __attribute__((amdgpu_waves_per_eu(op_waves
         for (int s = 0; s < NSUB; ++s) {
             f32x4 inv = {1.f, 1.f, 1.f, 1.f};
             if constexpr (!LIN)
-                inv = op_inv_a(k_[s], a0, P.eps, c.g);
+                inv = op_inv_a(k_[s], a0, eps, c.g);
             const f32x4 w = LIN ? q_[s] : q_[s] * inv;
             f32x4 acc = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
@@ -584,6 +589,7 @@ RACE_DEV void op_gk(const ScanParams &P, const OpCtx &c, OpGkLds<ST, DP> &lds)
     for (int k = 0; k < NTD; ++k)
         dS[k].load(P.ws2B, P.ws3B, row * P.DPw + k * 16 + 4 * c.g, 1);
     double ga = LIN ? 0.0 : (double)P.ws2A[row] + (double)P.ws3A[row];
+    const float eps = op_eps(P, c, col);
     float a_next = 0.0f;
     RS rs;
     const int nst = (c.t_end - c.t_begin + TS - 1) / TS;
@@ -618,7 +624,7 @@ RACE_DEV void op_gk(const ScanParams &P, const OpCtx &c, OpGkLds<ST, DP> &lds)
         for (int s = 0; s < NSUB; ++s) {
             w[s] = pq[s];
             if constexpr (!LIN) {
-                w[s] *= op_inv_a(pk[s], a0, P.eps, c.g);
+                w[s] *= op_inv_a(pk[s], a0, eps, c.g);
                 gA[s] = -gq[s] * w[s];
             }
         }
@@ -802,7 +808,7 @@ RACE_DEV void op_value(const ScanParams &P, const OpCtx &c, OpValueLds<ST, DP> &
                     for (int r = 0; r < 4; ++r)
 #pragma unroll
                         for (int e = 0; e < 4; ++e)
-                            w[r][e] *= frcp(base[e] + p[r][e] + P.eps);
+                            w[r][e] *= frcp(base[e] + p[r][e] + op_eps(P, c, VEC ? col : col + e));
                     if constexpr (!REV) {
 #pragma unroll
                         for (int e = 0; e < 4; ++e)

@@ -17,10 +17,6 @@ static hipError_t launch_v(OpKernel k, const ScanParams &P, dim3 grid, hipStream
     // the bucket kernels of a 128-bucket tile run as two workgroups of 64 buckets: V and gO are
     // read twice, but two or three independent workgroups share a CU instead of one (before the
     // suffixes moved to fp64, 200003 tokens x 4 streams, S = 128, D = 64: gq 565 -> 535, gk 521 ->
-    // 508 us; 32 buckets: 785 and 560)
-    // the bucket kernels of a 128-bucket tile run as two workgroups of 64 buckets: V and gO are
-    // read twice, but two or three independent workgroups share a CU instead of one (before the
-    // suffixes moved to fp64, 200003 tokens x 4 streams, S = 128, D = 64: gq 565 -> 535, gk 521 ->
     // 508 us; 32 buckets: 785 and 560). Side by side (op_place) against one half of the buckets
     // after the other: totals 182 -> 176, gq 623 -> 615, gk 527 -> 506
     constexpr int BT = ST < 64 ? ST : 64, NWG = ST / BT;

@@ -100,3 +100,17 @@ def test_values_beyond_a_block_do_not_leak(dev):
     out = race_fused_fwd(pk, pq, v, EPS, 48)
     assert torch.equal(out[0, :48], clean[0, :48])
     assert not torch.isfinite(out[0, 48:]).any()
+
+
+@pytest.mark.parametrize("T,S,D", [(50, 24, 64), (200, 192, 64), (70, 129, 128), (40, 15, 33)])
+def test_eps_zero_with_padding_buckets(dev, T, S, D):
+    """eps = 0 is taken: the padding buckets of a tile, whose mass is zero, reach no output."""
+    from race_attention_amd.race_causal_cuda import race_backward, race_fused_fwd
+    pk, pq, v, go = probs(2, T, S, D, seed=T + S + D)
+    out_t, gpk_t, gpq_t, gv_t, _, _ = oracle_op(pk, pq, v, go, 0.0)
+    pkc, pqc, vc, goc = (x.float().to(dev) for x in (pk, pq, v, go))
+    check("out", race_fused_fwd(pkc, pqc, vc, 0.0, 0), out_t, 2e-5)
+    floors = fp32_formula_floor(pk, pq, v, go, 0.0, (gpk_t, gpq_t, gv_t))
+    for name, g, ref, f in zip(("gpK", "gpQ", "gV"), race_backward(pkc, pqc, vc, goc, 0.0, 0),
+                               (gpk_t, gpq_t, gv_t), floors):
+        check(name, g, ref, max(1e-4, 2.0 * f))
