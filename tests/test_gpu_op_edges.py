@@ -114,3 +114,16 @@ def test_eps_zero_with_padding_buckets(dev, T, S, D):
     for name, g, ref, f in zip(("gpK", "gpQ", "gV"), race_backward(pkc, pqc, vc, goc, 0.0, 0),
                                (gpk_t, gpq_t, gv_t), floors):
         check(name, g, ref, max(1e-4, 2.0 * f))
+
+
+@pytest.mark.parametrize("pitch", [1 << 22, (1 << 22) + 4])
+def test_value_row_pitch(dev, pitch):
+    """Both sides of the row pitch up to which the totals move V in range-checked runs."""
+    from race_attention_amd.noncausal import BatchedACE
+    T, D = 40, 64
+    ace = BatchedACE(D, 3, 3, 1, device=dev, share_planes=True)
+    g = torch.Generator().manual_seed(0)
+    k, v, q = (torch.randn(1, 1, T, 1, D, generator=g).to(dev) for _ in range(3))
+    wide = torch.full((1, 1, T, 1, pitch), float("nan"), device=dev)
+    wide[..., :D] = v
+    assert torch.equal(ace(k, wide[..., :D], q, EPS), ace(k, v, q, EPS))
