@@ -47,10 +47,13 @@ class RaceDecodeState:
         The state must be fresh (prefill starts from zero)."""
         if self.tokens:
             raise RuntimeError("prefill on a non-empty state; call reset() first")
-        own = (self.A, self.Bs) if q.shape[0] * k.shape[1] == self.B * self.Hkv and q.shape[3] == self.D else None
+        streams = q.shape[0] * k.shape[1]
+        if q.shape[3] != self.D or streams not in (1, self.B * self.Hkv):
+            raise ValueError(f"prefill expects k/v [{self.B},{self.Hkv},T,{self.D}], got {tuple(k.shape)}")
+        own = (self.A, self.Bs) if streams == self.B * self.Hkv else None
         out, A, Bs = race_causal_attention_with_state(q, k, v, self.planes, self.L, self.K, self.scale, self.eps,
                                                       out_dtype, own, bthd)
-        if own is None:  # one stream's prompt for all sequences (any other size is refused here)
+        if own is None:  # one stream's prompt for all sequences
             self.A.copy_(A)
             self.Bs.copy_(Bs)
         self.tokens = q.shape[2]

@@ -80,7 +80,7 @@ def test_prefill_forms(dev, T):
     assert torch.equal(st.prefill(q[:, :, :T], k, v), out)
     assert st.tokens == T and torch.equal(st.A, A.expand_as(st.A)) and torch.equal(st.Bs, Bs.expand_as(st.Bs))
     two = [x.expand(2, -1, -1, -1) for x in (q, k, v)]
-    with pytest.raises(RuntimeError):
+    with pytest.raises(ValueError):
         RaceDecodeState(B, G, 1, D, L, K, planes, eps=EPS, device=dev).prefill(*two)
     with pytest.raises(ValueError):
         race_causal_attention_with_state(q, k[:, :, :T], v, planes, L, K, eps=EPS)
