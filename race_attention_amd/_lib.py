@@ -95,6 +95,11 @@ SIGNATURES = {
                                         ctypes.c_size_t, _vp, ctypes.c_size_t, _vp]),
     "race_op_bwd_kept": (ctypes.c_int, [_vp, _vp, _vp, _vp, _vp, _vp, _vp, _i64, _i64, _i64, _i64, ctypes.c_float,
                                         _i64, _vp, ctypes.c_size_t, _vp, ctypes.c_size_t, _vp]),
+    "race_op_fwd_bf16_rows": (ctypes.c_int, [_vp, _vp, Tensor4, Tensor4, _i64, _i64, _i64, _i64, _i64, ctypes.c_float,
+                                             _i64, _vp, ctypes.c_size_t, _vp, ctypes.c_size_t, _vp]),
+    "race_op_bwd_bf16_rows": (ctypes.c_int, [_vp, _vp, Tensor4, Tensor4, _vp, _vp, Tensor4, _i64, _i64, _i64, _i64,
+                                             _i64, ctypes.c_float, _i64, _vp, ctypes.c_size_t, _vp, ctypes.c_size_t,
+                                             _vp]),
     "race_qkv_state_bytes": (ctypes.c_size_t, [ctypes.POINTER(QKVShape)]),
     "race_qkv_scratch_bytes": (ctypes.c_size_t, [ctypes.POINTER(QKVShape), ctypes.c_int]),
     "race_qkv_fwd": (ctypes.c_int, [ctypes.POINTER(QKVShape), Tensor4, Tensor4, Tensor4, _vp, Tensor4,

@@ -468,13 +468,13 @@ static int run_scan_op(OpKernel k, const Geo &g, const ScanParams &P, hipStream_
     return hip_check(launch_scan_op(k, g.ST, g.DP, P, grid, s), "race_op kernel launch");
 }
 
-// rows move as 16-byte range-checked runs where every row of the operands starts 16-byte aligned, no rows
+// fp32 rows move as 16-byte range-checked runs where every row of the operands starts 16-byte aligned, no rows
 // overlap (the range ends behind a stage's last row) and a stage of 64 rows stays below the 2^31 bytes
 // that an offset covers
 static void op_vec(ScanParams &P)
 {
     const auto apart = [&](const View &x) { return x.st >= P.D && x.st <= (1 << 22); };
-    P.vec = P.S % 4 == 0 && P.D % 4 == 0 && aligned16(P.pK) && aligned16(P.pQ) && aligned16(P.V) && aligned16(P.gO) &&
+    P.rows = P.S % 4 == 0 && P.D % 4 == 0 && aligned16(P.pK) && aligned16(P.pQ) && aligned16(P.V) && aligned16(P.gO) &&
             !((P.v.sb | P.v.sh | P.v.st | P.go.sb | P.go.sh | P.go.st) & 3) && apart(P.v) && apart(P.go);
 }
 
@@ -513,9 +513,47 @@ static void state_views(const Geo &g, const float *state, float *&wsB, float *&w
     wsA = wsB + align256(g.state_elems_B * 4) / 4;
 }
 
+// bf16 rows through views ([B][H][T][D], stream z = b * H + h): 8-byte runs, one bucket tile
+struct OpBf16Rows {
+    race_tensor V, go, out;  // go: the backward's upstream gradient, out: the output or gV
+    int64_t H;
+};
+
+static int op_bf16_check(const OpBf16Rows &r, const race_tensor *go, int64_t B, int64_t T, int64_t S, int64_t D,
+                         const float *pK, const float *pQ, const char *who)
+{
+    if (B <= 0 || r.H <= 0 || B > (1 << 30) || r.H > (1 << 30))
+        return fail(RACE_ERR_INVALID, "%s: B and H must be positive", who);
+    if (S > 128 || S % 4 || D % 4 || !aligned16(pK) || !aligned16(pQ))
+        return fail(RACE_ERR_UNSUPPORTED, "%s: bf16 rows need S <= 128, S %% 4 == 0, D %% 4 == 0 and 16-byte aligned "
+                    "probabilities", who);
+    for (const race_tensor *t : {&r.V, go, &r.out}) {
+        if (!t)
+            continue;
+        RACE_TRY(check_view(*t, who, false));
+        if ((reinterpret_cast<uintptr_t>(t->data) & 7) || ((t->stride_b | t->stride_h | t->stride_t) & 3) ||
+            t->stride_t < D || t->stride_t > (1 << 22))
+            return fail(RACE_ERR_UNSUPPORTED, "%s: bf16 rows must start 8-byte aligned, at least D and at most 2^22 "
+                        "elements apart", who);
+    }
+    if ((r.out.stride_h < D && r.H > 1) || (r.out.stride_b < D && B > 1))
+        return fail(RACE_ERR_INVALID, "%s: the streams of the result share rows", who);
+    return RACE_OK;
+}
+
+static void op_bf16_params(ScanParams &P, const OpBf16Rows &r, OutView &result)
+{
+    P.rows = 2;  // (ROWS_BF16)
+    P.zH = (int)r.H;
+    P.v = to_view(r.V);
+    P.go = to_view(r.go);
+    result = to_out(r.out, 0);
+}
+
 static int op_fwd_impl(const float *pK, const float *pQ, const float *V, float *out, int64_t N, int64_t T,
                        int64_t S, int64_t D, float eps, int64_t block, void *workspace, size_t workspace_bytes,
-                       race_stream stream, int linear, const char *who, float *state = nullptr)
+                       race_stream stream, int linear, const char *who, float *state = nullptr,
+                       const OpBf16Rows *bf16 = nullptr)
 {
     Geo g;
     RACE_TRY(op_geometry(N, T, S, D, block, g));
@@ -535,6 +573,8 @@ static int op_fwd_impl(const float *pK, const float *pQ, const float *V, float *
     float *part = g.n_st > 1 ? cv.take((size_t)g.n_st * N * T * D) : nullptr;
     P.out = part ? OutView{part, T * D, 0, D, N * T * D, 1} : OutView{out, T * D, 0, D, 0, 1};
     op_vec(P);
+    if (bf16)
+        op_bf16_params(P, *bf16, P.out);
     const hipStream_t s = hs(stream);
     RACE_TRY(run_scan_op(OP_TOTALS, g, P, s));
     RACE_TRY(hip_check(prof_block_scan(P.wsB, (int64_t)g.S_pad * g.DP, P.wsA, g.S_pad, (int)g.NB, (int)g.Z, 0, s), "block scan"));
@@ -556,7 +596,7 @@ int race_op_fwd(const float *pK, const float *pQ, const float *V, float *out, in
 static int op_bwd_impl(const float *pK, const float *pQ, const float *V, const float *gO, float *gpK, float *gpQ,
                        float *gV, int64_t N, int64_t T, int64_t S, int64_t D, float eps, int64_t block,
                        void *workspace, size_t workspace_bytes, race_stream stream, int linear, const char *who,
-                       const float *state = nullptr)
+                       const float *state = nullptr, const OpBf16Rows *bf16 = nullptr)
 {
     Geo g;
     RACE_TRY(op_geometry(N, T, S, D, block, g));
@@ -583,6 +623,8 @@ static int op_bwd_impl(const float *pK, const float *pQ, const float *V, const f
     float *part = g.n_st > 1 ? cv.take((size_t)g.n_st * N * T * D) : nullptr;
     P.dv = part ? OutView{part, T * D, 0, D, N * T * D, 1} : OutView{gV, T * D, 0, D, 0, 1};
     op_vec(P);
+    if (bf16)
+        op_bf16_params(P, *bf16, P.dv);
     const hipStream_t s = hs(stream);
     if (state) {  // forward block states kept by race_op_fwd_keep (only read from here on)
         state_views(g, state, P.wsB, P.wsA);
@@ -627,6 +669,32 @@ int race_op_bwd_kept(const float *pK, const float *pQ, const float *V, const flo
     RACE_TRY(kept_state_check(state, state_bytes, N, T, S, D, block, "race_op_bwd_kept"));
     return op_bwd_impl(pK, pQ, V, gO, gpK, gpQ, gV, N, T, S, D, eps, block, workspace, workspace_bytes, stream, 0,
                        "race_op_bwd_kept", state);
+}
+
+int race_op_fwd_bf16_rows(const float *pK, const float *pQ, race_tensor V, race_tensor out, int64_t B, int64_t H,
+                          int64_t T, int64_t S, int64_t D, float eps, int64_t block, void *workspace,
+                          size_t workspace_bytes, float *state, size_t state_bytes, race_stream stream)
+{
+    const char *who = "race_op_fwd_bf16_rows";
+    const OpBf16Rows rows{V, V, out, H};
+    RACE_TRY(op_bf16_check(rows, nullptr, B, T, S, D, pK, pQ, who));
+    RACE_TRY(kept_state_check(state, state_bytes, B * H, T, S, D, block, who));
+    return op_fwd_impl(pK, pQ, static_cast<const float *>(V.data), static_cast<float *>(out.data), B * H, T, S, D, eps,
+                       block, workspace, workspace_bytes, stream, 0, who, state, &rows);
+}
+
+int race_op_bwd_bf16_rows(const float *pK, const float *pQ, race_tensor V, race_tensor gO, float *gpK, float *gpQ,
+                          race_tensor gV, int64_t B, int64_t H, int64_t T, int64_t S, int64_t D, float eps,
+                          int64_t block, void *workspace, size_t workspace_bytes, const float *state,
+                          size_t state_bytes, race_stream stream)
+{
+    const char *who = "race_op_bwd_bf16_rows";
+    const OpBf16Rows rows{V, gO, gV, H};
+    RACE_TRY(op_bf16_check(rows, &gO, B, T, S, D, pK, pQ, who));
+    RACE_TRY(kept_state_check(state, state_bytes, B * H, T, S, D, block, who));
+    return op_bwd_impl(pK, pQ, static_cast<const float *>(V.data), static_cast<const float *>(gO.data), gpK, gpQ,
+                       static_cast<float *>(gV.data), B * H, T, S, D, eps, block, workspace, workspace_bytes, stream, 0,
+                       who, state, &rows);
 }
 
 int race_op_bwd(const float *pK, const float *pQ, const float *V, const float *gO, float *gpK, float *gpQ,

@@ -34,6 +34,13 @@
 
 namespace race {
 
+// How the rows of V, gO, out and gV lie (ScanParams::rows): fp32 rows of any alignment; fp32 rows that
+// move as 16-byte runs; bf16 rows that move as 8-byte runs, out and gV rounded to bf16 as they are
+// stored. The last are the activations of a bf16 model in their own layout: products, states and
+// sums stay fp32 and the results are those of fp32 copies to the bit, but no pass casts and transposes
+// V, gO, out and gV (16 x 2047 tokens, 6 heads of 128, S = 24: forward and backward 675 -> 529 us)
+enum { ROWS_ANY = 0, ROWS_F32 = 1, ROWS_BF16 = 2 };
+
 // tokens per stage of the bucket kernels (also the spacing of the A checkpoints): as many as leave
 // two workgroups' V and go tiles room in LDS (32 tokens at D = 128, S = 32: gq 106 against 100, gk 84
 // against 79 us at 32752 tokens x 6 streams)
@@ -72,13 +79,13 @@ RACE_DEV void st4(float *p, const f32x4 &v) { *reinterpret_cast<f32x4 *>(p) = v;
 // lane without a column takes the offset OP_OOB; addresses are one 32-bit add per access.
 typedef __amdgpu_buffer_rsrc_t OpBuf;
 constexpr uint32_t OP_OOB = 0x80000000u;
-RACE_DEV OpBuf op_buf(const float *p, int64_t floats)
+RACE_DEV OpBuf op_buf(const void *p, int64_t floats, int bytes = 4)
 {
     // (the same in every lane: stated, so that no loop over the lanes' descriptors is made of it)
     const uint64_t a = reinterpret_cast<uint64_t>(p);
     const uint32_t lo = __builtin_amdgcn_readfirstlane((int)a), hi = __builtin_amdgcn_readfirstlane((int)(a >> 32));
     return __builtin_amdgcn_make_buffer_rsrc(reinterpret_cast<void *>((uint64_t)hi << 32 | lo), 0,
-                                             __builtin_amdgcn_readfirstlane((int)(floats * 4)), 0x00027000);
+                                             __builtin_amdgcn_readfirstlane((int)(floats * bytes)), 0x00027000);
 }
 RACE_DEV float buf_ld(OpBuf b, uint32_t off)
 {
@@ -87,6 +94,22 @@ RACE_DEV float buf_ld(OpBuf b, uint32_t off)
 RACE_DEV f32x4 buf_ld4(OpBuf b, uint32_t off)
 {
     return __builtin_bit_cast(f32x4, __builtin_amdgcn_raw_buffer_load_b128(b, off, 0, 0));
+}
+RACE_DEV u32x2 buf_ld2(OpBuf b, uint32_t off)
+{
+    return __builtin_bit_cast(u32x2, __builtin_amdgcn_raw_buffer_load_b64(b, off, 0, 0));
+}
+// fp32 of what a load left: fp32, pairs of bf16, or a bf16 in each low half
+RACE_DEV f32x4 op_widen(const f32x4 &v) { return v; }
+RACE_DEV f32x4 op_widen(const u32x2 &v)
+{
+    return __builtin_bit_cast(f32x4, u32x4{v[0] << 16, v[0] & 0xffff0000u, v[1] << 16, v[1] & 0xffff0000u});
+}
+RACE_DEV f32x4 op_widen(const u32x4 &v) { return __builtin_bit_cast(f32x4, v << 16); }
+RACE_DEV uint32_t buf_ld_h(OpBuf b, uint32_t off) { return __builtin_amdgcn_raw_buffer_load_b16(b, off, 0, 0); }
+RACE_DEV void buf_st_h(OpBuf b, uint32_t off, float v)
+{
+    __builtin_amdgcn_raw_buffer_store_b16(__builtin_bit_cast(unsigned short, (__bf16)v), b, off, 0, 0);
 }
 RACE_DEV void buf_st(OpBuf b, uint32_t off, float v)
 {
@@ -144,28 +167,37 @@ RACE_DEV void op_place(const ScanParams &P, int &blk, int &w)
 
 // Rows of V (and go) of one stage into LDS, row-major [TS][DP + 8] and / or transposed
 // [DP][TS + 8]. A thread moves 4 rows x 4 columns, so both layouts are written as 16-byte runs.
-// Rows beyond the stage and columns >= D read as zeros. VEC: rows move as 16-byte runs (compiled apart: a branch between the two forms of
+// Rows beyond the stage and columns >= D read as zeros. bf16 rows wait as they are and are widened on
+// their way into LDS. The kinds of rows are compiled apart (: a branch between the two forms of
 // a load makes the compiler wait for it on the spot, 278 -> 200 us for the block totals of 200003
 // tokens x 4 streams, S = 128, D = 64). Up to 4 items per thread wait in registers, fetched a stage ahead; more
 // (few waves, wide rows) are moved when the stage begins.
-template <int TS, int DP, int NTH, int NT, bool VEC>
+template <int TS, int DP, int NTH, int NT, int ROWS>
 struct RowStage {
     static constexpr int CH = DP / 4, IT = (TS / 4) * CH, N = (NT * IT + NTH - 1) / NTH;
     static constexpr bool AHEAD = N <= 4;
     static constexpr int LDX = op_pitch(DP), LDT = op_pitch(TS);
     static_assert(IT % 64 == 0, "one tensor per wave and item");
-    f32x4 x[AHEAD ? N : 1][4];
+    typedef typename std::conditional<ROWS == ROWS_BF16, u32x2, f32x4>::type Raw;
+    Raw x[AHEAD ? N : 1][4];
 
-    struct Src {
+    struct Src {  // (p: the address of the stream's first row, whatever its elements)
         const float *p;
         int64_t st;
     };
 
     // item i, rows t0 .. of which nv belong to the stage
-    static RACE_DEV void load(f32x4 (&v)[4], const Src &s, int i, int t0, int nv, int D)
+    static RACE_DEV void load(Raw (&v)[4], const Src &s, int i, int t0, int nv, int D)
     {
         const int r = (i % IT) / CH * 4, c = (i % IT) % CH * 4;
-        if constexpr (VEC) {
+        if constexpr (ROWS == ROWS_BF16) {
+            const OpBuf b = op_buf(reinterpret_cast<const __bf16 *>(s.p) + (int64_t)t0 * s.st,
+                                   nv > 0 ? (int64_t)(nv - 1) * s.st + D : 0, 2);
+            const uint32_t st = (uint32_t)s.st * 2, off = c < D ? r * st + c * 2 : OP_OOB;
+#pragma unroll
+            for (int j = 0; j < 4; ++j)
+                v[j] = buf_ld2(b, off + j * st);
+        } else if constexpr (ROWS == ROWS_F32) {
             const OpBuf b = op_buf(s.p + (int64_t)t0 * s.st, nv > 0 ? (int64_t)(nv - 1) * s.st + D : 0);
             const uint32_t st = (uint32_t)s.st * 4, off = c < D ? r * st + c * 4 : OP_OOB;
 #pragma unroll
@@ -182,9 +214,10 @@ struct RowStage {
         }
     }
 
-    static RACE_DEV void store(const f32x4 (&v)[4], float *rm, float *tr, int i)
+    static RACE_DEV void store(const Raw (&raw)[4], float *rm, float *tr, int i)
     {
         const int r = (i % IT) / CH * 4, c = (i % IT) % CH * 4;
+        const f32x4 v[4] = {op_widen(raw[0]), op_widen(raw[1]), op_widen(raw[2]), op_widen(raw[3])};
         if (rm) {
 #pragma unroll
             for (int j = 0; j < 4; ++j)
@@ -335,10 +368,18 @@ constexpr int op_shares(int NW, int NSUB, int ksteps)
     return ks;
 }
 
-template <class RS>
+template <int ROWS>
+RACE_DEV const float *op_first_row(const float *p, const View &v, int zH, int z)
+{
+    if constexpr (ROWS == ROWS_BF16)
+        return reinterpret_cast<const float *>(reinterpret_cast<const __bf16 *>(p) + op_row_offset(v.sb, v.sh, zH, z));
+    else
+        return op_rows(p, v, zH, z);
+}
+template <class RS, int ROWS>
 RACE_DEV typename RS::Src op_src(const float *p, const View &v, int zH, int z)
 {
-    return typename RS::Src{op_rows(p, v, zH, z), v.st};
+    return typename RS::Src{op_first_row<ROWS>(p, v, zH, z), v.st};
 }
 
 // state tiles St^T[d][s] <-> workspace [s][DPw]: a lane owns 4 consecutive d of its bucket
@@ -406,19 +447,19 @@ RACE_DEV void put_hilo(float *hi, float *lo, int64_t o, double v)
 
 // ============================================================================ block totals
 // sum pK^T v and sum pK of each block -> workspace slot blk
-template <int ST, int DP, int NWG, bool VEC>
+template <int ST, int DP, int NWG, int ROWS>
 __global__ __launch_bounds__(ST * 4) void race_op_totals(const ScanParams P)
 {
     using CF = OpCfg<ST, DP>;
     constexpr int NTD = CF::NTD, NTH = ST * 4, TS = CF::TS, NSUB = TS / 16;
-    using RS = RowStage<TS, DP, NTH, 1, VEC>;
+    using RS = RowStage<TS, DP, NTH, 1, ROWS>;
     __shared__ __align__(16) float sVt[DP * RS::LDT];
     int blk, wg;
     op_place<NWG>(P, blk, wg);
     const OpCtx c = op_ctx<ST>(P, blk, blockIdx.y * NWG + wg);
     const int col = c.wave * 16 + c.n;
     const uint32_t S4 = P.S * 4, off = col < c.S_here ? 4 * c.g * S4 + (c.s0 + col) * 4 : OP_OOB;
-    const typename RS::Src src = op_src<RS>(P.V, P.v, P.zH, c.z);
+    const typename RS::Src src = op_src<RS, ROWS>(P.V, P.v, P.zH, c.z);
     const float *pK = P.pK + (int64_t)c.z * P.T * P.S;
 
     f32x4 St[NTD], pk[NSUB];
@@ -463,13 +504,13 @@ __global__ __launch_bounds__(ST * 4) void race_op_totals(const ScanParams P)
 // ============================================================================ gpQ and suffix totals
 // Forward walk: gW = go St^T + tril(go V^T) pK, gpQ = gW / (A + eps), the block totals of W^T go
 // and gA = -gpQ W, and A at every stage start for the reverse walks.
-template <int ST, int DP, int NWG, bool LIN, bool VEC>
+template <int ST, int DP, int NWG, bool LIN, int ROWS>
 __global__ __launch_bounds__(ST * 4) __attribute__((amdgpu_waves_per_eu(op_waves_gq(ST, DP)))) void race_op_gq(const ScanParams P)
 {
     using CF = OpCfg<ST, DP>;
     constexpr int NTD = CF::NTD, NW = ST / 16, NTH = ST * 4, TS = CF::TS, NSUB = TS / 16, LDM = 24;
     constexpr int KS = op_shares(NW, NSUB, DP / 16);
-    using RS = RowStage<TS, DP, NTH, 2, VEC>;
+    using RS = RowStage<TS, DP, NTH, 2, ROWS>;
     __shared__ __align__(16) float sV[TS * RS::LDX], sGO[TS * RS::LDX];
     __shared__ __align__(16) float sVt[DP * RS::LDT], sGOt[DP * RS::LDT];
     __shared__ __align__(16) float sM[KS * NSUB * 16 * LDM];
@@ -478,7 +519,7 @@ __global__ __launch_bounds__(ST * 4) __attribute__((amdgpu_waves_per_eu(op_waves
     const OpCtx c = op_ctx<ST>(P, blk, blockIdx.y * NWG + wg);
     const int col = c.wave * 16 + c.n;
     const uint32_t S4 = P.S * 4, off = col < c.S_here ? 4 * c.g * S4 + (c.s0 + col) * 4 : OP_OOB;
-    const typename RS::Src sv = op_src<RS>(P.V, P.v, P.zH, c.z), sg = op_src<RS>(P.gO, P.go, P.zH, c.z);
+    const typename RS::Src sv = op_src<RS, ROWS>(P.V, P.v, P.zH, c.z), sg = op_src<RS, ROWS>(P.gO, P.go, P.zH, c.z);
     const float *pK = P.pK + (int64_t)c.z * P.T * P.S, *pQ = P.pQ + (int64_t)c.z * P.T * P.S;
     float *gpQ = P.gpQ + (int64_t)c.z * P.T * P.S;
     float *ck = P.ckA + (((int64_t)c.z * P.NB + c.blk) * P.NCK) * P.S_pad + c.s0 + col;
@@ -568,17 +609,17 @@ struct OpGkLds {
     float V[TS * LDX], GO[TS * LDX], GOt[DP * LDT], M[KS * NSUB * 16 * LDM];
 };
 
-template <int ST, int DP, bool LIN, bool VEC>
+template <int ST, int DP, bool LIN, int ROWS>
 RACE_DEV void op_gk(const ScanParams &P, const OpCtx &c, OpGkLds<ST, DP> &lds)
 {
     using CF = OpCfg<ST, DP>;
     using LD = OpGkLds<ST, DP>;
     constexpr int NTD = CF::NTD, NW = LD::NW, NTH = ST * 4, TS = LD::TS, NSUB = LD::NSUB, LDM = LD::LDM, KS = LD::KS;
-    using RS = RowStage<TS, DP, NTH, 2, VEC>;
+    using RS = RowStage<TS, DP, NTH, 2, ROWS>;
     float *const sV = lds.V, *const sGO = lds.GO, *const sGOt = lds.GOt, *const sM = lds.M;
     const int col = c.wave * 16 + c.n;
     const uint32_t S4 = P.S * 4, off = col < c.S_here ? 4 * c.g * S4 + (c.s0 + col) * 4 : OP_OOB;
-    const typename RS::Src sv = op_src<RS>(P.V, P.v, P.zH, c.z), sg = op_src<RS>(P.gO, P.go, P.zH, c.z);
+    const typename RS::Src sv = op_src<RS, ROWS>(P.V, P.v, P.zH, c.z), sg = op_src<RS, ROWS>(P.gO, P.go, P.zH, c.z);
     const int64_t zoff = (int64_t)c.z * P.T * P.S;
     const float *ck = P.ckA + (((int64_t)c.z * P.NB + c.blk) * P.NCK) * P.S_pad + c.s0 + col;
 
@@ -661,13 +702,13 @@ RACE_DEV void op_gk(const ScanParams &P, const OpCtx &c, OpGkLds<ST, DP> &lds)
     }
 }
 
-template <int ST, int DP, int NWG, bool LIN, bool VEC>
+template <int ST, int DP, int NWG, bool LIN, int ROWS>
 __global__ __launch_bounds__(ST * 4) __attribute__((amdgpu_waves_per_eu(op_waves_gk(DP)))) void race_op_gk(const ScanParams P)
 {
     __shared__ __align__(16) OpGkLds<ST, DP> lds;
     int blk, wg;
     op_place<NWG>(P, blk, wg);
-    op_gk<ST, DP, LIN, VEC>(P, op_ctx<ST>(P, blk, blockIdx.y * NWG + wg), lds);
+    op_gk<ST, DP, LIN, ROWS>(P, op_ctx<ST>(P, blk, blockIdx.y * NWG + wg), lds);
 }
 
 // ============================================================================ readout / gv
@@ -683,7 +724,7 @@ struct OpValueLds {
     float Q[TS * LDS_], K[TS * LDS_], Kt[ST * LDT], M[KS * NSUB * 16 * LDM];
 };
 
-template <int ST, int DP, bool REV, bool LIN, bool VEC>
+template <int ST, int DP, bool REV, bool LIN, int ROWS>
 RACE_DEV void op_value(const ScanParams &P, const OpCtx &c, OpValueLds<ST, DP> &lds)
 {
     using CF = OpCfg<ST, DP>;
@@ -693,13 +734,15 @@ RACE_DEV void op_value(const ScanParams &P, const OpCtx &c, OpValueLds<ST, DP> &
     // W: a wave job covers CW buckets of the whole stage, lane (rg, lc): 4 tokens x 4 buckets
     constexpr int CW = 1024 / TS, NJ = ST / CW, JPW = (NJ + NW - 1) / NW, LC = CW / 4, RG = TS / 4;
     static_assert(NJ >= 1 && LC * RG == 64, "one job per 1024 probabilities");
+    constexpr bool VEC = ROWS != ROWS_ANY, BF = ROWS == ROWS_BF16;
     float *const sQ = lds.Q, *const sK = lds.K, *const sKt = lds.Kt, *const sM = lds.M;
     const int rg = c.lane / LC, lc = c.lane % LC;
     const int64_t zoff = (int64_t)c.z * P.T * P.S;
-    const float *xsrc = REV ? op_rows(P.gO, P.go, P.zH, c.z) : op_rows(P.V, P.v, P.zH, c.z);
+    const float *xsrc = REV ? op_first_row<ROWS>(P.gO, P.go, P.zH, c.z) : op_first_row<ROWS>(P.V, P.v, P.zH, c.z);
     const int64_t xst = REV ? P.go.st : P.v.st;
 
-    f32x4 xn[TD][NSUB], pk[JPW][4], pq[JPW][4], a0[JPW];
+    f32x4 pk[JPW][4], pq[JPW][4], a0[JPW];
+    typename std::conditional<BF, u32x4, f32x4>::type xn[TD][NSUB];  // (bf16 in the low halves)
     typename std::conditional<REV, Suffix, Prefix>::type St[TD][NTS];
     {
         const int64_t row = (REV ? c.slot + 1 : c.slot) * P.S_pad + c.s0 + 4 * c.g;
@@ -744,7 +787,16 @@ RACE_DEV void op_value(const ScanParams &P, const OpCtx &c, OpValueLds<ST, DP> &
 #pragma unroll
         for (int td = 0; td < TD; ++td) {
             const int d = (c.wave + td * NW) * 16 + c.n;
-            if constexpr (VEC) {
+            if constexpr (BF) {
+                const OpBuf bx = op_buf(reinterpret_cast<const __bf16 *>(xsrc) + (int64_t)t0 * xst,
+                                        nv > 0 ? (nv - 1) * xst + P.D : 0, 2);
+                const uint32_t st = (uint32_t)xst * 2, off = d < P.D ? 4 * c.g * st + d * 2 : OP_OOB;
+#pragma unroll
+                for (int s = 0; s < NSUB; ++s)
+#pragma unroll
+                    for (int e = 0; e < 4; ++e)
+                        xn[td][s][e] = buf_ld_h(bx, off + (s * 16 + e) * st);
+            } else if constexpr (VEC) {
                 const OpBuf bx = op_buf(xsrc + (int64_t)t0 * xst, nv > 0 ? (nv - 1) * xst + P.D : 0);
                 const uint32_t st = (uint32_t)xst * 4, off = d < P.D ? 4 * c.g * st + d * 4 : OP_OOB;
 #pragma unroll
@@ -831,15 +883,19 @@ RACE_DEV void op_value(const ScanParams &P, const OpCtx &c, OpValueLds<ST, DP> &
         for (int td = 0; td < TD; ++td)
 #pragma unroll
             for (int s = 0; s < NSUB; ++s)
-                x[td][s] = xn[td][s];
+                x[td][s] = op_widen(xn[td][s]);
         fetch(REV ? i - 1 : i + 1);
         __syncthreads();
         op_diag<NSUB, KS, NW, ST, LDS_, LDM>(sM, sQ, sK, REV, c);
         __syncthreads();
         const OutView &o = REV ? P.dv : P.out;
-        const OpBuf dst = op_buf(reinterpret_cast<const float *>(o.p) + (int64_t)blockIdx.y * o.tile + c.z * o.sb +
-                                     (int64_t)t0 * P.D,
-                                 (int64_t)nv * P.D);  // (rows of D floats)
+        // fp32: rows of D floats; bf16 (one bucket tile): rows through the view
+        const OpBuf dst = BF ? op_buf(reinterpret_cast<const __bf16 *>(o.p) + op_row_offset(o.sb, o.sh, P.zH, c.z) +
+                                          (int64_t)t0 * o.st,
+                                      (int64_t)(nv - 1) * o.st + P.D, 2)
+                             : op_buf(reinterpret_cast<const float *>(o.p) + (int64_t)blockIdx.y * o.tile +
+                                          c.z * o.sb + (int64_t)t0 * P.D,
+                                      (int64_t)nv * P.D);
 #pragma unroll
         for (int ss = 0; ss < NSUB; ++ss) {
             const int s = REV ? NSUB - 1 - ss : ss;
@@ -862,25 +918,32 @@ RACE_DEV void op_value(const ScanParams &P, const OpCtx &c, OpValueLds<ST, DP> &
             for (int td = 0; td < TD; ++td) {
                 mma4(acc[td], m, x[td][s]);
                 const int d = (c.wave + td * NW) * 16 + c.n;
-                const uint32_t st = P.D * 4;
-                op_store_tile(dst, d < P.D ? 4 * c.g * st + d * 4 : OP_OOB, st, s * 16, acc[td]);
+                const uint32_t st = BF ? (uint32_t)o.st * 2 : P.D * 4;
+                const uint32_t off = d < P.D ? 4 * c.g * st + d * (BF ? 2 : 4) : OP_OOB;
+                if constexpr (BF) {
+#pragma unroll
+                    for (int e = 0; e < 4; ++e)
+                        buf_st_h(dst, off + (s * 16 + e) * st, acc[td][e]);
+                } else {
+                    op_store_tile(dst, off, st, s * 16, acc[td]);
+                }
             }
         }
         __syncthreads();
     }
 }
 
-template <int ST, int DP, bool REV, bool LIN, bool VEC>
+template <int ST, int DP, bool REV, bool LIN, int ROWS>
 __global__ __launch_bounds__((OpCfg<ST, DP>::DW * 64)) __attribute__((amdgpu_waves_per_eu(op_waves_value(ST, DP)))) void race_op_out(const ScanParams P)
 {
     __shared__ __align__(16) OpValueLds<ST, DP> lds;
-    op_value<ST, DP, REV, LIN, VEC>(P, op_ctx<ST>(P, blockIdx.x, blockIdx.y), lds);
+    op_value<ST, DP, REV, LIN, ROWS>(P, op_ctx<ST>(P, blockIdx.x, blockIdx.y), lds);
 }
 
 // ============================================================================ gpK and gv in one launch
 // The gpK workgroups of a block (ST / BT of them) and its gv workgroup side by side: both walk the block
 // in reverse over the same pQ, go, pK and A checkpoints.
-template <int ST, int BT, int DP, bool LIN, bool VEC>
+template <int ST, int BT, int DP, bool LIN, int ROWS>
 __global__ __launch_bounds__(BT * 4) __attribute__((amdgpu_waves_per_eu(op_waves_value(ST, DP)))) void race_op_gkv(const ScanParams P)
 {
     static_assert(BT == OpCfg<ST, DP>::DW * 16, "one workgroup size");
@@ -889,9 +952,9 @@ __global__ __launch_bounds__(BT * 4) __attribute__((amdgpu_waves_per_eu(op_waves
     int blk, wg;
     op_place<NB_ + 1>(P, blk, wg);
     if (wg < NB_)
-        op_gk<BT, DP, LIN, VEC>(P, op_ctx<BT>(P, blk, blockIdx.y * NB_ + wg), lds.k);
+        op_gk<BT, DP, LIN, ROWS>(P, op_ctx<BT>(P, blk, blockIdx.y * NB_ + wg), lds.k);
     else
-        op_value<ST, DP, true, LIN, VEC>(P, op_ctx<ST>(P, blk, blockIdx.y), lds.v);
+        op_value<ST, DP, true, LIN, ROWS>(P, op_ctx<ST>(P, blk, blockIdx.y), lds.v);
 }
 
 }  // namespace race

@@ -42,7 +42,7 @@ struct ScanParams {
     View q, k, v, go;
     OutView out, dq, dk, dv;
     const float *planes;
-    // op path (fp32): probabilities [N][T][S], values/grads rows of D floats. Stream z reads its
+    // op path (fp32): probabilities [N][T][S], values/grads rows of D floats (or bf16: ScanParams::rows). Stream z reads its
     // V / gO rows as a [Z / zH][zH][T][D] view: row t of z at (z / zH) sb + (z % zH) sh + t st,
     // strides in v / go (their p unused); contiguous [N][T][D] is zH = 1, sb = T D, st = D
     const float *pK, *pQ, *V, *gO;
@@ -56,7 +56,7 @@ struct ScanParams {
     // op path, backward: A at every stage start of every block, [Z][NB][NCK][S_pad]
     float *ckA;
     int NCK;
-    int vec;  // op path: every row of the operands starts 16-byte aligned
+    int rows;  // op path: how the rows of V, gO, out and gV lie (ROWS_* of race_op_scan.h)
     // fused readout of a sequence that is one block: no totals pass and no block scan have run. The
     // state starts at zero, and its final value goes to finB / finA (rows s < finS of stream z at
     // z * finBz / z * finAz; DPw floats per row); with wsB, zeros go to block 0's prefix there.

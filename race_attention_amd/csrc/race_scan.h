@@ -125,9 +125,13 @@ RACE_DEV void load_rows_bf16(__bf16 *dst, __bf16 *dstT, const View &vw, int b, i
 }
 
 // op path: first row of stream z in a V / gO view (ScanParams::zH; zH <= 1: stream stride sb)
+RACE_DEV int64_t op_row_offset(int64_t sb, int64_t sh, int zH, int z)
+{
+    return zH <= 1 ? z * sb : (int64_t)(z / zH) * sb + (int64_t)(z % zH) * sh;
+}
 RACE_DEV const float *op_rows(const float *p, const View &v, int zH, int z)
 {
-    return zH <= 1 ? p + (int64_t)z * v.sb : p + (int64_t)(z / zH) * v.sb + (int64_t)(z % zH) * v.sh;
+    return p + op_row_offset(v.sb, v.sh, zH, z);
 }
 
 // ------------------------------------------------------------------ soft-hash pieces

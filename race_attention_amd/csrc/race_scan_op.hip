@@ -11,7 +11,7 @@ namespace race {
 template <int ST, int BT, int DP>
 constexpr bool op_one_launch = BT == 16 * OpCfg<ST, DP>::DW;
 
-template <int ST, int DP, bool VEC>
+template <int ST, int DP, int ROWS>
 static hipError_t launch_v(OpKernel k, const ScanParams &P, dim3 grid, hipStream_t s)
 {
     // the bucket kernels of a 128-bucket tile run as two workgroups of 64 buckets: V and gO are
@@ -19,38 +19,39 @@ static hipError_t launch_v(OpKernel k, const ScanParams &P, dim3 grid, hipStream
     // suffixes moved to fp64, 200003 tokens x 4 streams, S = 128, D = 64: gq 565 -> 535, gk 521 ->
     // 508 us; 32 buckets: 785 and 560). Side by side (op_place) against one half of the buckets
     // after the other: totals 182 -> 176, gq 623 -> 615, gk 527 -> 506
+    constexpr bool LIN = ROWS != ROWS_BF16;  // (bf16 rows: RACE only, the host asks for nothing else)
     constexpr int BT = ST < 64 ? ST : 64, NWG = ST / BT;
     const dim3 bucket(BT * 4), value(OpCfg<ST, DP>::DW * 64);
     const dim3 bgrid(grid.x * NWG, grid.y, grid.z);
     switch (k) {
     case OP_TOTALS:
-        hipLaunchKernelGGL((race_op_totals<BT, DP, NWG, VEC>), bgrid, bucket, 0, s, P);
+        hipLaunchKernelGGL((race_op_totals<BT, DP, NWG, ROWS>), bgrid, bucket, 0, s, P);
         break;
     case OP_READOUT:
         if (P.linear)
-            hipLaunchKernelGGL((race_op_out<ST, DP, false, true, VEC>), grid, value, 0, s, P);
+            hipLaunchKernelGGL((race_op_out<ST, DP, false, LIN, ROWS>), grid, value, 0, s, P);
         else
-            hipLaunchKernelGGL((race_op_out<ST, DP, false, false, VEC>), grid, value, 0, s, P);
+            hipLaunchKernelGGL((race_op_out<ST, DP, false, false, ROWS>), grid, value, 0, s, P);
         break;
     case OP_GQ:
         if (P.linear)
-            hipLaunchKernelGGL((race_op_gq<BT, DP, NWG, true, VEC>), bgrid, bucket, 0, s, P);
+            hipLaunchKernelGGL((race_op_gq<BT, DP, NWG, LIN, ROWS>), bgrid, bucket, 0, s, P);
         else
-            hipLaunchKernelGGL((race_op_gq<BT, DP, NWG, false, VEC>), bgrid, bucket, 0, s, P);
+            hipLaunchKernelGGL((race_op_gq<BT, DP, NWG, false, ROWS>), bgrid, bucket, 0, s, P);
         break;
     case OP_GKV:
         if constexpr (op_one_launch<ST, BT, DP>) {
             const dim3 vgrid(grid.x * (NWG + 1), grid.y, grid.z);
             if (P.linear)
-                hipLaunchKernelGGL((race_op_gkv<ST, BT, DP, true, VEC>), vgrid, bucket, 0, s, P);
+                hipLaunchKernelGGL((race_op_gkv<ST, BT, DP, LIN, ROWS>), vgrid, bucket, 0, s, P);
             else
-                hipLaunchKernelGGL((race_op_gkv<ST, BT, DP, false, VEC>), vgrid, bucket, 0, s, P);
+                hipLaunchKernelGGL((race_op_gkv<ST, BT, DP, false, ROWS>), vgrid, bucket, 0, s, P);
         } else if (P.linear) {
-            hipLaunchKernelGGL((race_op_gk<BT, DP, NWG, true, VEC>), bgrid, bucket, 0, s, P);
-            hipLaunchKernelGGL((race_op_out<ST, DP, true, true, VEC>), grid, value, 0, s, P);
+            hipLaunchKernelGGL((race_op_gk<BT, DP, NWG, LIN, ROWS>), bgrid, bucket, 0, s, P);
+            hipLaunchKernelGGL((race_op_out<ST, DP, true, LIN, ROWS>), grid, value, 0, s, P);
         } else {
-            hipLaunchKernelGGL((race_op_gk<BT, DP, NWG, false, VEC>), bgrid, bucket, 0, s, P);
-            hipLaunchKernelGGL((race_op_out<ST, DP, true, false, VEC>), grid, value, 0, s, P);
+            hipLaunchKernelGGL((race_op_gk<BT, DP, NWG, false, ROWS>), bgrid, bucket, 0, s, P);
+            hipLaunchKernelGGL((race_op_out<ST, DP, true, false, ROWS>), grid, value, 0, s, P);
         }
         break;
     }
@@ -67,7 +68,10 @@ int op_stage_tokens(int DP) { return op_stage(DP); }
 
 hipError_t launch_scan_op(OpKernel k, int ST, int DP, const ScanParams &P, dim3 grid, hipStream_t s)
 {
-#define X(a, b) if (ST == a && DP == b) return P.vec ? launch_v<a, b, true>(k, P, grid, s) : launch_v<a, b, false>(k, P, grid, s);
+#define X(a, b) if (ST == a && DP == b) \
+        return P.rows == ROWS_BF16  ? launch_v<a, b, ROWS_BF16>(k, P, grid, s) \
+               : P.rows == ROWS_F32 ? launch_v<a, b, ROWS_F32>(k, P, grid, s) \
+                                    : launch_v<a, b, ROWS_ANY>(k, P, grid, s);
     RACE_OP_VARIANTS(X)
 #undef X
     return hipErrorInvalidValue;

@@ -35,7 +35,7 @@ from torch.autograd import Function
 from . import _lib
 from .attention import RaceAttentionFn
 from .decode import RaceDecodeState
-from .race_causal_cuda import op_state, race_backward, race_fused_fwd
+from .race_causal_cuda import op_state, race_backward, race_fused_fwd, state_arg, state_buffer
 from .race_common import build_planes_protos, hash_bwd, hash_code, hash_fwd
 
 
@@ -135,10 +135,19 @@ def _group_sum(x, rep):
     return x if rep == 1 else x.view(x.shape[0] // rep, rep, *x.shape[1:]).sum(1)
 
 
+def _bf16_rows(x):
+    """[B,T,H,D] bf16 activations as the [B,H,T,D] view that the scan reads: itself where its rows allow it."""
+    sb, st, sh, sd = x.stride()
+    if sd != 1 or x.data_ptr() % 8 or (sb | st | sh) % 4 or not x.shape[3] <= st <= 1 << 22:
+        x = x.contiguous()
+    return x.transpose(1, 2)
+
+
 class _RaceSeamFn(Function):
     """y [B,T,Hq,D] = causal RACE in fp32 of activations q [B,T,Hq,D], k, v [B,T,Hkv,D], y in q's dtype;
     query head h reads kv head h // (Hq / Hkv). bf16 q and k are hashed as they are (their values
-    are exact in fp32; the planes stay fp32), in the activations' own layout."""
+    are exact in fp32; the planes stay fp32), in the activations' own layout. With one query head per kv
+    head the scan reads and writes bf16 rows there too; grouped heads sum their gradients in fp32."""
 
     @staticmethod
     def forward(ctx, q, k, v, planes_T, L, Kbits, scale, eps):
@@ -147,7 +156,9 @@ class _RaceSeamFn(Function):
         rep = Hq // k.shape[2]
         if k.shape != (B, T, k.shape[2], D) or v.shape[:3] != k.shape[:3] or Hq % k.shape[2]:
             raise ValueError(f"q {tuple(q.shape)} / k {tuple(k.shape)} / v {tuple(v.shape)} mismatch")
-        planes = _lib.f32_planes(planes_T)
+        planes, S = _lib.f32_planes(planes_T), L << Kbits
+        direct = (rep == 1 and q.dtype == v.dtype == torch.bfloat16 and v.shape[3] % 4 == 0 and S % 4 == 0
+                  and S <= 128 and v.shape[2] * v.shape[3] <= 1 << 22)  # (as race_op_fwd_bf16_rows takes them)
         kinds, rows = [], []
         for x in (q, k):
             if x.dtype not in (torch.float32, torch.bfloat16):
@@ -156,18 +167,40 @@ class _RaceSeamFn(Function):
             p, xc = hash_fwd(x.transpose(1, 2), planes, L, Kbits, 1, False, scale, code)
             kinds.append((code, p))
             rows.append(xc)
+        ctx.cfg = (L, Kbits, float(scale), float(eps), rep, kinds[0][0], kinds[1][0], q.dtype, k.dtype, v.dtype, direct)
+        if direct:
+            (_, pQ), (_, pK), V = *kinds, _bf16_rows(v)
+            out = torch.empty(B, T, Hq, V.shape[3], dtype=q.dtype, device=q.device)
+            nbytes = _lib.size("race_op_state_bytes", B * Hq, T, S, V.shape[3], 0)
+            state = state_buffer(nbytes, q.device, "race_op_state_bytes")
+            ws = _lib.workspace(_lib.size("race_op_workspace_bytes", B * Hq, T, S, V.shape[3], 0, 0), q.device)
+            _lib.check(_lib.lib().race_op_fwd_bf16_rows(
+                pK.data_ptr(), pQ.data_ptr(), _lib.view4(V)[0], _lib.view4(out.transpose(1, 2))[0], B, Hq, T, S,
+                V.shape[3], float(eps), 0, ws.data_ptr(), ws.numel(), *state_arg(state), _lib.stream_of(q)),
+                "race_op_fwd_bf16_rows")
+            ctx.save_for_backward(*rows, planes, pK, pQ, V, state)
+            return out
         pQ, pK, V = kinds[0][1], _per_query_head(kinds[1][1], rep), _per_query_head(_streams(v), rep)
         state = op_state(pK, V)  # the forward block states stay there for the backward
         out = race_fused_fwd(pK, pQ, V, eps, 0, state=state)
         ctx.save_for_backward(*rows, planes, pK, pQ, V, state)
-        ctx.cfg = (L, Kbits, float(scale), float(eps), rep, kinds[0][0], kinds[1][0], q.dtype, k.dtype, v.dtype)
         return _activations(out, B, q.dtype).detach()  # (no view, as attention._out_rows)
 
     @staticmethod
     def backward(ctx, grad):
         qc, kc, planes, pK, pQ, V, state = ctx.saved_tensors
-        L, Kbits, scale, eps, rep, q_code, k_code, q_dtype, k_dtype, v_dtype = ctx.cfg
-        gpk, gpq, gv = race_backward(pK, pQ, V, _streams(grad), eps, 0, state=state)
+        L, Kbits, scale, eps, rep, q_code, k_code, q_dtype, k_dtype, v_dtype, direct = ctx.cfg
+        if direct:
+            B, Hq, T, D = V.shape
+            go, gpk, gpq = _bf16_rows(grad), torch.empty_like(pK), torch.empty_like(pQ)
+            gv = torch.empty(B, T, Hq, D, dtype=v_dtype, device=V.device)
+            ws = _lib.workspace(_lib.size("race_op_workspace_bytes", B * Hq, T, L << Kbits, D, 0, 1), V.device)
+            _lib.check(_lib.lib().race_op_bwd_bf16_rows(
+                pK.data_ptr(), pQ.data_ptr(), _lib.view4(V)[0], _lib.view4(go)[0], gpk.data_ptr(), gpq.data_ptr(),
+                _lib.view4(gv.transpose(1, 2))[0], B, Hq, T, L << Kbits, D, eps, 0, ws.data_ptr(), ws.numel(),
+                *state_arg(state), _lib.stream_of(V)), "race_op_bwd_bf16_rows")
+        else:
+            gpk, gpq, gv = race_backward(pK, pQ, V, _streams(grad), eps, 0, state=state)
         needs, dq, dk, dv = ctx.needs_input_grad, None, None, None
         if needs[0]:
             dq = hash_bwd(qc, planes, gpq, L, Kbits, 1, False, scale, q_code).transpose(1, 2).to(q_dtype)
@@ -175,7 +208,7 @@ class _RaceSeamFn(Function):
             dk = hash_bwd(kc, planes, _group_sum(gpk, rep), L, Kbits, 1, False, scale, k_code)
             dk = dk.transpose(1, 2).to(k_dtype)
         if needs[2]:
-            dv = _activations(_group_sum(gv, rep), qc.shape[0], v_dtype)
+            dv = gv if direct else _activations(_group_sum(gv, rep), qc.shape[0], v_dtype)
         return dq, dk, dv, None, None, None, None, None
 
 

@@ -273,3 +273,31 @@ def test_integration_bindings_match_the_library_signatures():
     for name, res in re.findall(r"\b_?lib\.(race_\w+)\.restype = ([\w.]+)", text):
         assert alias.get(res.replace("ctypes.", ""), getattr(ctypes, res.replace("ctypes.", ""), None)) \
             == _lib.SIGNATURES[name][0], name
+
+
+def test_bf16_rows_refusals():
+    """race_op_fwd_bf16_rows / race_op_bwd_bf16_rows refuse, on the host, what their loads do not cover: wide
+    or ragged bucket counts, ragged head dims, unaligned or overlapping rows, and results that share rows."""
+    lib = _lib.lib()
+    H, T, D = 4, 100, 64
+    ok = _lib.Tensor4(64, T * H * D, D, H * D)
+    state = (ctypes.c_void_p(256), 1 << 40)
+    ws = (ctypes.c_void_p(256), 1 << 40)
+    p, n = ctypes.c_void_p(256), None
+
+    def fwd(V=ok, out=ok, B=2, S=24, D=D, pK=p):
+        return lib.race_op_fwd_bf16_rows(pK, p, V, out, B, H, T, S, D, 1e-6, 0, *ws, *state, n)
+
+    def bwd(gO=ok, gV=ok):
+        return lib.race_op_bwd_bf16_rows(p, p, ok, gO, p, p, gV, 2, H, T, 24, D, 1e-6, 0, *ws, *state, n)
+
+    invalid, unsupported = 1, 2
+    assert fwd(B=0) == invalid
+    for kw in (dict(S=132), dict(S=22), dict(D=62), dict(pK=ctypes.c_void_p(260))):
+        assert fwd(**kw) == unsupported, kw
+    for bad in (_lib.Tensor4(68, T * H * D, D, H * D), _lib.Tensor4(64, T * H * D, D + 2, H * D),
+                _lib.Tensor4(64, T * H * D, D, D - 4), _lib.Tensor4(64, T * H * D, D, (1 << 22) + 4)):
+        assert fwd(V=bad) == fwd(out=bad) == bwd(gO=bad) == bwd(gV=bad) == unsupported
+    shared = _lib.Tensor4(64, T * H * D, 0, H * D)
+    assert fwd(out=shared) == bwd(gV=shared) == invalid
+    assert fwd(V=_lib.Tensor4(0, T * H * D, D, H * D)) == invalid

@@ -98,3 +98,35 @@ def test_outputs_change_in_place(dev, call, H):
 
     for a, b in zip(grads(lambda y: y.mul_(2)), grads(lambda y: y * 2)):
         assert torch.equal(a, b)
+
+
+@pytest.mark.parametrize("B,T,H,D,L,K", [(2, 1, 1, 64, 2, 2), (2, 33, 3, 128, 3, 3), (1, 130, 2, 36, 1, 2), (1, 95, 2, 64, 8, 4),
+                                         (3, 600, 2, 256, 2, 4), (1, 2100, 6, 32, 4, 4), (1, 40, 2, 20, 5, 3)])
+@pytest.mark.parametrize("layout", ["contiguous", "packed", "odd_rows"])
+def test_bf16_rows_equal_the_cast_rows(dev, B, T, H, D, L, K, layout):
+    """The scan on bf16 rows in place against the same scan on fp32 copies, rounded once: equal to the bit,
+    at the edges of stages and tiles, for slices of one [B,T,3,H,D] tensor and for rows that start at odd
+    addresses (copied first)."""
+    from race_attention_amd import RaceCausalFn, build_planes_protos
+    from race_attention_amd.nanochat import race_attend
+    from race_attention_amd.race_common import hash_code, hash_fwd
+    print(f"bf16 rows B={B} T={T} H={H} D={D} L={L} K={K} {layout}", flush=True)
+    g = torch.Generator().manual_seed(T + D)
+    planes, protos = build_planes_protos(D, K, L, 1, device=dev, seed=0)
+    wide = torch.randn(B, T, 3, H, D + 1, generator=g).to(torch.bfloat16).to(dev)
+    if layout == "odd_rows":
+        q, k, v = (wide[:, :, i, :, 1:].detach().requires_grad_(True) for i in range(3))
+    else:
+        x = wide[..., :D].contiguous()
+        q, k, v = (t.detach().requires_grad_(True) for t in x.unbind(2)) if layout == "packed" else (
+            t.contiguous().detach().requires_grad_(True) for t in x.unbind(2))
+    go = torch.randn(B, T, H, D, generator=g).to(torch.bfloat16).to(dev)
+    y = race_attend(q, k, v, planes, L, K, EPS, precision="fp32", protos_T=protos)
+    dv, = torch.autograd.grad(y, v, go)
+    probs = [hash_fwd(t.detach().transpose(1, 2), planes, L, K, 1, False, math.sqrt(D), hash_code(t, fp32_planes=True))[0]
+             for t in (k, q)]
+    vf = v.detach().transpose(1, 2).float().reshape(B * H, T, D).requires_grad_(True)
+    out = RaceCausalFn.apply(*probs, vf, EPS)
+    dvf, = torch.autograd.grad(out, vf, go.transpose(1, 2).float().reshape(B * H, T, D))
+    assert torch.equal(y, out.detach().view(B, H, T, D).transpose(1, 2).to(torch.bfloat16))
+    assert torch.equal(dv, dvf.view(B, H, T, D).transpose(1, 2).to(torch.bfloat16))
