@@ -753,26 +753,59 @@ RACE_DEV void shm_project(float *sU, float *sX, const float *sPlT, const SoftHas
             }
     } else {
         f32x4 xr[DP / 32][2];
+        if constexpr (sizeof(TX) == 2) {
+            // all loads of the tile ahead of the first use, from clamped addresses: the widening right
+            // behind a load in its range check waited for each in turn (16 x 2047 tokens, 6 heads of 128,
+            // L*K = 9: forward 25.2 -> 22.4, backward 47.6 -> 42.2 us, with the gradients' loads below).
+            // fp32, with nothing to widen, keeps the checks (2^20 tokens x 4 streams of 128, the
+            // non-causal pass 5979 us against 6190)
+            typedef TX tx4 __attribute__((ext_vector_type(4)));
+            tx4 raw[DP / 32][2];
 #pragma unroll
-        for (int c = 0; c < DP / 32; ++c)
+            for (int c = 0; c < DP / 32; ++c)
 #pragma unroll
-            for (int it = 0; it < 2; ++it) {
-                const int r = it * 8 + lane / 8, col = 32 * c + 4 * (lane % 8);
-                f32x4 v = {0.0f, 0.0f, 0.0f, 0.0f};
-                if (t0 + r < tok1 && col < P.D) {
-                    const TX *p = x + (int64_t)(t0 + r) * P.x.st + col;
+                for (int it = 0; it < 2; ++it) {
+                    const int col = 32 * c + 4 * (lane % 8);
+                    const TX *row = x + (int64_t)min(t0 + it * 8 + lane / 8, tok1 - 1) * P.x.st;
                     if (vec) {
-                        typedef TX tx4 __attribute__((ext_vector_type(4)));
-                        const tx4 w = *reinterpret_cast<const tx4 *>(p);
-                        v = f32x4{(float)w[0], (float)w[1], (float)w[2], (float)w[3]};
+                        raw[c][it] = *reinterpret_cast<const tx4 *>(row + min(col, P.D - 4));
                     } else {
 #pragma unroll
                         for (int e = 0; e < 4; ++e)
-                            v[e] = col + e < P.D ? (float)p[e] : 0.0f;
+                            raw[c][it][e] = row[min(col + e, P.D - 1)];
                     }
                 }
-                xr[c][it] = v;
-            }
+#pragma unroll
+            for (int c = 0; c < DP / 32; ++c)
+#pragma unroll
+                for (int it = 0; it < 2; ++it)
+#pragma unroll
+                    for (int e = 0; e < 4; ++e)
+                        xr[c][it][e] = t0 + it * 8 + lane / 8 < tok1 && 32 * c + 4 * (lane % 8) + e < P.D
+                                           ? (float)raw[c][it][e]
+                                           : 0.0f;
+        } else {
+#pragma unroll
+            for (int c = 0; c < DP / 32; ++c)
+#pragma unroll
+                for (int it = 0; it < 2; ++it) {
+                    const int r = it * 8 + lane / 8, col = 32 * c + 4 * (lane % 8);
+                    f32x4 v = {0.0f, 0.0f, 0.0f, 0.0f};
+                    if (t0 + r < tok1 && col < P.D) {
+                        const TX *p = x + (int64_t)(t0 + r) * P.x.st + col;
+                        if (vec) {
+                            typedef TX tx4 __attribute__((ext_vector_type(4)));
+                            const tx4 w = *reinterpret_cast<const tx4 *>(p);
+                            v = f32x4{(float)w[0], (float)w[1], (float)w[2], (float)w[3]};
+                        } else {
+#pragma unroll
+                            for (int e = 0; e < 4; ++e)
+                                v[e] = col + e < P.D ? (float)p[e] : 0.0f;
+                        }
+                    }
+                    xr[c][it] = v;
+                }
+        }
 #pragma unroll
         for (int c = 0; c < DP / 32; ++c) {
 #pragma unroll
@@ -894,12 +927,40 @@ __global__ __launch_bounds__(SHM_W * 64) void race_softhash_bwd_mfma(SoftHashPar
     shm_load_planes<NJT, DP>(sPlT, sPl, P.planes, P, Y);
     __syncthreads();
     float gsu = 0.0f;  // sum of gu * u over this lane's (token, table) items
+    constexpr bool AHEAD = sizeof(TX) == 2;
+    constexpr int NP = (16 * (16 * NJT / KB) + 63) / 64;  // passes over the 16 L items (L K <= 16 NJT)
     const int span = P.tpw * SHM_W * 16;
     const int tok0 = blockIdx.x * span, tok1 = min(P.T, tok0 + span);
     for (int t0 = tok0 + 16 * w; t0 < tok1; t0 += 16 * SHM_W) {
+        // bf16: the probabilities' gradients of this lane's (token, table) items, in flight during the
+        // projection (fp32 x takes more registers: 200003 tokens x 4 streams, L*K = 32, the layer 2615 ->
+        // 2676 us)
+        float grads[AHEAD ? NP : 1][R];
+        auto load_grads = [&](float(&gr)[R], int i) {
+            const int r = i / P.L, l = i - r * P.L;
+            const float *gp = gprobs + (int64_t)min(t0 + r, tok1 - 1) * S + l * R;
+            if (R % 4 == 0 && vec_in) {
+#pragma unroll
+                for (int c = 0; c < R; c += 4) {
+                    const f32x4 v4 = *reinterpret_cast<const f32x4 *>(gp + c);
+#pragma unroll
+                    for (int e = 0; e < 4; ++e)
+                        gr[c + e] = v4[e];
+                }
+            } else {
+#pragma unroll
+                for (int c = 0; c < R; ++c)
+                    gr[c] = gp[c];
+            }
+        };
+        if constexpr (AHEAD) {
+#pragma unroll
+            for (int p = 0; p < NP; ++p)
+                load_grads(grads[p], min(lane + 64 * p, 16 * P.L - 1));
+        }
         shm_project<TX, NJT, DP>(sU, sX, sPlT, P, Y, x, t0, tok1, vec_x, lane, n16, g);
         // (token, table) items: gu_k = d loss / d u_k, gproj = gu * (1 - tanh^2) / scale
-        for (int i = lane; i < 16 * P.L; i += 64) {
+        auto item = [&](int i, float(&gr)[R]) {
             const int r = i / P.L, l = i - r * P.L;
             float u[KB], s0[KB], s1[KB], gu[KB];
 #pragma unroll
@@ -909,23 +970,11 @@ __global__ __launch_bounds__(SHM_W * 64) void race_softhash_bwd_mfma(SoftHashPar
                 gu[k] = 0.0f;
             }
             if (t0 + r < tok1) {
-                const float *gp = gprobs + (int64_t)(t0 + r) * S + l * R;
+                if constexpr (!AHEAD)
+                    load_grads(gr, i);
                 // gz_c = p_c (gp_c - sum p gp); gu_k = sum_c sign_k(c) gz_c with sign +1 where bit k
                 // of c is set: a butterfly from the least significant bit
-                float p[R], z[R], gr[R];
-                if (R % 4 == 0 && vec_in) {
-#pragma unroll
-                    for (int c = 0; c < R; c += 4) {
-                        const f32x4 v4 = *reinterpret_cast<const f32x4 *>(gp + c);
-#pragma unroll
-                        for (int e = 0; e < 4; ++e)
-                            gr[c + e] = v4[e];
-                    }
-                } else {
-#pragma unroll
-                    for (int c = 0; c < R; ++c)
-                        gr[c] = gp[c];
-                }
+                float p[R], z[R];
                 corner_probs<KB>(s0, s1, p);
                 float dot = 0.0f;
 #pragma unroll
@@ -954,6 +1003,15 @@ __global__ __launch_bounds__(SHM_W * 64) void race_softhash_bwd_mfma(SoftHashPar
                 const float th = u[k] * sh_scale(P);
                 sGP[r * Y.PD + l * KB + k] = gu[k] * sh_inv_scale(P) * (1.0f - th * th);
             }
+        };
+        if constexpr (AHEAD) {
+#pragma unroll
+            for (int p = 0; p < NP; ++p)
+                if (lane + 64 * p < 16 * P.L)
+                    item(lane + 64 * p, grads[p]);
+        } else {
+            for (int i = lane; i < 16 * P.L; i += 64)
+                item(i, grads[0]);
         }
         // dx^T tiles of 16 d: A = planes rows d (4-byte reads, pitch 4 x odd), B = gproj of token n16;
         // k-steps over the planes (L*K <= 16 NJT, rounded to 4). Two tiles (32 columns) at a time pass
