@@ -463,7 +463,7 @@ __global__ __launch_bounds__(ST * 4) void race_op_totals(const ScanParams P)
     const float *pK = P.pK + (int64_t)c.z * P.T * P.S;
 
     f32x4 St[NTD], pk[NSUB];
-    float a = 0.0f;
+    double a = 0.0;  // (one-signed terms: no rounding of a long sum, beside MFMA-bound waves)
 #pragma unroll
     for (int k = 0; k < NTD; ++k)
         St[k] = f32x4{0.f, 0.f, 0.f, 0.f};
@@ -484,7 +484,7 @@ __global__ __launch_bounds__(ST * 4) void race_op_totals(const ScanParams P)
 #pragma unroll
         for (int s = 0; s < NSUB; ++s) {
             p[s] = pk[s];
-            a += (p[s][0] + p[s][1]) + (p[s][2] + p[s][3]);
+            a += (double)((p[s][0] + p[s][1]) + (p[s][2] + p[s][3]));
         }
         fetch(t0 + TS);
         __syncthreads();
@@ -496,9 +496,10 @@ __global__ __launch_bounds__(ST * 4) void race_op_totals(const ScanParams P)
         __syncthreads();
     }
     op_st_state<NTD>(P.wsB + (c.slot * P.S_pad + c.s0) * P.DPw, St, P.DPw, c);
-    const GroupSums gs(a);
+    a += __shfl_xor(a, 16);
+    a += __shfl_xor(a, 32);
     if (c.g == 0)
-        P.wsA[c.slot * P.S_pad + c.s0 + col] = P.linear ? 0.0f : gs.total;
+        P.wsA[c.slot * P.S_pad + c.s0 + col] = P.linear ? 0.0f : (float)a;
 }
 
 // ============================================================================ gpQ and suffix totals
