@@ -213,6 +213,23 @@ def view4(t):
     return Tensor4(t.data_ptr(), s[0], s[1], s[2]), t
 
 
+def out_view4(t):
+    """race_tensor of a 4-D [B,H,T,D] result that the kernels write. Never a copy: what is written to one
+    would be lost, so a last dim that is not contiguous is refused."""
+    if t.dim() != 4 or t.stride(3) != 1:
+        raise RaceError(f"results are written to [B,H,T,D] rows, got shape {tuple(t.shape)}, strides {t.stride()}")
+    s = t.stride()
+    return Tensor4(t.data_ptr(), s[0], s[1], s[2])
+
+
+def rows_like(x):
+    """A new tensor for the gradient of x [B,H,T,D], in x's memory order where that keeps the rows of D
+    together (autograd then hands it on without a layout copy), contiguous otherwise: torch.empty_like
+    orders the dims by stride, and windows one element apart (x.unfold(2, D, 1)) have two of stride 1."""
+    g = torch.empty_like(x)
+    return g if g.stride(3) == 1 else torch.empty(x.shape, dtype=x.dtype, device=x.device)
+
+
 def dtype_code(dt):
     if dt == torch.float32:
         return RACE_F32

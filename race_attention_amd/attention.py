@@ -73,7 +73,7 @@ class RaceAttentionFn(Function):
         qv, _ = _lib.view4(q)
         kv_, _ = _lib.view4(k)
         vv, _ = _lib.view4(v)
-        ov, _ = _lib.view4(out)
+        ov = _lib.out_view4(out)
         _lib.check(lib.race_qkv_fwd(sh, qv, kv_, vv, _lib.ptr(planes), ov, _lib.dtype_code(out_dtype),
                                     _lib.ptr(state), state.numel(), _lib.ptr(scratch), scratch.numel(),
                                     _lib.stream_of(q)), "race_qkv_fwd")
@@ -89,8 +89,8 @@ class RaceAttentionFn(Function):
         sh = qkv_shape(q, k, L, Kbits, scale, eps, block)
         lib = _lib.lib()
         scratch = _lib.workspace(lib.race_qkv_scratch_bytes(sh, 1), q.device)
-        dq, dk, dv = torch.empty_like(q), torch.empty_like(k), torch.empty_like(v)
-        views = [_lib.view4(t)[0] for t in (q, k, v, go, dq, dk, dv)]
+        dq, dk, dv = (_lib.rows_like(t) for t in (q, k, v))
+        views = [_lib.view4(t)[0] for t in (q, k, v, go)] + [_lib.out_view4(t) for t in (dq, dk, dv)]
         _lib.check(lib.race_qkv_bwd(sh, views[0], views[1], views[2], views[3], _lib.ptr(planes),
                                     _lib.ptr(state), state.numel(), views[4], views[5], views[6],
                                     _lib.ptr(scratch), scratch.numel(), _lib.stream_of(q)), "race_qkv_bwd")
@@ -141,7 +141,8 @@ def race_causal_attention_with_state(q, k, v, planes_T, L, Kbits, scale=None, ep
                 or A.dtype != torch.float32 or Bs.dtype != torch.float32 or A.device != q.device
                 or Bs.device != q.device):
             raise ValueError(f"state_out must be contiguous fp32 [{B * Hkv},{S}] and [{B * Hkv},{S},{D}] on {q.device}")
-    qv, kv_, vv, ov = (_lib.view4(t)[0] for t in (q, k, v, out))
+    qv, kv_, vv = (_lib.view4(t)[0] for t in (q, k, v))
+    ov = _lib.out_view4(out)
     _lib.check(lib.race_qkv_prefill(sh, qv, kv_, vv, _lib.ptr(planes), ov, _lib.dtype_code(out_dtype), _lib.ptr(A),
                                     _lib.ptr(Bs), _lib.ptr(work), work.numel(), _lib.ptr(scratch), scratch.numel(),
                                     _lib.stream_of(q)), "race_qkv_prefill")

@@ -175,7 +175,7 @@ class _RaceSeamFn(Function):
             state = state_buffer(nbytes, q.device, "race_op_state_bytes")
             ws = _lib.workspace(_lib.size("race_op_workspace_bytes", B * Hq, T, S, V.shape[3], 0, 0), q.device)
             _lib.check(_lib.lib().race_op_fwd_bf16_rows(
-                pK.data_ptr(), pQ.data_ptr(), _lib.view4(V)[0], _lib.view4(out.transpose(1, 2))[0], B, Hq, T, S,
+                pK.data_ptr(), pQ.data_ptr(), _lib.view4(V)[0], _lib.out_view4(out.transpose(1, 2)), B, Hq, T, S,
                 V.shape[3], float(eps), 0, ws.data_ptr(), ws.numel(), *state_arg(state), _lib.stream_of(q)),
                 "race_op_fwd_bf16_rows")
             ctx.save_for_backward(*rows, planes, pK, pQ, V, state)
@@ -197,7 +197,7 @@ class _RaceSeamFn(Function):
             ws = _lib.workspace(_lib.size("race_op_workspace_bytes", B * Hq, T, L << Kbits, D, 0, 1), V.device)
             _lib.check(_lib.lib().race_op_bwd_bf16_rows(
                 pK.data_ptr(), pQ.data_ptr(), _lib.view4(V)[0], _lib.view4(go)[0], gpk.data_ptr(), gpq.data_ptr(),
-                _lib.view4(gv.transpose(1, 2))[0], B, Hq, T, L << Kbits, D, eps, 0, ws.data_ptr(), ws.numel(),
+                _lib.out_view4(gv.transpose(1, 2)), B, Hq, T, L << Kbits, D, eps, 0, ws.data_ptr(), ws.numel(),
                 *state_arg(state), _lib.stream_of(V)), "race_op_bwd_bf16_rows")
         else:
             gpk, gpq, gv = race_backward(pK, pQ, V, _streams(grad), eps, 0, state=state)

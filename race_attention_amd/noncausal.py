@@ -123,7 +123,7 @@ class RaceNonCausalViewFn(Function):
         state = state_buffer(_lib.size("race_op_state_bytes", N, T, S, D, 0), Vv.device, "race_op_state_bytes")
         ws = _lib.workspace(_lib.size("race_nc_op_workspace_bytes", N, T, S, D, 0, 0), Vv.device)
         vv, Vv = _lib.view4(Vv)
-        ov, _ = _lib.view4(_bhtd(out))
+        ov = _lib.out_view4(_bhtd(out))
         _lib.check(lib.race_nc_fwd_view(_lib.ptr(pK), _lib.ptr(pQ), vv, ov, M * B, H, T, S, D, float(eps), 0,
                                         _lib.ptr(ws), ws.numel(), *state_arg(state), _lib.stream_of(Vv)),
                    "race_nc_fwd_view")
@@ -145,7 +145,7 @@ class RaceNonCausalViewFn(Function):
         ws = _lib.workspace(_lib.size("race_nc_op_workspace_bytes", N, T, S, D, 0, 1), pK.device)
         vv, _ = _lib.view4(Vv)
         gov, gv_in = _lib.view4(gv_in)
-        gvv, _ = _lib.view4(_bhtd(gV))
+        gvv = _lib.out_view4(_bhtd(gV))
         _lib.check(lib.race_nc_bwd_view(_lib.ptr(pK), _lib.ptr(pQ), vv, gov, _lib.ptr(gpK), _lib.ptr(gpQ), gvv, M * B,
                                         H, T, S, D, ctx.eps, 0, _lib.ptr(ws), ws.numel(), *state_arg(state),
                                         _lib.stream_of(pK)), "race_nc_bwd_view")
@@ -187,11 +187,9 @@ class SoftHashTempFn(Function):
         B, H, T, D = Xc.shape
         Mp = M if unshared else 1
         g = gprobs.float().contiguous().view(Mp, B * H, T, -1)
-        # in X's own layout (a strided view of the caller's tensor): autograd hands it to the leaf
-        # without a layout copy
-        dX = torch.empty_like(Xc)
+        dX = _lib.rows_like(Xc)
         xv, _ = _lib.view4(Xc)
-        dv, _ = _lib.view4(dX)
+        dv = _lib.out_view4(dX)
         sh = _hash_shape(Xc, L, Kbits, Mp, unshared, 1.0)
         lib = _lib.lib()
         part = torch.empty(lib.race_soft_hash_bwd_partials(sh), dtype=torch.float32, device=Xc.device)

@@ -58,11 +58,11 @@ def hash_fwd(X, planes, L, Kbits, M, unshared, scale, code):
 
 
 def hash_bwd(Xc, planes, gprobs, L, Kbits, M, unshared, scale, code):
-    """dX, in X's own memory order (no layout copy on the way to a leaf), from gprobs fp32 contiguous."""
-    dX = torch.empty_like(Xc)
+    """dX, in X's own memory order (_lib.rows_like), from gprobs fp32 contiguous."""
+    dX = _lib.rows_like(Xc)
     sh = _hash_shape(Xc, L, Kbits, M if unshared else 1, unshared, scale)
     _lib.check(_lib.lib().race_soft_hash_bwd(sh, _lib.view4(Xc)[0], code, planes.data_ptr(), gprobs.data_ptr(),
-                                             _lib.view4(dX)[0], _lib.stream_of(Xc)), "race_soft_hash_bwd")
+                                             _lib.out_view4(dX), _lib.stream_of(Xc)), "race_soft_hash_bwd")
     return dX
 
 

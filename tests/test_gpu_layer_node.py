@@ -38,3 +38,32 @@ def test_layer_node_equals_its_parts(dtype, v_dtype, B, H, T, D, L, K, layout, n
     wanted = [x for x in leaves if x.requires_grad]
     for x, a, b in zip(wanted, torch.autograd.grad(got, wanted, go), torch.autograd.grad(ref, wanted, go)):
         assert a.dtype == x.dtype and torch.equal(a, b)
+
+
+@pytest.mark.parametrize("T,D", [(50, 64), (7, 64), (130, 128)])
+@pytest.mark.parametrize("call", ["module", "seam", "temperature"])
+def test_overlapping_windows_have_the_gradients_of_their_copies(T, D, call):
+    """Inputs whose tokens are windows one element apart (token and channel stride 1, which orders
+    torch.empty_like's dims differently): outputs and gradients equal those of contiguous copies."""
+    from race_attention_amd.nanochat import race_attend
+    from race_attention_amd.noncausal import SoftHashTempFn
+    L, K, B, H = 3, 2, 2, 2
+    m = RaceCausalCuda(D, K, L, 1, device="cuda", seed=3)
+    gen = torch.Generator("cuda").manual_seed(T)
+    xs = [torch.randn(B, H, T + D - 1, device="cuda", generator=gen).unfold(2, D, 1) for _ in range(3)]
+    go = torch.randn(B, H, T, D, device="cuda", generator=gen)
+
+    def grads(copy):
+        x = [(t.contiguous() if copy else t).detach().requires_grad_() for t in xs]
+        if call == "module":
+            y = m(*x)
+        elif call == "seam":
+            y = race_attend(*(t.transpose(1, 2) for t in x), m.planes_T, L, K, 1e-6, precision="fp32",
+                            protos_T=m.protos_T).transpose(1, 2)
+        else:
+            y = SoftHashTempFn.apply(x[0], m.planes_T, L, K, 1, False, torch.tensor(4.0, device="cuda"))
+            return (y, *torch.autograd.grad(y, x[:1], torch.ones_like(y).cumsum(-1)))
+        return (y, *torch.autograd.grad(y, x, go))
+
+    for a, b in zip(grads(False), grads(True)):
+        assert torch.equal(a, b)

@@ -1,0 +1,70 @@
+"""Where the host code lets the kernels write, without a GPU: the library is replaced by one that
+records the addresses it was given."""
+import pytest
+import torch
+
+from race_attention_amd import _lib, noncausal, race_common
+
+
+def layouts(B, H, T, D):
+    """[B,H,T,D] inputs whose last dim is contiguous, by name."""
+    x = torch.randn(B, H, T, D)
+    return {
+        "bhtd": x,
+        "bthd": torch.randn(B, T, H, D).transpose(1, 2),
+        "windows_step_1": torch.randn(B, H, T + D - 1).unfold(2, D, 1),  # two dims of stride 1
+        "windows_step_8": torch.randn(B, H, 8 * T + D).unfold(2, D, 8)[:, :, :T],
+        "one_head_for_all": x[:, :1].expand(B, H, T, D),
+        "one_token_for_all": x[:, :, :1].expand(B, H, T, D),
+        "fused_qkv": torch.randn(B, T, 3, H, D)[:, :, 1].transpose(1, 2),
+        "every_other_row": torch.randn(B, H, 2 * T, D)[:, :, ::2],
+    }
+
+
+class Recorder:
+    """Stands in for the library: every call succeeds and its arguments are kept."""
+
+    def __init__(self):
+        self.calls = {}
+
+    def __getattr__(self, name):
+        def call(*args):
+            self.calls[name] = args
+            return 16 if name.endswith("_partials") else 0
+        return call
+
+
+@pytest.fixture
+def recorder(monkeypatch):
+    r = Recorder()
+    monkeypatch.setattr(_lib, "lib", lambda: r)
+    monkeypatch.setattr(_lib, "stream_of", lambda t: 0)
+    monkeypatch.setattr(_lib, "require_device", lambda *t: None)
+    return r
+
+
+def same_rows(view, t):
+    assert view.data == t.data_ptr(), "the kernel writes somewhere else than into the result"
+    assert (view.stride_b, view.stride_h, view.stride_t, 1) == t.stride()
+
+
+@pytest.mark.parametrize("B,H,T,D", [(2, 3, 7, 64), (1, 2, 50, 64), (1, 1, 100, 16), (2, 2, 1, 8), (1, 2, 5, 1)])
+@pytest.mark.parametrize("layout", sorted(layouts(1, 1, 1, 8)))
+def test_soft_hash_gradients_are_written_into_the_result(recorder, B, H, T, D, layout):
+    X = layouts(B, H, T, D)[layout]
+    L, K = 2, 2
+    planes, g = torch.randn(D, L * K), torch.randn(B * H, T, L << K)
+    dX = race_common.hash_bwd(X, planes, g, L, K, 1, False, 8.0, _lib.RACE_F32)
+    assert dX.shape == X.shape and dX.dtype == X.dtype
+    same_rows(recorder.calls["race_soft_hash_bwd"][5], dX)
+    X.requires_grad_()
+    probs = noncausal.SoftHashTempFn.apply(X, planes, L, K, 1, False, torch.tensor(8.0))
+    dX, = torch.autograd.grad(probs, X, g)
+    same_rows(recorder.calls["race_soft_hash_bwd_dscale"][6], dX)
+
+
+def test_a_result_whose_rows_are_scattered_is_refused():
+    with pytest.raises(_lib.RaceError, match="rows"):
+        _lib.out_view4(torch.empty(1, 2, 64, 7).transpose(2, 3))
+    with pytest.raises(_lib.RaceError, match="rows"):
+        _lib.out_view4(torch.empty(2, 64, 7))
