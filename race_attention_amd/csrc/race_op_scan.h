@@ -186,10 +186,11 @@ struct RowStage {
         int64_t st;
     };
 
-    // item i, rows t0 .. of which nv belong to the stage
-    static RACE_DEV void load(Raw (&v)[4], const Src &s, int i, int t0, int nv, int D)
+    // item i of the stage at t0 of a block that ends at t_end (t0 >= t_end: nothing is read, or the
+    // block's last row again)
+    static RACE_DEV void load(Raw (&v)[4], const Src &s, int i, int t0, int t_end, int D)
     {
-        const int r = (i % IT) / CH * 4, c = (i % IT) % CH * 4;
+        const int r = (i % IT) / CH * 4, c = (i % IT) % CH * 4, nv = min(TS, t_end - t0);
         if constexpr (ROWS == ROWS_BF16) {
             const OpBuf b = op_buf(reinterpret_cast<const __bf16 *>(s.p) + (int64_t)t0 * s.st,
                                    nv > 0 ? (int64_t)(nv - 1) * s.st + D : 0, 2);
@@ -208,7 +209,7 @@ struct RowStage {
             for (int j = 0; j < 4; ++j)
 #pragma unroll
                 for (int e = 0; e < 4; ++e) {
-                    const float x = s.p[(int64_t)max(t0 + min(r + j, nv - 1), 0) * s.st + min(c + e, D - 1)];
+                    const float x = s.p[(int64_t)op_clamped_row(t0, r + j, t_end) * s.st + min(c + e, D - 1)];
                     v[j][e] = r + j < nv && c + e < D ? x : 0.0f;
                 }
         }
@@ -237,19 +238,19 @@ struct RowStage {
     }
 
     // NT = 2: items of tensor a first, then of tensor b
-    RACE_DEV void fetch(const Src &a, const Src &b, int t0, int nv, int D)
+    RACE_DEV void fetch(const Src &a, const Src &b, int t0, int t_end, int D)
     {
         if constexpr (AHEAD) {
 #pragma unroll
             for (int k = 0; k < N; ++k) {
                 const int i = threadIdx.x + k * NTH;
                 if (NT * IT % NTH == 0 || i < NT * IT)
-                    load(x[k], of_first(k) ? a : b, i, t0, nv, D);
+                    load(x[k], of_first(k) ? a : b, i, t0, t_end, D);
             }
         }
     }
 
-    RACE_DEV void put(const Src &a, const Src &b, float *rma, float *tra, float *rmb, float *trb, int t0, int nv,
+    RACE_DEV void put(const Src &a, const Src &b, float *rma, float *tra, float *rmb, float *trb, int t0, int t_end,
                       int D)
     {
 #pragma unroll
@@ -258,7 +259,7 @@ struct RowStage {
             if (NT * IT % NTH == 0 || i < NT * IT) {
                 const bool first = of_first(k);
                 if constexpr (!AHEAD)
-                    load(x[0], first ? a : b, i, t0, nv, D);
+                    load(x[0], first ? a : b, i, t0, t_end, D);
                 store(x[AHEAD ? k : 0], first ? rma : rmb, first ? tra : trb, i);
             }
         }
@@ -470,7 +471,7 @@ __global__ __launch_bounds__(ST * 4) void race_op_totals(const ScanParams P)
     RS rs;
     auto fetch = [&](int t0) {  // (past the block end: nothing is read)
         const int nv = max(min(TS, c.t_end - t0), 0);
-        rs.fetch(src, src, t0, nv, P.D);
+        rs.fetch(src, src, t0, c.t_end, P.D);
         const OpBuf bk = op_buf(pK + (int64_t)t0 * P.S, (int64_t)nv * P.S);
 #pragma unroll
         for (int s = 0; s < NSUB; ++s)
@@ -478,8 +479,7 @@ __global__ __launch_bounds__(ST * 4) void race_op_totals(const ScanParams P)
     };
     fetch(c.t_begin);
     for (int t0 = c.t_begin; t0 < c.t_end; t0 += TS) {
-        const int nv = min(TS, c.t_end - t0);
-        rs.put(src, src, nullptr, sVt, nullptr, nullptr, t0, nv, P.D);
+        rs.put(src, src, nullptr, sVt, nullptr, nullptr, t0, c.t_end, P.D);
         f32x4 p[NSUB];
 #pragma unroll
         for (int s = 0; s < NSUB; ++s) {
@@ -534,7 +534,7 @@ __global__ __launch_bounds__(ST * 4) __attribute__((amdgpu_waves_per_eu(op_waves
     RS rs;
     auto fetch = [&](int t0) {
         const int nv = max(min(TS, c.t_end - t0), 0);
-        rs.fetch(sv, sg, t0, nv, P.D);
+        rs.fetch(sv, sg, t0, c.t_end, P.D);
         const OpBuf bk = op_buf(pK + (int64_t)t0 * P.S, (int64_t)nv * P.S);
         const OpBuf bq = op_buf(pQ + (int64_t)t0 * P.S, (int64_t)nv * P.S);
 #pragma unroll
@@ -546,7 +546,7 @@ __global__ __launch_bounds__(ST * 4) __attribute__((amdgpu_waves_per_eu(op_waves
     fetch(c.t_begin);
     for (int t0 = c.t_begin; t0 < c.t_end; t0 += TS) {
         const int nv = min(TS, c.t_end - t0);
-        rs.put(sv, sg, sV, sVt, sGO, sGOt, t0, nv, P.D);
+        rs.put(sv, sg, sV, sVt, sGO, sGOt, t0, c.t_end, P.D);
         f32x4 k_[NSUB], q_[NSUB];
 #pragma unroll
         for (int s = 0; s < NSUB; ++s) {
@@ -638,7 +638,7 @@ RACE_DEV void op_gk(const ScanParams &P, const OpCtx &c, OpGkLds<ST, DP> &lds)
     auto fetch = [&](int i) {  // stage i (below 0: stage 0 again, not used)
         const int j = max(i, 0), t0 = c.t_begin + j * TS;
         const int nv = min(TS, c.t_end - t0);
-        rs.fetch(sv, sg, t0, nv, P.D);
+        rs.fetch(sv, sg, t0, c.t_end, P.D);
         const int64_t first = zoff + (int64_t)t0 * P.S, floats = (int64_t)nv * P.S;
         const OpBuf bq = op_buf(P.pQ + first, floats);
 #pragma unroll
@@ -659,7 +659,7 @@ RACE_DEV void op_gk(const ScanParams &P, const OpCtx &c, OpGkLds<ST, DP> &lds)
     for (int i = nst - 1; i >= 0; --i) {
         const int t0 = c.t_begin + i * TS;
         const int nv = min(TS, c.t_end - t0);
-        rs.put(sv, sg, sV, nullptr, sGO, sGOt, t0, nv, P.D);
+        rs.put(sv, sg, sV, nullptr, sGO, sGOt, t0, c.t_end, P.D);
         f32x4 w[NSUB], gA[NSUB];
         float a0 = a_next;
 #pragma unroll
@@ -809,7 +809,7 @@ RACE_DEV void op_value(const ScanParams &P, const OpCtx &c, OpValueLds<ST, DP> &
 #pragma unroll
                     for (int e = 0; e < 4; ++e) {
                         const int r = s * 16 + 4 * c.g + e;
-                        const float x = xsrc[(int64_t)max(t0 + min(r, nv - 1), 0) * xst + min(d, P.D - 1)];
+                        const float x = xsrc[(int64_t)op_clamped_row(t0, r, c.t_end) * xst + min(d, P.D - 1)];
                         xn[td][s][e] = r < nv && d < P.D ? x : 0.0f;
                     }
             }

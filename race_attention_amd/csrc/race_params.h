@@ -67,4 +67,9 @@ struct ScanParams {
     int linear;
 };
 
+// op path, rows loaded one element at a time: the token that stands in for token t0 + r of a block that ends
+// at t_end. Never behind the block's last one, also where the whole stage lies behind it (the look-ahead
+// of the last stage), so that every address formed is one of the tensor's rows.
+constexpr int op_clamped_row(int t0, int r, int t_end) { return t0 + r < t_end ? t0 + r : t_end - 1; }
+
 }  // namespace race

@@ -1,5 +1,8 @@
-"""Where the host code lets the kernels write, without a GPU: the library is replaced by one that
-records the addresses it was given."""
+"""Where the kernels read and write, without a GPU: the library is replaced by one that records the
+addresses it was given, and the index arithmetic of the headers is compiled for the host."""
+import os
+import subprocess
+
 import pytest
 import torch
 
@@ -68,3 +71,40 @@ def test_a_result_whose_rows_are_scattered_is_refused():
         _lib.out_view4(torch.empty(1, 2, 64, 7).transpose(2, 3))
     with pytest.raises(_lib.RaceError, match="rows"):
         _lib.out_view4(torch.empty(2, 64, 7))
+
+
+ROWS = r"""
+#include "race_params.h"
+#include <cstdio>
+int main()
+{
+    const int stages[] = {16, 32, 64};
+    for (int ts : stages)
+        for (int T = 1; T <= 3 * 64 + 1; ++T)
+            for (int CB = 16; CB <= T + 16; CB += 16)
+                for (int t_begin = 0; t_begin < T; t_begin += CB) {
+                    const int t_end = t_begin + CB < T ? t_begin + CB : T;
+                    for (int t0 = t_begin; t0 < t_end + ts; t0 += ts)  // the stages and one look-ahead
+                        for (int r = 0; r < ts; ++r) {
+                            const int row = race::op_clamped_row(t0, r, t_end);
+                            if (row < t_begin || row >= t_end || (t0 + r < t_end && row != t0 + r)) {
+                                std::printf("T=%d CB=%d stage=%d: row %d of [%d,%d) read for %d\n", T, CB, ts, row,
+                                            t_begin, t_end, t0 + r);
+                                return 1;
+                            }
+                        }
+                }
+    return 0;
+}
+"""
+
+
+def test_rows_loaded_ahead_stay_inside_the_block(tmp_path):
+    """Every row that the element-wise loads of the fp32 scan address, the look-ahead past a block's last
+    stage among them, is a row of that block."""
+    src, exe = tmp_path / "rows.cpp", tmp_path / "rows"
+    src.write_text(ROWS)
+    csrc = os.path.join(os.path.dirname(_lib.__file__), "csrc")
+    subprocess.run(["g++", "-std=c++17", "-O1", "-I", csrc, str(src), "-o", str(exe)], check=True)
+    r = subprocess.run([str(exe)], capture_output=True, text=True)
+    assert r.returncode == 0, r.stdout
