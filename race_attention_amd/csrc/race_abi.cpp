@@ -468,14 +468,13 @@ static int run_scan_op(OpKernel k, const Geo &g, const ScanParams &P, hipStream_
     return hip_check(launch_scan_op(k, g.ST, g.DP, P, grid, s), "race_op kernel launch");
 }
 
-// fp32 rows move as 16-byte range-checked runs where every row of the operands starts 16-byte aligned, no rows
-// overlap (the range ends behind a stage's last row) and a stage of 64 rows stays below the 2^31 bytes
-// that an offset covers
+// fp32 rows move as 16-byte range-checked runs (which need no more than 4-byte alignment) where a run holds
+// valid columns or none, no rows overlap (the range ends behind a stage's last row) and a stage of 64 rows
+// stays below the 2^31 bytes that an offset covers
 static void op_vec(ScanParams &P)
 {
     const auto apart = [&](const View &x) { return x.st >= P.D && x.st <= (1 << 22); };
-    P.rows = P.S % 4 == 0 && P.D % 4 == 0 && aligned16(P.pK) && aligned16(P.pQ) && aligned16(P.V) && aligned16(P.gO) &&
-            !((P.v.sb | P.v.sh | P.v.st | P.go.sb | P.go.sh | P.go.st) & 3) && apart(P.v) && apart(P.go);
+    P.rows = P.S % 4 == 0 && P.D % 4 == 0 && apart(P.v) && apart(P.go);
 }
 
 static int op_check(const float *pK, const float *pQ, const float *V, float eps, void *ws,

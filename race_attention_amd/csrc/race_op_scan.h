@@ -34,8 +34,9 @@
 
 namespace race {
 
-// How the rows of V, gO, out and gV lie (ScanParams::rows): fp32 rows of any alignment; fp32 rows that
-// move as 16-byte runs; bf16 rows that move as 8-byte runs, out and gV rounded to bf16 as they are
+// How the rows of V, gO, out and gV lie (ScanParams::rows): fp32 rows of any length and pitch, moved one
+// element at a time; fp32 rows that move as 16-byte runs (S % 4 == 0, D % 4 == 0, any address: 200003
+// tokens x 4 streams, S = 128, D = 64 at odd addresses, forward and backward 2260 -> 2077 us); bf16 rows that move as 8-byte runs, out and gV rounded to bf16 as they are
 // stored. The last are the activations of a bf16 model in their own layout: products, states and
 // sums stay fp32 and the results are those of fp32 copies to the bit, but no pass casts and transposes
 // V, gO, out and gV (16 x 2047 tokens, 6 heads of 128, S = 24: forward and backward 675 -> 529 us)
@@ -168,7 +169,11 @@ RACE_DEV void op_place(const ScanParams &P, int &blk, int &w)
 // Rows of V (and go) of one stage into LDS, row-major [TS][DP + 8] and / or transposed
 // [DP][TS + 8]. A thread moves 4 rows x 4 columns, so both layouts are written as 16-byte runs.
 // Rows beyond the stage and columns >= D read as zeros. bf16 rows wait as they are and are widened on
-// their way into LDS. The kinds of rows are compiled apart (: a branch between the two forms of
+// their way into LDS. Rows of any length and pitch are loaded one element at a time from clamped addresses, a
+// thread's 4 columns DP / 4 apart so that the lanes of a load read consecutive ones, and are masked on
+// their way into LDS: masked where they are loaded, the compiler moves each load under its mask and waits
+// for it there (200003 tokens x 4 streams, forward and backward: S = 10, D = 64 1724 -> 682 us; S = 128,
+// D = 50 3145 -> 2186). The kinds of rows are compiled apart (a branch between the two forms of
 // a load makes the compiler wait for it on the spot, 278 -> 200 us for the block totals of 200003
 // tokens x 4 streams, S = 128, D = 64). Up to 4 items per thread wait in registers, fetched a stage ahead; more
 // (few waves, wide rows) are moved when the stage begins.
@@ -206,28 +211,42 @@ struct RowStage {
                 v[j] = buf_ld4(b, off + j * st);
         } else {
 #pragma unroll
-            for (int j = 0; j < 4; ++j)
+            for (int j = 0; j < 4; ++j) {
+                const float *row = s.p + (int64_t)op_clamped_row(t0, r + j, t_end) * s.st;
 #pragma unroll
-                for (int e = 0; e < 4; ++e) {
-                    const float x = s.p[(int64_t)op_clamped_row(t0, r + j, t_end) * s.st + min(c + e, D - 1)];
-                    v[j][e] = r + j < nv && c + e < D ? x : 0.0f;
-                }
+                for (int e = 0; e < 4; ++e)
+                    v[j][e] = row[min(c / 4 + e * CH, D - 1)];
+            }
         }
     }
 
-    static RACE_DEV void store(const Raw (&raw)[4], float *rm, float *tr, int i)
+    static RACE_DEV void store(const Raw (&raw)[4], float *rm, float *tr, int i, int t0, int t_end, int D)
     {
         const int r = (i % IT) / CH * 4, c = (i % IT) % CH * 4;
-        const f32x4 v[4] = {op_widen(raw[0]), op_widen(raw[1]), op_widen(raw[2]), op_widen(raw[3])};
+        f32x4 v[4] = {op_widen(raw[0]), op_widen(raw[1]), op_widen(raw[2]), op_widen(raw[3])};
+        if constexpr (ROWS == ROWS_ANY) {
+#pragma unroll
+            for (int j = 0; j < 4; ++j)
+#pragma unroll
+                for (int e = 0; e < 4; ++e)
+                    v[j][e] = t0 + r + j < t_end && c / 4 + e * CH < D ? v[j][e] : 0.0f;
+        }
         if (rm) {
 #pragma unroll
             for (int j = 0; j < 4; ++j)
-                st4(rm + (r + j) * LDX + c, v[j]);
+                if constexpr (ROWS == ROWS_ANY) {
+#pragma unroll
+                    for (int e = 0; e < 4; ++e)
+                        rm[(r + j) * LDX + c / 4 + e * CH] = v[j][e];
+                } else {
+                    st4(rm + (r + j) * LDX + c, v[j]);
+                }
         }
         if (tr) {
 #pragma unroll
             for (int e = 0; e < 4; ++e)
-                st4(tr + (c + e) * LDT + r, f32x4{v[0][e], v[1][e], v[2][e], v[3][e]});
+                st4(tr + (ROWS == ROWS_ANY ? c / 4 + e * CH : c + e) * LDT + r,
+                    f32x4{v[0][e], v[1][e], v[2][e], v[3][e]});
         }
     }
 
@@ -260,7 +279,7 @@ struct RowStage {
                 const bool first = of_first(k);
                 if constexpr (!AHEAD)
                     load(x[0], first ? a : b, i, t0, t_end, D);
-                store(x[AHEAD ? k : 0], first ? rma : rmb, first ? tra : trb, i);
+                store(x[AHEAD ? k : 0], first ? rma : rmb, first ? tra : trb, i, t0, t_end, D);
             }
         }
     }
@@ -807,11 +826,9 @@ RACE_DEV void op_value(const ScanParams &P, const OpCtx &c, OpValueLds<ST, DP> &
 #pragma unroll
                 for (int s = 0; s < NSUB; ++s)
 #pragma unroll
-                    for (int e = 0; e < 4; ++e) {
-                        const int r = s * 16 + 4 * c.g + e;
-                        const float x = xsrc[(int64_t)op_clamped_row(t0, r, c.t_end) * xst + min(d, P.D - 1)];
-                        xn[td][s][e] = r < nv && d < P.D ? x : 0.0f;
-                    }
+                    for (int e = 0; e < 4; ++e)  // (masked where they are used)
+                        xn[td][s][e] = xsrc[(int64_t)op_clamped_row(t0, s * 16 + 4 * c.g + e, c.t_end) * xst +
+                                            min(d, P.D - 1)];
             }
         }
     };
@@ -883,8 +900,14 @@ RACE_DEV void op_value(const ScanParams &P, const OpCtx &c, OpValueLds<ST, DP> &
 #pragma unroll
         for (int td = 0; td < TD; ++td)
 #pragma unroll
-            for (int s = 0; s < NSUB; ++s)
+            for (int s = 0; s < NSUB; ++s) {
                 x[td][s] = op_widen(xn[td][s]);
+                if constexpr (ROWS == ROWS_ANY) {
+#pragma unroll
+                    for (int e = 0; e < 4; ++e)
+                        x[td][s][e] = s * 16 + 4 * c.g + e < nv && (c.wave + td * NW) * 16 + c.n < P.D ? x[td][s][e] : 0.0f;
+                }
+            }
         fetch(REV ? i - 1 : i + 1);
         __syncthreads();
         op_diag<NSUB, KS, NW, ST, LDS_, LDM>(sM, sQ, sK, REV, c);

@@ -1,6 +1,6 @@
 """The fp32 op-path kernels at the edges of their tiles, against the fp64 oracle: sub-chunks of 16
 tokens, stages of 16 / 32, bucket tiles of 16 .. 128 (and several), head-dim tiles of 32 .. 256, and
-operands whose rows are not 16-byte aligned, which move as single floats.
+operands whose rows are not 16-byte aligned, and sizes that are no multiple of 4, whose rows move as single floats.
 
 Bars as tests/test_gpu_op.py: forward 2e-5, gradients 1e-4 or twice what the reference formula itself
 loses in fp32 (gradProbsK cancels at a sequence's first tokens)."""
@@ -71,8 +71,8 @@ def test_linear_tile_edges(dev, T, E, M):
 
 @pytest.mark.parametrize("S,D", [(24, 64), (128, 128), (64, 256)])
 def test_unaligned_rows_equal_aligned_ones(dev, S, D):
-    """Rows that start 4 bytes off a 16-byte boundary take the kernels that move single floats: the
-    same arithmetic, so the results are bitwise those of the aligned operands."""
+    """Rows that start 4 bytes off a 16-byte boundary: the same arithmetic, so the results are bitwise
+    those of the aligned operands."""
     from race_attention_amd.race_causal_cuda import race_backward, race_fused_fwd
     args = [x.float().to(dev) for x in probs(2, 150, S, D, seed=S)]
 
@@ -87,6 +87,21 @@ def test_unaligned_rows_equal_aligned_ones(dev, S, D):
     assert torch.equal(race_fused_fwd(*args[:3], EPS), race_fused_fwd(*off[:3], EPS))
     for name, a, b in zip(("gpK", "gpQ", "gV"), race_backward(*args, EPS), race_backward(*off, EPS)):
         assert torch.equal(a, b), name
+
+
+@pytest.mark.parametrize("S,D", [(6, 30), (18, 62), (24, 126), (10, 250), (66, 65), (130, 33), (3, 3)])
+@pytest.mark.parametrize("T,block", [(1, 0), (33, 0), (150, 48)])
+def test_odd_sizes_equal_padded_ones(dev, S, D, T, block):
+    """Bucket counts or head dims that are no multiple of 4 take the kernels that move single floats; zeros
+    behind the buckets and columns make the same call for those that move 16-byte runs. The arithmetic
+    is the same, so the results are to the bit."""
+    from race_attention_amd.race_causal_cuda import race_backward, race_fused_fwd
+    print(f"odd sizes S={S} D={D} T={T} block={block}", flush=True)
+    args = [x.float().to(dev) for x in probs(2, T, S, D, seed=S + T)]
+    pad = [torch.nn.functional.pad(x, (0, -x.shape[2] % 4)) for x in args]
+    assert torch.equal(race_fused_fwd(*args[:3], EPS, block), race_fused_fwd(*pad[:3], EPS, block)[:, :, :D])
+    for name, a, b in zip(("gpK", "gpQ", "gV"), race_backward(*args, EPS, block), race_backward(*pad, EPS, block)):
+        assert torch.equal(a, b[:, :, :a.shape[2]]), name
 
 
 def test_values_beyond_a_block_do_not_leak(dev):
