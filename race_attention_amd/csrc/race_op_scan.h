@@ -20,13 +20,13 @@
 // gpQ that it wrote, instead of a second pass over go St^T with a second copy of the state.
 //
 // Measured against the kernels with the state in LDS that these replace (us, one MI355X):
-//   RACE, 200003 tokens x 4 streams, S = 128, D = 64: totals 189 -> 176, readout 525 -> 365 (and no
-//     partial outputs of two bucket tiles to add, 2 x 96), gpQ + totals 707 -> 610, gpK and gv
-//     1356 -> 927
-//   linear attention, 2^20 tokens x 4 streams, 64 x 64: 421 -> 424, 1205 -> 895, 1687 -> 1390,
-//     3185 -> 1960: at 3.3 - 5.0 TB/s of the compulsory reads and writes (a plain copy moves 4.8)
+//   RACE, 200003 tokens x 4 streams, S = 128, D = 64: totals 189 -> 178, readout 525 -> 355 (and no
+//     partial outputs of two bucket tiles to add, 2 x 96), gpQ + totals 707 -> 533, gpK and gv
+//     1356 -> 873
+//   linear attention, 2^20 tokens x 4 streams, 64 x 64: 421 -> 428, 1205 -> 888, 1687 -> 1334,
+//     3185 -> 1864: at 3.2 - 5.0 TB/s of the compulsory reads and writes (a plain copy moves 4.8)
 //     with the matrix cores busy 64, 74, 66 and 68 % of the time
-//   32752 tokens x 6 streams, S = 24, D = 128: 35 -> 29, 76 -> 60, 153 -> 119, 337 -> 89 + 84
+//   2047 tokens x 96 streams, bf16 rows, S = 24, D = 128: 35 -> 32, 76 -> 55, 153 -> 110, 337 -> 162
 #pragma once
 #include <type_traits>
 
@@ -70,6 +70,28 @@ RACE_DEV void mma4(f32x4 &c, const f32x4 &a, const f32x4 &b)
     for (int e = 0; e < 4; ++e)
         c = __builtin_amdgcn_mfma_f32_16x16x4f32(a[e], b[e], c, 0, 0, 0);
 }
+
+// A sum over N reduction steps of 16 in CH chains. One running sum rounds every term at the size of the
+// whole; in 4 chains, out of the fp32 layer at 2048 tokens, 128 buckets, is 1.07e-7 off 64 bits (relative
+// 2-norm) instead of 1.63e-7, gv 1.23e-7 instead of 1.69e-7, in the same time. The gradients of the
+// probabilities, sums over the head dim, take 1 (4 chains: gq 532 -> 579 us at 200003 tokens x 4 streams,
+// S = 128, for a tenth of their error), for gpQ of linear attention 2 (1357 -> 1285 us at 2^20 tokens)
+template <int N, int C>
+struct Chains {
+    static constexpr int CH = N < C ? N : C;
+    f32x4 c[CH] = {};
+    RACE_DEV void add(int i, const f32x4 &a, const f32x4 &b) { mma4(c[i % CH], a, b); }
+    RACE_DEV f32x4 sum() const
+    {
+        f32x4 x = c[0];
+        if constexpr (CH == 2)
+            x += c[1];
+        else if constexpr (CH == 4)
+            x = (x + c[1]) + (c[2] + c[3]);
+        static_assert(CH == 1 || CH == 2 || CH == 4, "chains are added in pairs");
+        return x;
+    }
+};
 
 RACE_DEV f32x4 ld4(const float *p) { return *reinterpret_cast<const f32x4 *>(p); }
 RACE_DEV void st4(float *p, const f32x4 &v) { *reinterpret_cast<f32x4 *>(p) = v; }
@@ -510,8 +532,11 @@ __global__ __launch_bounds__(ST * 4) void race_op_totals(const ScanParams P)
 #pragma unroll
         for (int s = 0; s < NSUB; ++s)
 #pragma unroll
-            for (int k = 0; k < NTD; ++k)
-                mma4(St[k], ld4(sVt + (k * 16 + c.n) * RS::LDT + s * 16 + 4 * c.g), p[s]);
+            for (int k = 0; k < NTD; ++k) {
+                f32x4 t = {0.f, 0.f, 0.f, 0.f};
+                mma4(t, ld4(sVt + (k * 16 + c.n) * RS::LDT + s * 16 + 4 * c.g), p[s]);
+                St[k] += t;  // (one rounding per sub-chunk at the size of the block's sum)
+            }
         __syncthreads();
     }
     op_st_state<NTD>(P.wsB + (c.slot * P.S_pad + c.s0) * P.DPw, St, P.DPw, c);
@@ -588,11 +613,12 @@ __global__ __launch_bounds__(ST * 4) __attribute__((amdgpu_waves_per_eu(op_waves
             if constexpr (!LIN)
                 inv = op_inv_a(k_[s], a0, eps, c.g);
             const f32x4 w = LIN ? q_[s] : q_[s] * inv;
-            f32x4 acc = {0.f, 0.f, 0.f, 0.f};
+            Chains<NTD, LIN ? 2 : 1> sum;
+            sum.add(0, op_m<NSUB, KS, LDM>(sM, s, c), k_[s]);
 #pragma unroll
             for (int k = 0; k < NTD; ++k)
-                mma4(acc, ld4(sGO + (s * 16 + c.n) * RS::LDX + k * 16 + 4 * c.g), St[k]);
-            mma4(acc, op_m<NSUB, KS, LDM>(sM, s, c), k_[s]);
+                sum.add(k, ld4(sGO + (s * 16 + c.n) * RS::LDX + k * 16 + 4 * c.g), St[k]);
+            f32x4 acc = sum.sum();
 #pragma unroll
             for (int k = 0; k < NTD; ++k) {
                 Tt[k].add(ld4(sGOt + (k * 16 + c.n) * RS::LDT + s * 16 + 4 * c.g), w);
@@ -696,11 +722,15 @@ RACE_DEV void op_gk(const ScanParams &P, const OpCtx &c, OpGkLds<ST, DP> &lds)
         const OpBuf out = op_buf(P.gpK + zoff + (int64_t)t0 * P.S, (int64_t)nv * P.S);
 #pragma unroll
         for (int s = NSUB - 1; s >= 0; --s) {
-            f32x4 acc = {0.f, 0.f, 0.f, 0.f};
+            Chains<NTD, 1> sum;
+            if constexpr (LIN)
+                sum.add(0, op_m<NSUB, KS, LDM>(sM, s, c), w[s]);
 #pragma unroll
             for (int k = 0; k < NTD; ++k)
-                mma4(acc, ld4(sV + (s * 16 + c.n) * RS::LDX + k * 16 + 4 * c.g), dS[k].value());
-            mma4(acc, op_m<NSUB, KS, LDM>(sM, s, c), w[s]);
+                sum.add(k, ld4(sV + (s * 16 + c.n) * RS::LDX + k * 16 + 4 * c.g), dS[k].value());
+            f32x4 acc = sum.sum();
+            if constexpr (!LIN)  // (large weights of a sequence's first tokens: last, as in the gv walk)
+                mma4(acc, op_m<NSUB, KS, LDM>(sM, s, c), w[s]);
 #pragma unroll
             for (int k = 0; k < NTD; ++k)
                 dS[k].add(ld4(sGOt + (k * 16 + c.n) * RS::LDT + s * 16 + 4 * c.g), w[s]);
@@ -923,33 +953,41 @@ RACE_DEV void op_value(const ScanParams &P, const OpCtx &c, OpValueLds<ST, DP> &
 #pragma unroll
         for (int ss = 0; ss < NSUB; ++ss) {
             const int s = REV ? NSUB - 1 - ss : ss;
-            f32x4 acc[TD];
+            Chains<NTS, 4> sum[TD];
+            const f32x4 m = op_m<NSUB, KS, LDM>(sM, s, c);
+            // the sub-chunk's own tokens first, below the size of the sum; where the weights W of a sequence's
+            // first tokens, up to 1 / eps, stand on the other side of m, last: the rest would be rounded
+            // at their size (gv of sharp probabilities, 3001 tokens, S = 24, D = 128: 4.5e-7 against 1.3e-7 off)
+            constexpr bool OWN_LAST = REV && !LIN;
+            if constexpr (!OWN_LAST) {
 #pragma unroll
-            for (int td = 0; td < TD; ++td)
-                acc[td] = f32x4{0.f, 0.f, 0.f, 0.f};
+                for (int td = 0; td < TD; ++td)
+                    sum[td].add(0, m, x[td][s]);
+            }
 #pragma unroll
             for (int st = 0; st < NTS; ++st) {
                 const f32x4 q = ld4(sQ + (s * 16 + c.n) * LDS_ + st * 16 + 4 * c.g);
                 const f32x4 k = ld4(sKt + (st * 16 + c.n) * LDT + s * 16 + 4 * c.g);
 #pragma unroll
                 for (int td = 0; td < TD; ++td) {
-                    mma4(acc[td], q, St[td][st].value());
+                    sum[td].add(st, q, St[td][st].value());
                     St[td][st].add(k, x[td][s]);
                 }
             }
-            const f32x4 m = op_m<NSUB, KS, LDM>(sM, s, c);
 #pragma unroll
             for (int td = 0; td < TD; ++td) {
-                mma4(acc[td], m, x[td][s]);
+                f32x4 acc = sum[td].sum();
+                if constexpr (OWN_LAST)
+                    mma4(acc, m, x[td][s]);
                 const int d = (c.wave + td * NW) * 16 + c.n;
                 const uint32_t st = BF ? (uint32_t)o.st * 2 : P.D * 4;
                 const uint32_t off = d < P.D ? 4 * c.g * st + d * (BF ? 2 : 4) : OP_OOB;
                 if constexpr (BF) {
 #pragma unroll
                     for (int e = 0; e < 4; ++e)
-                        buf_st_h(dst, off + (s * 16 + e) * st, acc[td][e]);
+                        buf_st_h(dst, off + (s * 16 + e) * st, acc[e]);
                 } else {
-                    op_store_tile(dst, off, st, s * 16, acc[td]);
+                    op_store_tile(dst, off, st, s * 16, acc);
                 }
             }
         }

@@ -142,3 +142,48 @@ def test_value_row_pitch(dev, pitch):
     wide = torch.full((1, 1, T, 1, pitch), float("nan"), device=dev)
     wide[..., :D] = v
     assert torch.equal(ace(k, wide[..., :D], q, EPS), ace(k, v, q, EPS))
+
+
+def norm_err(got, ref):
+    return ((got.double().cpu() - ref).norm() / ref.norm()).item()
+
+
+def test_rounding_of_the_layer_sums(dev):
+    """Errors of the fp32 layer against 64 bits, 128 buckets. The sum over the buckets runs on the matrix
+    cores, one rounding per 4 buckets: 32 in a row give u / sqrt(3) * sqrt(32 / 2) = 1.4e-7 (u = 2^-24) of a
+    sum of random signs, four chains of 8 half of that or less; the products' own inputs (probabilities, state)
+    add 0.8e-7. Measured: out 1.63e-7 in one running sum, 1.07e-7 in four chains; dv 1.69e-7 and 1.23e-7."""
+    from race_attention_amd.race_causal_cuda import RaceCausalCuda
+    from race_ref import oracle_layer
+    B, H, T, D, L, K = 1, 4, 2048, 64, 8, 4
+    m = RaceCausalCuda(D, K, L, 1, device=dev, seed=0)
+    g = torch.Generator().manual_seed(0)
+    q, k, v, go = (torch.randn(B, H, T, D, generator=g) for _ in range(4))
+    x = [t.to(dev).requires_grad_() for t in (q, k, v)]
+    out = m(*x)
+    out.backward(go.to(dev))
+    ref, _, _, dv = oracle_layer(q, k, v, m.planes_T.cpu(), L, K, D ** 0.5, m.eps, go)
+    errs = norm_err(out.detach(), ref), norm_err(x[2].grad, dv)
+    print("out, dv:", ["%.3e" % e for e in errs], flush=True)
+    assert errs[0] <= 1.35e-7 and errs[1] <= 1.45e-7, errs
+
+
+def test_rounding_of_the_linear_sums(dev):
+    """As above for causal linear attention on positive features (its sums grow with the sequence), 8 streams of
+    3001 tokens: out, dQ, dK, dV 1.21e-7, 2.29e-7, 1.48e-7, 1.14e-7 off in running sums over the head dim and
+    a block's tokens, 0.65e-7, 1.71e-7, 1.29e-7, 0.57e-7 in chains and one rounding per sub-chunk; the bars lie
+    between the two."""
+    from race_attention_amd.linear_attention import causal_linear_attention
+    g = torch.Generator().manual_seed(0)
+    q, k = (torch.rand(2, 4, 3001, 32, generator=g) for _ in range(2))
+    v, go = (torch.randn(2, 4, 3001, 32, generator=g) for _ in range(2))
+    ref_in = [t.double().requires_grad_() for t in (q, k, v)]
+    ref = orc.causal_linear_ref(*ref_in)
+    ref.backward(go.double())
+    got_in = [t.to(dev).requires_grad_() for t in (q, k, v)]
+    got = causal_linear_attention(*got_in)
+    got.backward(go.to(dev))
+    errs = [norm_err(a, b) for a, b in zip([got.detach()] + [t.grad for t in got_in],
+                                           [ref.detach()] + [t.grad for t in ref_in])]
+    print("out, dQ, dK, dV:", ["%.3e" % e for e in errs], flush=True)
+    assert all(e <= bar for e, bar in zip(errs, (0.95e-7, 2.0e-7, 1.4e-7, 0.85e-7))), errs
