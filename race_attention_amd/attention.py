@@ -29,7 +29,7 @@ def _bf16_rows(t):
     """A [B,H,T,D] bf16 view whose rows the kernels can read as 16-byte vectors."""
     sb, sh, st, sd = t.stride()
     if sd != 1 or t.data_ptr() % 16 or (sb | sh | st) % 8:
-        t = t.contiguous()
+        t = t.clone(memory_format=torch.contiguous_format)  # (contiguous() keeps an odd address)
     return t
 
 

@@ -139,7 +139,7 @@ def _bf16_rows(x):
     """[B,T,H,D] bf16 activations as the [B,H,T,D] view that the scan reads: itself where its rows allow it."""
     sb, st, sh, sd = x.stride()
     if sd != 1 or x.data_ptr() % 8 or (sb | st | sh) % 4 or not x.shape[3] <= st <= 1 << 22:
-        x = x.contiguous()
+        x = x.clone(memory_format=torch.contiguous_format)  # (contiguous() keeps an odd address, a stride of T = 1)
     return x.transpose(1, 2)
 
 

@@ -130,3 +130,31 @@ def test_bf16_rows_equal_the_cast_rows(dev, B, T, H, D, L, K, layout):
     dvf, = torch.autograd.grad(out, vf, go.transpose(1, 2).float().reshape(B * H, T, D))
     assert torch.equal(y, out.detach().view(B, H, T, D).transpose(1, 2).to(torch.bfloat16))
     assert torch.equal(dv, dvf.view(B, H, T, D).transpose(1, 2).to(torch.bfloat16))
+
+
+@pytest.mark.parametrize("precision", ["fp32", "bf16"])
+@pytest.mark.parametrize("T", [1, 70])
+def test_rows_at_odd_addresses(dev, precision, T):
+    """Contiguous q, k, v and an upstream gradient that start 2 bytes off (a part of a flat buffer): taken, with
+    the results of aligned copies."""
+    from race_attention_amd import build_planes_protos
+    from race_attention_amd.nanochat import race_attend
+    B, H, D, L, K = 2, 3, 64, 2, 3
+    planes, protos = build_planes_protos(D, K, L, 1, device=dev, seed=0)
+    g = torch.Generator().manual_seed(T)
+    rows = [torch.randn(B, T, H, D, generator=g).to(torch.bfloat16).to(dev) for _ in range(4)]
+
+    def shifted(x):
+        buf = torch.empty(x.numel() + 1, dtype=x.dtype, device=dev)
+        y = buf[1:].view(x.shape)
+        y.copy_(x)
+        assert y.data_ptr() % 8 == 2 and y.is_contiguous()
+        return y
+
+    def grads(move):
+        x = [move(r).requires_grad_(True) for r in rows[:3]]
+        y = race_attend(*x, planes, L, K, EPS, precision=precision, protos_T=protos)
+        return (y, *torch.autograd.grad(y, x, move(rows[3])))
+
+    for a, b in zip(grads(shifted), grads(torch.clone)):
+        assert torch.equal(a, b)

@@ -6,7 +6,7 @@ import subprocess
 import pytest
 import torch
 
-from race_attention_amd import _lib, noncausal, race_common
+from race_attention_amd import _lib, attention, nanochat, noncausal, race_common
 
 
 def layouts(B, H, T, D):
@@ -71,6 +71,31 @@ def test_a_result_whose_rows_are_scattered_is_refused():
         _lib.out_view4(torch.empty(1, 2, 64, 7).transpose(2, 3))
     with pytest.raises(_lib.RaceError, match="rows"):
         _lib.out_view4(torch.empty(2, 64, 7))
+
+
+def odd_rows(B, T, H, D):
+    """[B,T,H,D] bf16 rows that the kernels cannot read in place, by name."""
+    n = B * T * H * D
+    flat = torch.arange(4 * n + 64, dtype=torch.float32).to(torch.bfloat16)
+    return {
+        "contiguous_at_an_odd_address": flat[1:1 + n].view(B, T, H, D),
+        "one_token_with_an_odd_stride": flat.as_strided((B, 1, H, D), (2 * H * D + 8, 3 * H * D + 1, D, 1)),
+        "one_token_with_no_stride": flat.as_strided((B, 1, H, D), (H * D, 0, D, 1)),
+        "channels_apart": flat[:2 * n].view(B, T, H, 2 * D)[..., ::2],
+        "slice_of_wider_rows": flat[:B * T * H * (D + 1)].view(B, T, H, D + 1)[..., 1:],
+    }
+
+
+@pytest.mark.parametrize("B,T,H,D", [(2, 3, 2, 64), (1, 1, 1, 64), (1, 5, 3, 128)])
+@pytest.mark.parametrize("layout", sorted(odd_rows(1, 1, 1, 8)))
+def test_rows_are_copied_to_where_the_kernels_can_read_them(B, T, H, D, layout):
+    x = odd_rows(B, T, H, D)[layout]
+    y = nanochat._bf16_rows(x)  # (race_op_fwd_bf16_rows: 8-byte runs, tokens D .. 2^22 elements apart)
+    assert torch.equal(y, x.transpose(1, 2)) and y.stride(3) == 1 and y.data_ptr() % 8 == 0
+    assert not any(s % 4 for s in y.stride()[:3]) and D <= y.stride(2) <= 1 << 22
+    y = attention._bf16_rows(x.transpose(1, 2))  # (race_qkv_fwd: 16-byte runs)
+    assert torch.equal(y, x.transpose(1, 2)) and y.stride(3) == 1 and y.data_ptr() % 16 == 0
+    assert not any(s % 8 for s in y.stride()[:3])
 
 
 ROWS = r"""
