@@ -512,6 +512,28 @@ static void state_views(const Geo &g, const float *state, float *&wsB, float *&w
     wsA = wsB + align256(g.state_elems_B * 4) / 4;
 }
 
+// No two rows of a result [B][H][T][D] share an element: workgroups write them at the same time.
+static int rows_apart(const View &v, int64_t B, int64_t H, int64_t T, int64_t D, const char *name, const char *who)
+{
+    int64_t st[3] = {v.sb, v.sh, v.st}, n[3] = {B, H, T};
+    for (int i = 0; i < 3; ++i)  // sort the three dimensions by stride
+        for (int j = i + 1; j < 3; ++j)
+            if (st[j] < st[i]) {
+                std::swap(st[i], st[j]);
+                std::swap(n[i], n[j]);
+            }
+    int64_t span = D;  // elements covered by the dimensions taken so far
+    for (int i = 0; i < 3; ++i) {
+        if (n[i] <= 1)
+            continue;
+        if (st[i] < span)
+            return fail(RACE_ERR_INVALID, "%s: output %s has overlapping rows (strides %lld, %lld, %lld)", who, name,
+                        (long long)v.sb, (long long)v.sh, (long long)v.st);
+        span = st[i] * (n[i] - 1) + span;
+    }
+    return RACE_OK;
+}
+
 // bf16 rows through views ([B][H][T][D], stream z = b * H + h): 8-byte runs, one bucket tile
 struct OpBf16Rows {
     race_tensor V, go, out;  // go: the backward's upstream gradient, out: the output or gV
@@ -535,9 +557,7 @@ static int op_bf16_check(const OpBf16Rows &r, const race_tensor *go, int64_t B, 
             return fail(RACE_ERR_UNSUPPORTED, "%s: bf16 rows must start 8-byte aligned, at least D and at most 2^22 "
                         "elements apart", who);
     }
-    if ((r.out.stride_h < D && r.H > 1) || (r.out.stride_b < D && B > 1))
-        return fail(RACE_ERR_INVALID, "%s: the streams of the result share rows", who);
-    return RACE_OK;
+    return rows_apart(to_view(r.out), B, r.H, T, D, go ? "gV" : "out", who);
 }
 
 static void op_bf16_params(ScanParams &P, const OpBf16Rows &r, OutView &result)
@@ -814,24 +834,8 @@ static int nc_view_check(const View &v, int64_t Bz, int64_t H, int64_t T, int64_
         return fail(RACE_ERR_INVALID, "%s: null %s", who, name);
     if (v.sb < 0 || v.sh < 0 || v.st < D || v.st >= ((int64_t)1 << 31))
         return fail(RACE_ERR_INVALID, "%s: %s strides must be >= 0 with D <= token stride < 2^31", who, name);
-    if (output) {
-        int64_t st[3] = {v.sb, v.sh, v.st}, n[3] = {Bz, H, T};
-        for (int i = 0; i < 3; ++i)  // sort the three dimensions by stride
-            for (int j = i + 1; j < 3; ++j)
-                if (st[j] < st[i]) {
-                    std::swap(st[i], st[j]);
-                    std::swap(n[i], n[j]);
-                }
-        int64_t span = D;  // elements covered by the dimensions taken so far
-        for (int i = 0; i < 3; ++i) {
-            if (n[i] <= 1)
-                continue;
-            if (st[i] < span)
-                return fail(RACE_ERR_INVALID, "%s: output %s has overlapping rows (strides %lld, %lld, %lld)", who,
-                            name, (long long)v.sb, (long long)v.sh, (long long)v.st);
-            span = st[i] * (n[i] - 1) + span;
-        }
-    }
+    if (output)
+        return rows_apart(v, Bz, H, T, D, name, who);
     return RACE_OK;
 }
 

@@ -298,6 +298,9 @@ def test_bf16_rows_refusals():
     for bad in (_lib.Tensor4(68, T * H * D, D, H * D), _lib.Tensor4(64, T * H * D, D + 2, H * D),
                 _lib.Tensor4(64, T * H * D, D, D - 4), _lib.Tensor4(64, T * H * D, D, (1 << 22) + 4)):
         assert fwd(V=bad) == fwd(out=bad) == bwd(gO=bad) == bwd(gV=bad) == unsupported
-    shared = _lib.Tensor4(64, T * H * D, 0, H * D)
-    assert fwd(out=shared) == bwd(gV=shared) == invalid
+    for sb, sh, st in ((T * H * D, 0, H * D), (T * H * D, D, D),        # heads on one row, on the next token's
+                       (D, T * D, D), (T * H * D, T * D // 2, D),       # batches, heads half way through another's
+                       (H * D, D, H * D), (T * H * D - D, D, H * D)):   # batches a token on, a row short
+        shared = _lib.Tensor4(64, sb, sh, st)
+        assert fwd(out=shared) == bwd(gV=shared) == invalid, (sb, sh, st)
     assert fwd(V=_lib.Tensor4(0, T * H * D, D, H * D)) == invalid
