@@ -640,7 +640,10 @@ struct MoverRows {
 };
 
 // ============================================================================ forward readout
-template <int ST, int DP, int KB, int NW, bool OUT_F32, bool G1>
+// ONE: the sequence is this one block (ScanParams::single). A variant of its own, so that the general one
+// carries none of it (an extra product for the mass behind a test of P.single made the general one's
+// readout of 2^20 tokens x 4 heads 640 -> 649 us, in another place 700)
+template <int ST, int DP, int KB, int NW, bool OUT_F32, bool G1, bool ONE>
 __global__ __launch_bounds__(NW * 64) __attribute__((amdgpu_waves_per_eu(FCfg<ST, DP, KB, NW>::RO_WAVES)))
 void race_fused_fwd_readout(const ScanParams P)
 {
@@ -695,7 +698,7 @@ void race_fused_fwd_readout(const ScanParams P)
         for (int i = 0; i < TPW_S; ++i) {
             const int t = wave + i * NW;
             accS[i] = f32x4{0.f, 0.f, 0.f, 0.f};
-            if (t < CF::NTS * CF::NTD && !P.single) {  // (uniform)
+            if (!ONE && t < CF::NTS * CF::NTD) {
                 const int m0 = (t / CF::NTD) * 16, n0 = (t % CF::NTD) * 16;
                 const int r = acc_row(m0, lane), col = acc_col(n0, lane);
 #pragma unroll
@@ -705,7 +708,7 @@ void race_fused_fwd_readout(const ScanParams P)
         }
         const float *wA = P.wsA + slot * P.S_pad + c.s0;
         for (int s = tid; s < ST; s += NTH)
-            sA0[0][s] = P.single ? P.eps : wA[s] + P.eps;  // the carry holds A + eps
+            sA0[0][s] = ONE ? 0.0f : wA[s] + P.eps;  // the carry holds A + eps; ONE: A, the state it ends as
     }
 
     const int G = G1 ? 1 : P.G;  // G1: one query head per kv head, the head loop folds away
@@ -824,7 +827,7 @@ void race_fused_fwd_readout(const ScanParams P)
                             *reinterpret_cast<f32x4 *>(&sA0[nxt][s]) = a;
 #pragma unroll
                         for (int e = 0; e < 4; ++e)
-                            accA[i][e] = frcp(a[e]);
+                            accA[i][e] = frcp(ONE ? a[e] + P.eps : a[e]);
                     }
                     const bf16x4 q4 = *reinterpret_cast<const bf16x4 *>(&sPQ[tok][s]);
                     f32x4 w;
@@ -905,7 +908,7 @@ void race_fused_fwd_readout(const ScanParams P)
     }
     // last output rows
     store_out<OT, C, DP, LDO, NTH>(P.out, c.b, prev_h, c.st, prev_t0, prev_nv, sO, arO, tid);
-    if (P.single) {  // (uniform) the one block's end is the sequence's
+    if constexpr (ONE) {  // the one block's end is the sequence's
         float *fB = P.finB + c.z * P.finBz, *fA = P.finA + c.z * P.finAz;
 #pragma unroll
         for (int i = 0; i < TPW_S; ++i) {
@@ -923,7 +926,7 @@ void race_fused_fwd_readout(const ScanParams P)
         }
         for (int s = tid; s < ST; s += NTH) {
             if (c.s0 + s < P.finS)
-                fA[c.s0 + s] = sA0[nsub & 1][s] - P.eps;
+                fA[c.s0 + s] = sA0[nsub & 1][s];
             if (P.wsA)
                 P.wsA[slot * P.S_pad + c.s0 + s] = 0.0f;
         }

@@ -27,11 +27,17 @@ static hipError_t launch_fv(ScanKernel k, const ScanParams &P, dim3 grid, hipStr
             hipLaunchKernelGGL((race_fused_fwd_totals<ST, DP, KB, NW>), grid, block, 0, s, P);
         else
             return hipErrorInvalidValue;
-    } else if (k == K_FWD_READOUT && (P.out.f32 || P.out.stage_f32))
-        hipLaunchKernelGGL((race_fused_fwd_readout<ST, DP, KB, NW, true, G1>), grid, block, 0, s, P);
-    else if (k == K_FWD_READOUT)
-        hipLaunchKernelGGL((race_fused_fwd_readout<ST, DP, KB, NW, false, G1>), grid, block, 0, s, P);
-    else if (k == K_BWD_TOTALS && G1 && ST == 128 && DP == 64 && KB == 4 && !P.dq.f32) {
+    } else if (k == K_FWD_READOUT) {
+        const bool f32 = P.out.f32 || P.out.stage_f32;
+        if (P.single && f32)
+            hipLaunchKernelGGL((race_fused_fwd_readout<ST, DP, KB, NW, true, G1, true>), grid, block, 0, s, P);
+        else if (P.single)
+            hipLaunchKernelGGL((race_fused_fwd_readout<ST, DP, KB, NW, false, G1, true>), grid, block, 0, s, P);
+        else if (f32)
+            hipLaunchKernelGGL((race_fused_fwd_readout<ST, DP, KB, NW, true, G1, false>), grid, block, 0, s, P);
+        else
+            hipLaunchKernelGGL((race_fused_fwd_readout<ST, DP, KB, NW, false, G1, false>), grid, block, 0, s, P);
+    } else if (k == K_BWD_TOTALS && G1 && ST == 128 && DP == 64 && KB == 4 && !P.dq.f32) {
         // wave-specialised variant, bf16 dq: eight state waves and four helper waves (race_fused_ws.h),
         // also with fp32 staging of a later bucket tile (cfg2: 1 % faster than the 8-wave kernel
         // there); for the first tile's fp32 partial output the 8-wave kernel measured 1.5 % faster

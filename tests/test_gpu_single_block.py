@@ -66,6 +66,32 @@ def test_prefill_many_streams_leaves_the_state_in_place(dev):
         RaceDecodeState(B // 2, Hq, Hkv, D, L, K, planes, device=dev).prefill(q, k, v)
 
 
+@pytest.mark.parametrize("T,D,L,K,Hq,Hkv", [(1, 64, 8, 4, 2, 2), (77, 64, 8, 4, 4, 2), (96, 128, 16, 4, 3, 3), (33, 64, 5, 2, 4, 1)])
+def test_mass_of_a_single_block_holds_no_eps(dev, T, D, L, K, Hq, Hkv):
+    """The state's mass A is a sum of probabilities: whatever eps is (1e4 leaves 2^-11 of a sum that it is part
+    of), A has the same bits, and is the sum of the general path's totals."""
+    from race_attention_amd import _lib, build_planes_protos, race_causal_attention_with_state
+    from race_attention_amd.attention import qkv_shape
+    g = torch.Generator().manual_seed(T)
+    q, k, v = (torch.randn(1, h, T, D, generator=g).to(torch.bfloat16).to(dev) for h in (Hq, Hkv, Hkv))
+    planes, _ = build_planes_protos(D, K, L, 1, device=dev, seed=2)
+    scale, S = 0.5, L << K  # (sharp: masses down to 1e-6 of the largest)
+    A = [race_causal_attention_with_state(q, k, v, planes, L, K, scale=scale, eps=e)[1] for e in (1e-6, 1e-2, 1e4)]
+    assert torch.equal(A[0], A[1]) and torch.equal(A[0], A[2])
+    # the general path: the same call in blocks of 32 tokens
+    sh, lib = qkv_shape(q, k, L, K, scale, 1e-6, 32), _lib.lib()
+    state = _lib.workspace(lib.race_qkv_state_bytes(sh), dev)
+    scr = _lib.workspace(lib.race_qkv_scratch_bytes(sh, 0), dev)
+    out, A2, B2 = torch.empty_like(q), torch.empty_like(A[0]), torch.empty(Hkv, S, D, device=dev)
+    views = [_lib.view4(t)[0] for t in (q, k, v)]
+    _lib.check(lib.race_qkv_prefill(sh, *views, _lib.ptr(planes), _lib.out_view4(out), _lib.RACE_BF16, _lib.ptr(A2),
+                                    _lib.ptr(B2), _lib.ptr(state), state.numel(), _lib.ptr(scr), scr.numel(),
+                                    _lib.stream_of(q)), "race_qkv_prefill")
+    # a matrix step adds its 32 tokens to the running sum (or, there, to zero) in at most 8 additions of 4
+    # products, each off by up to an ulp of the sum, 2^-23 of it; the sums differ in what they start from
+    assert ((A[0] - A2).abs() <= 8 * (T // 32 + 1) * 2.0 ** -23 * A2.abs()).all()
+
+
 @pytest.mark.parametrize("T", [20, 3000])
 def test_prefill_forms(dev, T):
     """One stream's prompt prefills the state of every sequence, and rows of k and v behind the prompt are
