@@ -97,9 +97,11 @@ int op_geometry(int64_t N, int64_t T, int64_t S, int64_t D, int64_t block, Geo &
     if (D > 256)
         return fail(RACE_ERR_UNSUPPORTED, "race_op: head dim D = %lld > 256 is not compiled", (long long)D);
     g.DP = D <= 32 ? 32 : D <= 64 ? 64 : D <= 128 ? 128 : 256;
-    // bucket tiles of up to 128: every V and gO row is read once for all of them and no partial
-    // outputs are summed
-    g.ST = 128;
+    // bucket tiles of up to 128: every V and gO row is read once for all of them and no partial outputs are
+    // summed; beyond 128 buckets tiles of 64 where 128 would leave one empty (forward and backward of
+    // 2047 tokens x 96 streams, S = 192, D = 64 1165 -> 850 us, S = 320 1584 -> 1390; the kernels with
+    // tiles of 64 alone that were there before took 1105 and 1869)
+    g.ST = S > 128 && rup(S, 64) < rup(S, 128) ? 64 : 128;
     for (int st : {16, 32, 64})
         if (st >= S) {
             g.ST = st;

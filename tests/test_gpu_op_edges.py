@@ -89,6 +89,20 @@ def test_unaligned_rows_equal_aligned_ones(dev, S, D):
         assert torch.equal(a, b), name
 
 
+@pytest.mark.parametrize("S", [129, 192, 193, 256, 257, 320])
+@pytest.mark.parametrize("D", [40, 128])
+def test_several_bucket_tiles(dev, S, D):
+    """Both sides of the line between tiles of 64 and of 128 beyond 128 buckets: sums over 2 to 5 tiles."""
+    from race_attention_amd.race_causal_cuda import race_backward, race_fused_fwd
+    pk, pq, v, go = probs(3, 100, S, D, seed=S)
+    out_t, gpk_t, gpq_t, gv_t, _, _ = oracle_op(pk, pq, v, go, EPS)
+    a = [x.float().to(dev) for x in (pk, pq, v, go)]
+    check("out", race_fused_fwd(*a[:3], EPS), out_t, 2e-5)
+    floors = fp32_formula_floor(pk, pq, v, go, EPS, (gpk_t, gpq_t, gv_t))
+    for name, g, ref, f in zip(("gpK", "gpQ", "gV"), race_backward(*a, EPS), (gpk_t, gpq_t, gv_t), floors):
+        check(name, g, ref, max(1e-4, 2.0 * f))
+
+
 @pytest.mark.parametrize("S,D", [(6, 30), (18, 62), (24, 126), (10, 250), (66, 65), (130, 33), (3, 3)])
 @pytest.mark.parametrize("T,block", [(1, 0), (33, 0), (150, 48)])
 def test_odd_sizes_equal_padded_ones(dev, S, D, T, block):
