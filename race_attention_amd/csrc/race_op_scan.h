@@ -197,16 +197,14 @@ RACE_DEV void op_place(const ScanParams &P, int &blk, int &w)
 // for it there (200003 tokens x 4 streams, forward and backward: S = 10, D = 64 1724 -> 682 us; S = 128,
 // D = 50 3145 -> 2186). The kinds of rows are compiled apart (a branch between the two forms of
 // a load makes the compiler wait for it on the spot, 278 -> 200 us for the block totals of 200003
-// tokens x 4 streams, S = 128, D = 64). Up to 4 items per thread wait in registers, fetched a stage ahead; more
-// (few waves, wide rows) are moved when the stage begins.
+// tokens x 4 streams, S = 128, D = 64). All items wait in registers, fetched a stage ahead.
 template <int TS, int DP, int NTH, int NT, int ROWS>
 struct RowStage {
     static constexpr int CH = DP / 4, IT = (TS / 4) * CH, N = (NT * IT + NTH - 1) / NTH;
-    static constexpr bool AHEAD = N <= 4;
     static constexpr int LDX = op_pitch(DP), LDT = op_pitch(TS);
     static_assert(IT % 64 == 0, "one tensor per wave and item");
     typedef typename std::conditional<ROWS == ROWS_BF16, u32x2, f32x4>::type Raw;
-    Raw x[AHEAD ? N : 1][4];
+    Raw x[N][4];
 
     struct Src {  // (p: the address of the stream's first row, whatever its elements)
         const float *p;
@@ -281,27 +279,22 @@ struct RowStage {
     // NT = 2: items of tensor a first, then of tensor b
     RACE_DEV void fetch(const Src &a, const Src &b, int t0, int t_end, int D)
     {
-        if constexpr (AHEAD) {
 #pragma unroll
-            for (int k = 0; k < N; ++k) {
-                const int i = threadIdx.x + k * NTH;
-                if (NT * IT % NTH == 0 || i < NT * IT)
-                    load(x[k], of_first(k) ? a : b, i, t0, t_end, D);
-            }
+        for (int k = 0; k < N; ++k) {
+            const int i = threadIdx.x + k * NTH;
+            if (NT * IT % NTH == 0 || i < NT * IT)
+                load(x[k], of_first(k) ? a : b, i, t0, t_end, D);
         }
     }
 
-    RACE_DEV void put(const Src &a, const Src &b, float *rma, float *tra, float *rmb, float *trb, int t0, int t_end,
-                      int D)
+    RACE_DEV void put(float *rma, float *tra, float *rmb, float *trb, int t0, int t_end, int D)
     {
 #pragma unroll
         for (int k = 0; k < N; ++k) {
             const int i = threadIdx.x + k * NTH;
             if (NT * IT % NTH == 0 || i < NT * IT) {
                 const bool first = of_first(k);
-                if constexpr (!AHEAD)
-                    load(x[0], first ? a : b, i, t0, t_end, D);
-                store(x[AHEAD ? k : 0], first ? rma : rmb, first ? tra : trb, i, t0, t_end, D);
+                store(x[k], first ? rma : rmb, first ? tra : trb, i, t0, t_end, D);
             }
         }
     }
@@ -408,6 +401,23 @@ constexpr int op_shares(int NW, int NSUB, int ksteps)
     while (ks < 4 && 2 * ks * NSUB <= NW && ksteps % (2 * ks) == 0)
         ks *= 2;
     return ks;
+}
+
+// Whether V and go also lie transposed in LDS, for the products that sum over tokens (their operand is then one
+// 16-byte read). One wave to a workgroup and rows of 256 would leave one wave to a CU: 4 single reads
+// of the rows instead leave 4 (100003 tokens x 4 streams, S = 16, D = 256: gq 1198 -> 290 us, gk and gv 811 -> 460)
+constexpr bool op_transposed(int ST, int DP) { return ST > 16 || DP < 256; }
+
+// rows k (of the transposed tile; columns of the row-major one) x tokens of sub-chunk s
+template <bool TR, int LDX, int LDT>
+RACE_DEV f32x4 op_tokens(const float *rm, const float *tr, int k, int s, const OpCtx &c)
+{
+    if constexpr (TR) {
+        return ld4(tr + (k * 16 + c.n) * LDT + s * 16 + 4 * c.g);
+    } else {
+        const float *p = rm + (s * 16 + 4 * c.g) * LDX + k * 16 + c.n;
+        return f32x4{p[0], p[LDX], p[2 * LDX], p[3 * LDX]};
+    }
 }
 
 template <int ROWS>
@@ -520,7 +530,7 @@ __global__ __launch_bounds__(ST * 4) void race_op_totals(const ScanParams P)
     };
     fetch(c.t_begin);
     for (int t0 = c.t_begin; t0 < c.t_end; t0 += TS) {
-        rs.put(src, src, nullptr, sVt, nullptr, nullptr, t0, c.t_end, P.D);
+        rs.put(nullptr, sVt, nullptr, nullptr, t0, c.t_end, P.D);
         f32x4 p[NSUB];
 #pragma unroll
         for (int s = 0; s < NSUB; ++s) {
@@ -557,7 +567,8 @@ __global__ __launch_bounds__(ST * 4) __attribute__((amdgpu_waves_per_eu(op_waves
     constexpr int KS = op_shares(NW, NSUB, DP / 16);
     using RS = RowStage<TS, DP, NTH, 2, ROWS>;
     __shared__ __align__(16) float sV[TS * RS::LDX], sGO[TS * RS::LDX];
-    __shared__ __align__(16) float sVt[DP * RS::LDT], sGOt[DP * RS::LDT];
+    constexpr bool TR = op_transposed(ST, DP);
+    __shared__ __align__(16) float sVt[TR ? DP * RS::LDT : 1], sGOt[TR ? DP * RS::LDT : 1];
     __shared__ __align__(16) float sM[KS * NSUB * 16 * LDM];
     int blk, wg;
     op_place<NWG>(P, blk, wg);
@@ -590,7 +601,7 @@ __global__ __launch_bounds__(ST * 4) __attribute__((amdgpu_waves_per_eu(op_waves
     fetch(c.t_begin);
     for (int t0 = c.t_begin; t0 < c.t_end; t0 += TS) {
         const int nv = min(TS, c.t_end - t0);
-        rs.put(sv, sg, sV, sVt, sGO, sGOt, t0, c.t_end, P.D);
+        rs.put(sV, TR ? sVt : nullptr, sGO, TR ? sGOt : nullptr, t0, c.t_end, P.D);
         f32x4 k_[NSUB], q_[NSUB];
 #pragma unroll
         for (int s = 0; s < NSUB; ++s) {
@@ -621,8 +632,8 @@ __global__ __launch_bounds__(ST * 4) __attribute__((amdgpu_waves_per_eu(op_waves
             f32x4 acc = sum.sum();
 #pragma unroll
             for (int k = 0; k < NTD; ++k) {
-                Tt[k].add(ld4(sGOt + (k * 16 + c.n) * RS::LDT + s * 16 + 4 * c.g), w);
-                mma4(St[k], ld4(sVt + (k * 16 + c.n) * RS::LDT + s * 16 + 4 * c.g), k_[s]);
+                Tt[k].add(op_tokens<TR, RS::LDX, RS::LDT>(sGO, sGOt, k, s, c), w);
+                mma4(St[k], op_tokens<TR, RS::LDX, RS::LDT>(sV, sVt, k, s, c), k_[s]);
             }
             if constexpr (!LIN) {
                 acc *= inv;
@@ -652,7 +663,8 @@ template <int ST, int DP>
 struct OpGkLds {
     static constexpr int TS = op_stage(DP), NW = ST / 16, NSUB = TS / 16, LDM = 24;
     static constexpr int KS = op_shares(NW, NSUB, DP / 16), LDX = op_pitch(DP), LDT = op_pitch(TS);
-    float V[TS * LDX], GO[TS * LDX], GOt[DP * LDT], M[KS * NSUB * 16 * LDM];
+    static constexpr bool TR = op_transposed(ST, DP);
+    float V[TS * LDX], GO[TS * LDX], GOt[TR ? DP * LDT : 4], M[KS * NSUB * 16 * LDM];
 };
 
 template <int ST, int DP, bool LIN, int ROWS>
@@ -704,7 +716,7 @@ RACE_DEV void op_gk(const ScanParams &P, const OpCtx &c, OpGkLds<ST, DP> &lds)
     for (int i = nst - 1; i >= 0; --i) {
         const int t0 = c.t_begin + i * TS;
         const int nv = min(TS, c.t_end - t0);
-        rs.put(sv, sg, sV, nullptr, sGO, sGOt, t0, c.t_end, P.D);
+        rs.put(sV, nullptr, sGO, LD::TR ? sGOt : nullptr, t0, c.t_end, P.D);
         f32x4 w[NSUB], gA[NSUB];
         float a0 = a_next;
 #pragma unroll
@@ -733,7 +745,7 @@ RACE_DEV void op_gk(const ScanParams &P, const OpCtx &c, OpGkLds<ST, DP> &lds)
                 mma4(acc, op_m<NSUB, KS, LDM>(sM, s, c), w[s]);
 #pragma unroll
             for (int k = 0; k < NTD; ++k)
-                dS[k].add(ld4(sGOt + (k * 16 + c.n) * RS::LDT + s * 16 + 4 * c.g), w[s]);
+                dS[k].add(op_tokens<LD::TR, RS::LDX, RS::LDT>(sGO, sGOt, k, s, c), w[s]);
             if constexpr (!LIN) {
                 f32x4 q = gA[s];
 #pragma unroll

@@ -101,7 +101,7 @@ def test_outputs_change_in_place(dev, call, H):
 
 
 @pytest.mark.parametrize("B,T,H,D,L,K", [(2, 1, 1, 64, 2, 2), (2, 33, 3, 128, 3, 3), (1, 130, 2, 36, 1, 2), (1, 95, 2, 64, 8, 4),
-                                         (3, 600, 2, 256, 2, 4), (1, 2100, 6, 32, 4, 4), (1, 40, 2, 20, 5, 3)])
+                                         (3, 600, 2, 256, 2, 4), (1, 2100, 6, 32, 4, 4), (1, 40, 2, 20, 5, 3), (1, 90, 2, 256, 2, 2)])
 @pytest.mark.parametrize("layout", ["contiguous", "packed", "odd_rows"])
 def test_bf16_rows_equal_the_cast_rows(dev, B, T, H, D, L, K, layout):
     """The scan on bf16 rows in place against the same scan on fp32 copies, rounded once: equal to the bit,

@@ -89,6 +89,13 @@ def test_unaligned_rows_equal_aligned_ones(dev, S, D):
         assert torch.equal(a, b), name
 
 
+@pytest.mark.parametrize("S,D", [(3, 129), (8, 192), (16, 256)])
+@pytest.mark.parametrize("T,block", [(1, 0), (17, 0), (100, 48)])
+def test_one_wave_of_wide_rows(dev, S, D, T, block):
+    """Up to 16 buckets at head dims above 128: a workgroup is one wave, with V and go in LDS as rows only."""
+    test_tile_edges(dev, 2, T, S, D, block)
+
+
 @pytest.mark.parametrize("S", [129, 192, 193, 256, 257, 320])
 @pytest.mark.parametrize("D", [40, 128])
 def test_several_bucket_tiles(dev, S, D):
