@@ -1251,11 +1251,17 @@ hipError_t softhash_prepare(int D, int LK)
 // loaded at once straight to the registers that use them (in that order, so that waiting for the
 // inputs does not wait for the state), a projection is shared by D / 8 lanes of one wave (8 products
 // each, then lane shuffles), and the probabilities are products of per-bit sigmoids, one per thread.
-// Four workgroups of 256 threads per CU within 128 VGPRs: fewer registers spill (6 waves per SIMD:
-// 39 us, 8: 51), and eight small workgroups per CU that all start with their inputs (the former
-// kernel) leave the memory idle meanwhile. 32 q / 8 kv heads, D = 64, S = 128, bf16 (us per step):
-// 8 sequences 10.4 -> 7 (kernel alone), 64: 14.7 -> 10.2, 128: 18.5 -> 14.6, 256: 26.6 -> 24.3
-// (5.7 TB/s), 600: 66.1 -> 62.9; 256 sequences at D = 128: 67.9 -> 58.0.
+// Beyond two workgroups per CU, 256 threads and five workgroups per CU within 102 VGPRs: half of a
+// thread's first state rows are loaded with the inputs, the other half once the inputs have left
+// their registers (all at once: four workgroups; fewer registers yet spill, 39 to 51 us). A workgroup of
+// the next round then starts with its inputs, which a model has just written but a queue of prompts
+// may have left in HBM: the workgroup DEC_AHEAD before it has read them once, so that they wait in the
+// caches. 32 q / 8 kv heads, D = 64, S = 128, bf16, us per step with the same rows each time / with rows
+// that no cache holds: 256 sequences 26.8 / 27.1 with the former kernel (eight small workgroups per
+// CU), 24.1 / 27.7 with four workgroups and nothing read ahead, 23.9 / 24.6 now (5.7 TB/s); 600: 53.2 / 57.8,
+// 50.9 / 58.6, 50.6 / 54.0; 128: 16.8 / 17.2, 12.8 / 13.2, 12.6 / 13.1; 8: 10.0 / 10.9, 6.1 / 8.0, 6.1 / 7.9.
+// More than 4 query heads per kv head: four workgroups (600 sequences, 32 / 4 heads 46.2 / 48.0 with three,
+// 38.6 / 39.6; five spill, 39.3 / 40.2)
 template <class TX>
 struct DecRow8 {  // 8 consecutive elements of a row of any alignment
     struct __attribute__((packed, aligned(sizeof(TX)))) Raw {
@@ -1266,12 +1272,12 @@ struct DecRow8 {  // 8 consecutive elements of a row of any alignment
 };
 
 template <class TX, int D, int GM, int NT>
-__global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(GM <= 4 ? 1024 / NT : 1)))
+__global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(NT == 256 ? (GM <= 4 ? 5 : 4) : GM <= 4 ? 2 : 1)))
 void race_decode_step(DecodeParams P)
 {
     // state update: TPR threads per bucket row (VEC floats each), RIF rows per pass over the state,
-    // PFR rows per thread loaded together; GM >= G query heads
-    constexpr int VEC = 4, TPR = D / VEC, RIF = NT / TPR, PFR = 4, NWV = NT / 64;
+    // PFR rows per thread in flight, PF0 of the first ones beside the inputs; GM >= G query heads
+    constexpr int VEC = 4, TPR = D / VEC, RIF = NT / TPR, PFR = 4, PF0 = NT == 256 ? 2 : PFR, NWV = NT / 64;
     // projection: PARTS lanes share a column, CPW columns per wave and pass
     constexpr int PARTS = D / 8, CPW = 64 / PARTS;
     extern __shared__ float sm[];
@@ -1291,15 +1297,18 @@ void race_decode_step(DecodeParams P)
     const TX *v = reinterpret_cast<const TX *>(P.v) + (int64_t)z * D;
     f32x4 bpre[PFR];
     float apre[PFR], vv[VEC];
-    // loads of clamped rows (always inside the state), all in flight together
-    auto load_state = [&](int s0) {
+    // loads of clamped rows j0 .. j1 of a pass (always inside the state), all in flight together
+    auto load_state = [&](int s0, auto j0, auto j1) {
 #pragma unroll
-        for (int j = 0; j < PFR; ++j) {
+        for (int j = j0; j < j1; ++j) {
             const int sr = min(s0 + rr + j * RIF, S - 1);
             bpre[j] = *reinterpret_cast<const f32x4 *>(Bs + (int64_t)sr * D + dv);
             apre[j] = A[sr];
         }
     };
+    constexpr std::integral_constant<int, 0> row0{};
+    constexpr std::integral_constant<int, PF0> row1{};
+    constexpr std::integral_constant<int, PFR> row2{};
     auto load_value = [&]() {
 #pragma unroll
         for (int e = 0; e < VEC; ++e)
@@ -1319,7 +1328,7 @@ void race_decode_step(DecodeParams P)
             x[1 + g].load(q + min(g, G - 1) * D + part * 8);
         if constexpr (first) {
             load_value();
-            load_state(0);
+            load_state(0, row0, row1);
         }
 #pragma unroll
         for (int e = 0; e < 8; ++e)
@@ -1355,6 +1364,15 @@ void race_decode_step(DecodeParams P)
     project(wv * CPW, std::true_type());
     for (int j0 = (wv + NWV) * CPW; j0 < LK; j0 += NWV * CPW)
         project(j0, std::false_type());
+    load_state(0, row1, row2);
+    float ahead = 0.0f;
+    if constexpr (NT == 256) {  // one element per 64 bytes of the inputs of pair z + DEC_AHEAD
+        constexpr int EL = 64 / sizeof(TX), LPR = D / EL;
+        const int row = threadIdx.x / LPR, o = threadIdx.x % LPR * EL;
+        static_assert((GM + 2) * LPR <= NT, "one element per thread");
+        if (z + DEC_AHEAD < (int)gridDim.x && row < G + 2)
+            ahead = (float)(row < G ? q + ((int64_t)DEC_AHEAD * G + row) * D : (row == G ? k : v) + (int64_t)DEC_AHEAD * D)[o];
+    }
     __syncthreads();
     for (int i = threadIdx.x; i < (G + 1) * S; i += NT) {
         const int row = i / S, s = i % S;
@@ -1374,7 +1392,7 @@ void race_decode_step(DecodeParams P)
             acc[g][e] = 0.0f;
     for (int s0 = 0; s0 < S; s0 += PFR * RIF) {
         if (s0 > 0)
-            load_state(s0);
+            load_state(s0, row0, row2);
 #pragma unroll
         for (int j = 0; j < PFR; ++j) {
             const int s = s0 + rr + j * RIF;
@@ -1415,6 +1433,7 @@ void race_decode_step(DecodeParams P)
                     sRed[(wv * G + g) * D + dv + e] = x;
             }
     __syncthreads();
+    asm volatile("" ::"v"(ahead));  // (a use: the load stays)
     TX *out = reinterpret_cast<TX *>(P.out) + (int64_t)z * G * D;
     for (int i = threadIdx.x; i < G * D; i += NT) {
         float sum = 0.0f;

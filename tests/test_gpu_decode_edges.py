@@ -53,3 +53,23 @@ def test_decode_edges(dev, B, Hkv, G, D, L, K, dt, shift):
     check("out", out.reshape(Z, G, D), ref[0], 2.0 ** -8 if dt == torch.bfloat16 else 2e-6)
     check("A", st.A, ref[1], 1e-6)
     check("Bs", st.Bs, ref[2], 1e-6)
+
+
+@pytest.mark.parametrize("B,Hq,Hkv,D,dtype", [(1026, 1, 1, 64, torch.bfloat16), (207, 40, 5, 64, torch.bfloat16), (600, 4, 2, 128, torch.float32),
+                                              (260, 32, 8, 64, torch.bfloat16), (173, 18, 6, 128, torch.bfloat16)])
+def test_more_pairs_than_run_at_a_time(dev, B, Hq, Hkv, D, dtype):
+    """Beyond 1024 (sequence, kv head) pairs a workgroup also reads the inputs of a later one ahead: the same
+    step as two halves of the batch, to the bit, over three steps."""
+    from race_attention_amd import RaceDecodeState, build_planes_protos
+    L, K, n = 4, 3, B // 2
+    print(f"pairs B={B} Hq={Hq} Hkv={Hkv} D={D} {dtype}", flush=True)
+    planes, _ = build_planes_protos(D, K, L, 1, device=dev, seed=0)
+    g = torch.Generator(device=dev).manual_seed(B)
+    sizes = (B, n, B - n)
+    whole, first, second = (RaceDecodeState(b, Hq, Hkv, D, L, K, planes, device=dev) for b in sizes)
+    assert B * Hkv > 1024 and min(n, B - n) * Hkv > 512
+    for _ in range(3):
+        q, k, v = (torch.randn(B, h, D, generator=g, device=dev).to(dtype) for h in (Hq, Hkv, Hkv))
+        out = whole.step(q, k, v)
+        assert torch.equal(out, torch.cat([first.step(q[:n], k[:n], v[:n]), second.step(q[n:], k[n:], v[n:])]))
+    assert torch.equal(whole.A, torch.cat([first.A, second.A])) and torch.equal(whole.Bs, torch.cat([first.Bs, second.Bs]))
