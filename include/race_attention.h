@@ -132,7 +132,7 @@ int race_op_bwd_kept(const float *pK, const float *pQ, const float *V, const flo
  * of a bf16 model in their own layout) and the probabilities [B*H][T][S] fp32 contiguous, stream
  * n = b * H + h; sums and gradients of the probabilities stay fp32. For S <= 128, S % 4 == 0 and
  * D % 4 == 0, rows that start 8-byte aligned (strides % 4 == 0), D .. 2^22 elements apart; others are
- * refused with RACE_ERR_UNSUPPORTED. The reference casts such activations to fp32 and back
+ * refused with RACE_ERR_UNSUPPORTED, an out or gV whose rows share elements with RACE_ERR_INVALID. The reference casts such activations to fp32 and back
  * (gpt.py:132-140). */
 int race_op_fwd_bf16_rows(const float *pK, const float *pQ, race_tensor V, race_tensor out, int64_t B,
                           int64_t H, int64_t T, int64_t S, int64_t D, float eps, int64_t block,

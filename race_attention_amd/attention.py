@@ -122,7 +122,7 @@ def race_causal_attention_with_state(q, k, v, planes_T, L, Kbits, scale=None, ep
     q, k, v = _bf16_rows(q), _bf16_rows(k), _bf16_rows(v)
     B, Hq, T, D = q.shape
     Hkv, S = k.shape[1], L << Kbits
-    # (rows of k and v behind the T tokens of q are not read)
+    # (k and v may be larger than q's batch, tokens and head dim, v than k's heads: the rest is not read)
     if any(x.shape[0] < B or x.shape[1] < Hkv or x.shape[2] < T or x.shape[3] < D for x in (k, v)):
         raise ValueError(f"q {tuple(q.shape)} / k {tuple(k.shape)} / v {tuple(v.shape)} mismatch")
     planes = _lib.f32_planes(planes_T)

@@ -44,7 +44,8 @@ class RaceDecodeState:
         """Causal RACE over a prompt (q [B,Hq,T,D], k/v [B,Hkv,T,D] bf16) that also
         leaves this state at the end of the prompt. Returns the prompt's output [B,Hq,T,D]
         (`bthd`: in the memory order of [B,T,Hq,D]).
-        The state must be fresh (prefill starts from zero)."""
+        The state must be fresh (prefill starts from zero). Its streams (sequence, kv head) are taken in
+        order: a prompt that splits as many of them otherwise is taken too, and one stream's for all."""
         if self.tokens:
             raise RuntimeError("prefill on a non-empty state; call reset() first")
         streams = q.shape[0] * k.shape[1]
